@@ -26,12 +26,12 @@ using namespace procell;
 // across runs.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kSeedSlots = 4;  // pinned host staging slots for batch seeds
-// Segments per resident workgroup unless tuned.  1e7-cell histogram, 3
-// workgroups of 256 per CU, segment sizes decreasing geometrically: 1 ->
-// 0.321 ms per run, 2 -> 0.289, 3 -> 0.294, 4 -> 0.309, 8 -> 0.340 (more
-// segments: more set-up and window flushes).  A batch of many small sets
-// balances better with finer segments.
-constexpr uint32_t kSegmentsPerWorkgroup = 2;
+// Segments per resident workgroup unless tuned: each segment ends with its
+// wavefronts draining their last trees, and more of them balance the CUs
+// better, so the more work there is per resident workgroup, the more segments
+// (see segments_per_workgroup).  A batch of many small sets balances better
+// with finer segments.
+constexpr uint32_t kSegmentsPerWorkgroup = 2;  // 64-bit kernel
 constexpr uint32_t kBatchSegmentsPerWorkgroup = 8;
 // most lane-stack levels a batch keeps in LDS (a 256-lane workgroup: 2 KB per level)
 constexpr uint32_t kLdsStackLevels = 11;
@@ -129,6 +129,34 @@ void destroy_plan(procell_plan *pl)
     if (pl->own_stream && pl->stream)
         (void)hipStreamDestroy(pl->stream);
     delete pl;
+}
+
+// Whether the filtered kernel's error bounds cover these sets: times, means
+// and standard deviations of magnitudes that single precision holds with
+// their products and the differences of their 64-bit values (t_max 0 or
+// infinite, or beyond these ranges, goes to the 64-bit kernel).
+bool filter_covers(const std::vector<Setup> &sets)
+{
+    for (const Setup &s : sets) {
+        if (!(s.t_max >= 1e-9 && s.t_max <= 1e12))
+            return false;
+        for (size_t j = 0; j < s.type_mean.size(); ++j)
+            if (fabs(s.type_mean[j]) > 1e12 || fabs(s.type_sd[j]) > 1e12)
+                return false;
+    }
+    return true;
+}
+
+// Segments per resident workgroup of a single set, from the expected
+// lane-steps per resident workgroup.  Filtered kernel, 3 workgroups of 512 per
+// CU, the five-type histogram at 1e6 cells (4.6e3 lane-steps), 1e7 (4.6e4)
+// and 1e8 (4.6e5), microseconds per run with 1 / 2 / 3 / 4 segments:
+// 39 / 44 / 51 / 58, 154 / 143 / 153 / 160, 1292 / 1213 / 1103 / 1099.
+uint32_t segments_per_workgroup(double lane_steps, bool filter)
+{
+    if (!filter)
+        return kSegmentsPerWorkgroup;
+    return lane_steps < 1.5e4 ? 1 : lane_steps < 1.5e5 ? 2 : 4;
 }
 
 // A plan over n_sets parameter sets (1: a plain run).  Rows, cells, type
@@ -235,16 +263,20 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     // 2.65 ms per run at 2 workgroups per CU, 5.9 ms at 3 or 4 without a window).
     const bool gstack = n_sets > 1 && a.stack_levels > kLdsStackLevels;
     const uint32_t lds_levels = gstack ? 0u : a.stack_levels;
+    const bool filter = filter_covers(pl->setups);
     // row tables (8 bytes per row) go to LDS when they are small and do not
     // cost a resident workgroup (the root steps read them when a wavefront's
-    // rows advance, so from device memory they cost little)
-    uint32_t lds_rows = (size_t)(2 * n_rows + 1) * 4 <= 16384 ? n_rows : 0u;
-    int bs = tu.block_size ? (int)tu.block_size : 256;
+    // rows advance, so from device memory they cost little).  The filtered
+    // kernel's LDS is short of window rows, not of bandwidth: 8 KB of row
+    // tables left its three workgroups of 512 per CU no window on the
+    // 1024-bin histogram (0.80 ms per run of 1e7 cells; without them 0.143).
+    uint32_t lds_rows = (size_t)(2 * n_rows + 1) * 4 <= (filter ? 2048u : 16384u) ? n_rows : 0u;
+    int bs = tu.block_size ? (int)tu.block_size : filter ? (int)kFilterThreads : 256;
     int occ = 0;
     for (;;) {
-        const size_t base = sim_lds_bytes(0, kdim, T, lds_levels, (uint32_t)bs, lds_rows);
+        const size_t base = sim_lds_bytes(0, kdim, T, lds_levels, (uint32_t)bs, lds_rows, filter);
         int occ_v = 0;
-        if (sim_occupancy(bs, base, lds_rows != 0, kdim, gstack, &occ_v) != hipSuccess)
+        if (sim_occupancy(bs, base, lds_rows != 0, kdim, gstack, filter, &occ_v) != hipSuccess)
             return fail(PROCELL_E_HIP);
         if (occ_v >= 1) {
             occ = occ_v;
@@ -254,15 +286,18 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
             return fail(PROCELL_E_DEPTH);
         bs -= 64;  // deep trees: a smaller workgroup keeps the stack within LDS
     }
-    // by default at most 16 resident wavefronts per CU (4 per SIMD, the
-    // kernel's register budget): 4 workgroups of 256 per CU against 3 measured
-    // 0.2592 -> 0.2470 ms on the 1e7-cell histogram workload (more waves hide
-    // the division step's dependency waits; the smaller tally windows cost
-    // less than that)
-    const int want = tu.blocks_per_cu ? (int)tu.blocks_per_cu : std::max(1, 16 * 64 / bs);
+    // by default at most 16 resident wavefronts per CU for the 64-bit kernel (4
+    // per SIMD, its register budget) and 24 for the filtered one (6 per SIMD):
+    // with fewer vector instructions per step its wavefronts wait more on each
+    // other's latencies.  1e8-cell histogram: 16 wavefronts per CU in four
+    // workgroups of 256 1.236 ms per run, 20 1.248, 24 1.092, and 24 in three
+    // workgroups of 512 1.099 (fewer set-ups and window flushes on smaller
+    // runs); workgroups of 384 put 8 wavefronts on two of a CU's SIMDs and 4 on
+    // the others (1e7 cells: 0.187 against 0.143 ms).
+    const int want = tu.blocks_per_cu ? (int)tu.blocks_per_cu : std::max(1, (filter ? 24 : 16) * 64 / bs);
     if (lds_rows && occ < want) {
         int occ_g = 0;
-        if (sim_occupancy(bs, sim_lds_bytes(0, kdim, T, lds_levels, (uint32_t)bs, 0), false, kdim, gstack, &occ_g) !=
+        if (sim_occupancy(bs, sim_lds_bytes(0, kdim, T, lds_levels, (uint32_t)bs, 0, filter), false, kdim, gstack, filter, &occ_g) !=
             hipSuccess)
             return fail(PROCELL_E_HIP);
         if (occ_g > occ) {
@@ -273,7 +308,7 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     a.rows_in_lds = lds_rows ? 1u : 0u;
     occ = std::min<int>(occ, want);
     ls.block_size = bs;
-    const size_t base = sim_lds_bytes(0, kdim, T, lds_levels, (uint32_t)bs, lds_rows);
+    const size_t base = sim_lds_bytes(0, kdim, T, lds_levels, (uint32_t)bs, lds_rows, filter);
     const size_t budget = std::min(lds_per_cu / (size_t)occ, lds_per_block);
     const size_t row_bytes = (size_t)kdim * T * 4;
     uint32_t win_rows = budget > base + 16 ? (uint32_t)((budget - base - 16) / row_bytes) : 0;
@@ -285,8 +320,9 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     // batch each set gets segments in proportion to its expected work (at
     // least one).
     const uint32_t resident = (uint32_t)((int64_t)n_cu * occ);
-    const uint32_t per_wg = tu.segments ? std::min<uint32_t>(tu.segments, 64)
-                                        : (n_sets == 1 ? kSegmentsPerWorkgroup : kBatchSegmentsPerWorkgroup);
+    const uint32_t per_wg = tu.segments   ? std::min<uint32_t>(tu.segments, 64)
+                            : n_sets == 1 ? segments_per_workgroup(set_cost(pl->setups[0]) / resident, filter)
+                                          : kBatchSegmentsPerWorkgroup;
     std::vector<uint32_t> g_set(n_sets, 1);
     if (n_sets == 1) {
         g_set[0] = (uint32_t)std::min<uint64_t>((uint64_t)resident * per_wg,
@@ -304,7 +340,7 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     }
     // Segment sizes: a single set's decrease geometrically in launch order
     // (rounds of `resident` segments, each round's segments a factor q
-    // smaller, the last ones 1/8 of the first), so the last workgroups
+    // smaller, the last ones 1/8 or less of the first), so the last workgroups
     // dispatched are short and the CUs finish together; a batch's sets are
     // split evenly and all segments are launched largest first.
     // Within a round, segment k goes to CU slot (k mod resident) / n_cu: the
@@ -313,7 +349,10 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     // three per CU: 1175, 1570 and 2050 cycles per division step for the
     // oldest, middle and youngest), so a slot's segments are sized by its
     // issue rate, 1.32 per slot of age (1e7-cell histogram workload: 0.2617
-    // -> 0.2587 ms and 0.2644 -> 0.2603 ms on two boxes).
+    // -> 0.2587 ms and 0.2644 -> 0.2603 ms on two boxes).  The filtered
+    // kernel's wavefronts compete less for the vector unit: 1.1 per slot, and
+    // its last segments are 1/20 of the first (1.0, 1.1, 1.2 and 1.32 per slot
+    // at 1e7 cells: 0.146, 0.142, 0.145 and 0.184 ms).
     struct Seg {
         double cost;
         uint32_t set;
@@ -326,10 +365,10 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
         const uint32_t gi = g_set[i];
         std::vector<double> wseg(gi, 1.0);
         if (n_sets == 1 && per_wg > 1 && gi == resident * per_wg) {
-            const double q = pow(0.125, 1.0 / (double)(per_wg - 1));
+            const double q = pow(filter ? 0.05 : 0.125, 1.0 / (double)(per_wg - 1));
             for (uint32_t k = 0; k < gi; ++k) {
                 const uint32_t slot = (k % resident) / (uint32_t)n_cu;  // 0: oldest on its CU
-                wseg[k] = pow(q, (double)(k / resident)) * pow(1.32, (double)(occ - 1 - (int)slot));
+                wseg[k] = pow(q, (double)(k / resident)) * pow(filter ? 1.1 : 1.32, (double)(occ - 1 - (int)slot));
             }
         }
         std::vector<double> cum(gi);
@@ -386,9 +425,9 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     }
     // the window must not cost a resident workgroup (LDS allocation granularity)
     for (;;) {
-        ls.lds_bytes = sim_lds_bytes(win_rows, kdim, T, lds_levels, (uint32_t)bs, lds_rows);
+        ls.lds_bytes = sim_lds_bytes(win_rows, kdim, T, lds_levels, (uint32_t)bs, lds_rows, filter);
         int occ_w = 0;
-        if (sim_occupancy(bs, ls.lds_bytes, lds_rows != 0, kdim, gstack, &occ_w) != hipSuccess)
+        if (sim_occupancy(bs, ls.lds_bytes, lds_rows != 0, kdim, gstack, filter, &occ_w) != hipSuccess)
             return fail(PROCELL_E_HIP);
         // keep a margin for the per-workgroup LDS allocation granularity
         const bool fits = (size_t)occ * align_up(ls.lds_bytes, 2048) <= lds_per_cu;
@@ -418,7 +457,7 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     const size_t o_ss = off; off = align_up(off + (size_t)g * 4, 256);
     const size_t o_info = off; off = align_up(off + (size_t)n_sets * sizeof(SetInfo), 256);
     const size_t o_seed = off; off = align_up(off + (size_t)n_sets * 8, 256);
-    const size_t o_gs = off; off = align_up(off + (gstack ? (size_t)g * a.stack_levels * bs * sizeof(double) : 0), 256);
+    const size_t o_gs = off; off = align_up(off + (gstack ? (size_t)g * sim_stack_bytes(a.stack_levels, (uint32_t)bs, filter) : 0), 256);
     if (arena) {
         if (off > arena_bytes)
             return fail(PROCELL_E_SCRATCH);
@@ -444,7 +483,8 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     a.kdim = kdim;
     a.counters = (unsigned long long *)(dbase + o_cnt);
     a.tally = (unsigned long long *)(dbase + o_tally);
-    a.gstack = gstack ? (double *)(dbase + o_gs) : nullptr;
+    a.filter = filter ? 1u : 0u;
+    a.gstack = gstack ? dbase + o_gs : nullptr;
 
     a.row_start = (const uint32_t *)(dbase + o_rs);
     a.row_info = (const uint32_t *)(dbase + o_ri);
@@ -793,7 +833,6 @@ int procell_plan_autotune(procell_plan *plan, const uint64_t *seeds, uint32_t re
                     best = ms;
                     best_tu = ps[0].tuning;
                     best_tu.idle_lanes = idle;
-                    best_tu.block_size = (uint32_t)cand->shape.block_size;
                     if (best_plan && best_plan != cand)
                         destroy_plan(best_plan);
                     best_plan = cand;

@@ -41,6 +41,18 @@ struct QueueEntry {
 };
 static_assert(sizeof(QueueEntry) == 48, "three 16-byte LDS words");
 
+// The filtered kernel's entry: times in single precision.
+struct alignas(16) FilterEntry {
+    float s0;           // completion time of its first division minus t_max
+    float mean, sd;     // timer parameters of its type
+    float err;          // error bound of the cell's times
+    uint32_t cell;      // initial cell id, relative to the set
+    uint32_t tb;        // LDS byte offset of its window entry at generation 0, or none
+    uint32_t rowt;      // row relative to the set's first row | sorted type << 24
+    uint32_t kcap;      // generation cap of the row
+};
+static_assert(sizeof(FilterEntry) == 32, "two 16-byte LDS words");
+
 // Copies of the counters block: workgroup b adds into copy b % kCounterCopies,
 // so the device atomics on any one counter stay few; the host sums the copies.
 constexpr uint32_t kCounterCopies = 64;
@@ -57,6 +69,8 @@ struct RunArgs {
     uint32_t win_rows;      // rows of the LDS tally window (0: none)
     uint32_t idle_limit;    // idle lanes tolerated before a wavefront refills
     uint32_t rows_in_lds;   // nonzero: the row tables are copied to LDS
+    uint32_t filter;        // nonzero: sim_filter_kernel, else sim_kernel
+    uint32_t pad;
     const SetInfo *sets;         // [n_sets]
     const uint64_t *set_seed;    // [n_sets] seeds of a batch run (n_sets > 1)
     const uint32_t *seg_set;     // [segments] set of each segment
@@ -71,8 +85,11 @@ struct RunArgs {
     const uint32_t *seg_row;     // [segments] row of each segment's first cell (window base)
     unsigned long long *tally;   // per set [rows][kdim][n_types] of the set, file type order
     unsigned long long *counters;  // [n_sets][kCounterCopies][kNumCounters]
-    double *gstack;              // [segments][stack_levels][block] lane stacks in device memory, or null: in LDS
+    void *gstack;                // [segments] blocks of lane stacks in device memory (sim_stack_bytes each), or null: in LDS
 };
+
+// Most threads of a workgroup of sim_filter_kernel.
+constexpr uint32_t kFilterThreads = 512;
 
 struct LaunchShape {
     int blocks;             // = segments
@@ -81,13 +98,14 @@ struct LaunchShape {
 };
 
 size_t sim_lds_bytes(uint32_t win_rows, uint32_t kdim, uint32_t n_types, uint32_t stack_levels, uint32_t block_size,
-                     uint32_t lds_rows);
+                     uint32_t lds_rows, bool filter);
+size_t sim_stack_bytes(uint32_t stack_levels, uint32_t block_size, bool filter);
 hipError_t launch_zero(unsigned long long *p, uint64_t n, hipStream_t st);
 hipError_t launch_sim(const RunArgs &a, const LaunchShape &ls, hipStream_t st);
 hipError_t launch_debug_draws(uint64_t seed, const uint64_t *cell, const uint64_t *node,
                               const uint32_t *attempt, uint64_t n, uint32_t *words, double *z,
                               hipStream_t st);
-hipError_t sim_occupancy(int block_size, size_t lds_bytes, bool rows_in_lds, uint32_t kdim, bool gstack,
+hipError_t sim_occupancy(int block_size, size_t lds_bytes, bool rows_in_lds, uint32_t kdim, bool gstack, bool filter,
                          int *blocks_per_cu);
 
 }  // namespace procell

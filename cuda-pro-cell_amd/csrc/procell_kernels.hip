@@ -105,6 +105,9 @@ struct Counts {
     uint32_t div, rej, lost, cells, pool;
 };
 
+// place of the refused candidates among the sums flush_counts makes in `red`
+constexpr uint32_t kRedRejected = 3;
+
 // Adds a workgroup's counts to counter copy blockIdx.x % kCounterCopies:
 // wavefront sums, then one LDS atomic per wavefront and counter, then one
 // device atomic per counter.  `red` is kNumCounters u32 of LDS, zeroed and
@@ -234,7 +237,7 @@ __global__ void __launch_bounds__(256, 4) sim_kernel(RunArgs a)
     // the lanes' stacks: in LDS after the window, or (GStack: plans whose
     // deep trees would leave no LDS for the window) the workgroup's block of
     // device memory, same layout
-    double *stack = GStack ? a.gstack + (size_t)seg0 * a.stack_levels * bdim
+    double *stack = GStack ? (double *)a.gstack + (size_t)seg0 * a.stack_levels * bdim
                            : (double *)((unsigned char *)win + ((size_t)win_len * 4 + 4 + 15) / 16 * 16);
     // the lane's stack column: level l (1-based) at stk_pop + l * stride,
     // i.e. at stk_push + (l - 1) * stride (bytes)
@@ -643,6 +646,645 @@ __global__ void __launch_bounds__(256, 4) sim_kernel(RunArgs a)
     }
 }
 
+// ----------------------------------------------------------------------
+// The filter.  A run's outputs are whole numbers, and the times enter them
+// only through two tests: "timer > 0" and "completion time > t_max".  The
+// filtered kernel evaluates both from single-precision times whose distance
+// from the 64-bit times is bounded, accepts a test when the value is further
+// from the threshold than the bound, and otherwise evaluates the cell's times
+// again in 64 bits along its path from the root (exact_times: the same
+// operations in the same order as the 64-bit kernel), so every test comes out
+// as the 64-bit kernel's and the outputs are the same bit for bit.
+//
+// Why: the 64-bit Box-Muller pair is 87 of a division step's 180 vector
+// instructions at 4 cycles each; the hardware's log2, sqrt, sin and cos take
+// 8 cycles each and single-precision multiplies and adds 2.  Five-type
+// histogram, 1024 bins: 0.219 -> 0.143 ms per run at 1e7 cells, 2.05 -> 1.10
+// ms at 1e8 (2.58e8 divisions: 1.26e11 -> 2.35e11 per second; vector
+// instructions per division 4.56 -> 2.70).
+//
+// The bound.  For a block whose first word w0 lies in [2^16, 2^32 - 2^16)
+// (pair_sure; the others, 1 in 2^15, are evaluated in 64 bits)
+// normal_pair_f32 is within 5.6e-6 of the 64-bit pair.  Measured on gfx950
+// over all 2^32 values of each word: the radius is off by at most 5.42e-6 (next to u1 = 1, where it
+// is below 0.01) and 3.64e-6 for u1 <= 1/2, sine and cosine by 2.7e-7 (times
+// a radius of at most 4.71).  kPairErr allows 7e-6.  A timer fma(z, sd, mean)
+// adds the rounding of sd, mean and itself: at most 2^-23 (|mean| + 8.6 |sd|);
+// a completion time adds 2^-24 t_max per addition (times are kept relative to
+// t_max, so a value near the threshold is small, and no partial sum of a path
+// exceeds t_max) and 3.5 of those for t_max and the root's phase.  After k
+// levels below the root that is (k + 2) e + (k + 3.5) 2^-24 t_max with e =
+// 6.7e-6 |sd| + 1.2e-7 |mean|; type_err and cell_err round it up, with the
+// row's cap for k.
+// ----------------------------------------------------------------------
+constexpr float kPairErr = 7.0e-6f;
+constexpr uint32_t kPairLow = 1u << 16;
+
+__device__ __forceinline__ bool pair_sure(uint32_t w0) { return w0 - kPairLow < 0u - 2u * kPairLow; }
+
+__device__ __forceinline__ void normal_pair_f32(uint32_t w0, uint32_t w2, float &z0, float &z1)
+{
+    const float u1 = (float)w0 * 0x1p-32f;
+    const float rho = __builtin_amdgcn_sqrtf(__builtin_amdgcn_logf(u1) * -1.3862943611198906f);  // -2 ln 2
+    const float turn = (float)w2 * 0x1p-32f;
+    z0 = rho * __builtin_amdgcn_cosf(turn);
+    z1 = rho * __builtin_amdgcn_sinf(turn);
+}
+
+__device__ __forceinline__ float type_err(double mean, double sd, double t_max)
+{
+    return (float)(fabs(sd) * ((double)kPairErr + 0x1p-20) + 0x1p-22 * fabs(mean) + 0x1p-23 * t_max);
+}
+
+// Smaller of two magnitudes.
+__device__ __forceinline__ float min_abs(float x, float y) { return fminf(fabsf(x), fabsf(y)); }
+
+__device__ __forceinline__ float cell_err(uint32_t kcap, float terr) { return (float)(kcap + 4u) * terr; }
+
+// Completion times in 64 bits, minus t_max and rounded to single precision
+// (which keeps the sign of the 64-bit comparison: the difference of two
+// doubles of magnitude above 1e-20 is 0 or above 1e-36): of the division of
+// `node` (its daughters' l and r), or with node 0 of the root's first
+// division (l).  The path from the root is walked again; rej counts the
+// candidates refused for the returned times.  Needed
+// about once in a thousand steps.
+struct ExactTimes {
+    float l, r;
+    uint32_t rej;
+};
+
+__device__ __forceinline__ ExactTimes exact_times(uint64_t seed, uint32_t cell, uint64_t node, double mean, double sd,
+                                                  double t_max)
+{
+    const dev::Tables tb = dev::global_tables();
+    constexpr dev::Coeffs K = dev::coeffs();
+    const uint32_t levels = node ? 64u - (uint32_t)__builtin_clzll(node) : 0u;  // divisions on the path, this one included
+    double s = 0.0, last_l = 0.0;
+    uint32_t rej = 0;
+    // step 0: the root's first timer from block (cell, 0, 0); step i >= 1: the
+    // pair of the path's i-th node, of which the path takes one timer and the
+    // last node both
+    for (uint32_t step = 0; step <= levels; ++step) {
+        const uint64_t at = step ? node >> (levels - step) : 0ull;
+        Words w = dev::draw_block(seed, cell, at, 0u);
+        const double U = dev::uniform_oc_hi(w.w1);
+        if (step == 0)
+            w = Words{w.w2, 0u, w.w3, 0u};
+        double z0, z1;
+        dev::normal_pair(w, z0, z1, K, tb);
+        rej = 0;
+        const bool both = step == levels && step != 0;
+        for (uint32_t side = both ? 0u : step ? (uint32_t)(node >> (levels - step - 1)) & 1u : 0u; side < 2; ++side) {
+            double tau = fma(side ? z1 : z0, sd, mean);
+            if (!(tau > 0.0)) {
+                // truncated normal (cell.cu:106-122): the root's second
+                // candidate, then the node's redraw stream, the mean after
+                // 65535 blocks
+                ++rej;
+                uint32_t att = 1;
+                double y0 = z0, y1 = z1;
+                bool pair = step == 0;  // y1 still to be tried
+                for (;;) {
+                    if (pair) {
+                        tau = fma(y1, sd, mean);
+                        if (tau > 0.0)
+                            break;
+                        ++rej;
+                    }
+                    if (att > 65535u) {
+                        tau = mean;
+                        break;
+                    }
+                    dev::normal_pair(dev::draw_block(seed, cell, step ? at << 1 | side : 1ull, att), y0, y1, K, tb);
+                    ++att;
+                    tau = fma(y0, sd, mean);
+                    if (tau > 0.0)
+                        break;
+                    ++rej;
+                    pair = true;
+                }
+            }
+            if (both && side == 0) {
+                last_l = s + tau;
+                continue;
+            }
+            s = step ? s + tau : tau * U + tau;
+            break;
+        }
+    }
+    return levels ? ExactTimes{(float)(last_l - t_max), (float)(s - t_max), rej}
+                  : ExactTimes{(float)(s - t_max), 0.0f, rej};
+}
+
+// ======================================================================
+// sim_filter_kernel: the same run as sim_kernel (segments, claims, root
+// steps, hand-outs and division steps as there), with the two tests on times
+// filtered as described above; it runs every plan whose times the bound
+// covers (the host's filter_covers).  What bounds it is the vector unit's
+// issue rate (4 cycles per SIMD for nearly every instruction; 0.95 per CU and
+// clock at 1e8 cells) and, with fewer instructions per step than sim_kernel,
+// the latency of a wavefront's own instruction stream: 6 wavefronts per SIMD
+// instead of 4 gave 1.24 -> 1.09 ms, which holds it to 80 registers (the
+// 64-bit evaluation spills a few, in its own branch only).  The tree logic is
+// arranged for few instructions and few values carried round the loop:
+//  * a lane's pending right daughters are a mask relative to its level (bit i:
+//    level k - i), with one more bit for level 0 that no daughter uses.  Going
+//    down shifts the mask up by one; "the left daughter does not divide" takes
+//    the lowest set bit, whichever of the right daughter (bit 0) or an older
+//    level it is, and the same shift takes node and level there.  Taking the
+//    level-0 bit leaves the mask empty: the lane is idle exactly when its mask
+//    is 0.
+//  * idle lanes, and lanes with a redraw pending, are masked off (the exec
+//    mask, scalar work) instead of having every result selected.
+//  * the state of a redraw (1 in 10 steps has one) waits in LDS: in registers
+//    it cost some 20 copies per step at the loop's branches.
+//  * event counts are scalar; a step looks at tallies outside the window only
+//    where the workgroup's rows exceed it.
+// LDS: type tables ({mean, sd, error bound, file index}: 16 bytes [T]; last
+// drawn word + 1: u32 [T]) | row tables when they fit | counter sums u32 [8] |
+// root step cursor u32 [4] | buffered entries, per wavefront [64] | redraws,
+// per lane | window tally u32 [win_rows * kdim * T] | stacks float, per wavefront
+// [stack_levels][64]
+// ======================================================================
+struct alignas(16) FilterType {
+    float mean, sd;
+    float err;      // error bound of a completion time per level
+    uint32_t file;  // file index
+};
+
+// per wavefront: buffered entries, lanes' redraws
+__host__ __device__ constexpr uint32_t filter_wave_bytes()
+{
+    return kWave * (uint32_t)(sizeof(FilterEntry) + 16);
+}
+
+__host__ __device__ constexpr size_t filter_type_bytes(uint32_t n_types)
+{
+    return (size_t)n_types * sizeof(FilterType) + ((size_t)n_types * 4 + 15) / 16 * 16;
+}
+
+// A lane of sim_filter_kernel.
+template <typename N>
+struct FilterLane {
+    N node, pend;       // heap index; pending levels relative to k, 0: the lane is idle
+    float s;            // completion time of the node's division minus t_max
+    float mean, sd;
+    float err;          // bound of |s - its 64-bit value| at any level of the tree
+    uint32_t cell;      // initial cell, relative to its set
+    uint32_t tb;        // LDS address of the window entry (row, generation 0, type), or kNoWindow
+    uint32_t rowt;      // row relative to the set's first row | sorted type << 24
+    uint32_t k, kcap;
+};
+
+// A division with a redraw pending, kept in LDS (rarely used: in registers it
+// would be copied at every branch of the loop).
+struct alignas(16) FilterRedo {
+    float tl, tr;       // timers so far
+    uint32_t redo;      // bit 0 / bit 1: left / right timer still to redraw; attempt number << 2
+    uint32_t rej;       // refused candidates
+};
+
+typedef __attribute__((address_space(3))) unsigned int LdsWord;
+
+// LDS address of an entry of the dynamic block, and an add to such an entry.
+__device__ __forceinline__ uint32_t lds_address(void *p) { return (uint32_t)(uintptr_t)(LdsWord *)p; }
+__device__ __forceinline__ void lds_add(uint32_t at, uint32_t v)
+{
+    __hip_atomic_fetch_add((LdsWord *)(uintptr_t)at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+template <bool RowsLds, typename N, bool GStack>
+__global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a)
+{
+    extern __shared__ __align__(16) unsigned char lds[];
+    const uint32_t tid = threadIdx.x;
+    const uint32_t bdim = blockDim.x;
+    const uint32_t lane = tid & (kWave - 1);
+    const uint32_t wave = uni(tid / kWave);
+    const uint32_t n_waves = bdim / kWave;
+    const uint32_t seg0 = blockIdx.x;
+    const uint32_t set = a.n_sets > 1 ? a.seg_set[seg0] : 0u;
+    const SetInfo S = a.sets[set];
+    const uint64_t seed = a.n_sets > 1 ? a.set_seed[set] : a.seed;
+    const double t_max = S.t_max;
+    const float t_max32 = (float)t_max;
+    const uint32_t T = S.n_types;
+    const uint32_t kdim = S.kdim;
+    const uint32_t T4 = T * 4;
+    const uint32_t row_bytes = kdim * T4;
+    const uint32_t win_len = a.win_rows * kdim * T;
+    const uint32_t lds_rows = RowsLds ? a.n_rows : 0u;
+    FilterType *types = (FilterType *)lds;
+    uint32_t *lims = (uint32_t *)(types + T);
+    uint32_t *r_start = (uint32_t *)(lds + filter_type_bytes(T));
+    uint32_t *r_info = r_start + lds_rows + 1;
+    uint32_t *red = (uint32_t *)((unsigned char *)r_start + (RowsLds ? ((size_t)(2 * lds_rows + 1) * 4 + 15) / 16 * 16 : 0));
+    uint32_t *cursor = red + kNumCounters;  // root steps of the segment claimed so far
+    FilterEntry *ent = (FilterEntry *)((unsigned char *)red + kSimSharedBytes) + wave * kWave;
+    FilterRedo *redo = (FilterRedo *)((unsigned char *)red + kSimSharedBytes + n_waves * kWave * sizeof(FilterEntry)) + tid;
+    const uint32_t win_off = (uint32_t)((unsigned char *)red - lds) + kSimSharedBytes + n_waves * filter_wave_bytes();
+    const uint32_t win_base = lds_address(lds + win_off);
+    unsigned int *win = (unsigned int *)(lds + win_off);
+    constexpr uint32_t kStride = kWave * (uint32_t)sizeof(float);  // bytes between levels
+    const uint32_t levels = a.stack_levels;
+    // level l (1-based) at stack + l * kWave; "level 0" is what lies before,
+    // never stored to
+    float *stack = (GStack ? (float *)a.gstack + (size_t)seg0 * levels * bdim
+                           : (float *)(lds + win_off + ((size_t)win_len * 4 + 15) / 16 * 16)) +
+                   (size_t)wave * levels * kWave - kWave;
+    unsigned char *const stk = (unsigned char *)(stack + lane);
+
+    const uint64_t seg_begin = uni64(a.seg_begin[seg0]);
+    const uint64_t seg_end = uni64(a.seg_end[seg0]);
+    const uint64_t seg_cells = seg_end - seg_begin;
+    const uint32_t row_lo = uni(a.seg_row[seg0]);  // first row of the segment and of the tally window
+    const uint32_t cell0 = (uint32_t)(seg_begin - S.cell_base);
+    for (uint32_t i = tid; i < T; i += bdim) {
+        const double cum = a.type_cum[S.type_base + i], m = a.type_mean[S.type_base + i], sd = a.type_sd[S.type_base + i];
+        types[i] = FilterType{(float)m, (float)sd, type_err(m, sd, t_max), a.type_file[S.type_base + i]};
+        // w 2^-32 < cum for a whole number w: w < ceil(cum 2^32); a limit of
+        // 2^32 or more is stored as 2^32 - 1, and a drawn 2^32 - 1 looked at
+        // again (the sums are > 0: the largest proportion comes first and the
+        // last sum is 1)
+        lims[i] = (uint32_t)fmin(ceil(cum * 0x1p32), 0x1p32 - 1.0);
+    }
+    for (uint32_t i = tid; i <= lds_rows && RowsLds; i += bdim)
+        r_start[i] = a.row_start[i];
+    for (uint32_t i = tid; i < lds_rows; i += bdim)
+        r_info[i] = a.row_info[i];
+    for (uint32_t i = tid; i < win_len; i += bdim)
+        win[i] = 0u;
+    if (tid < kNumCounters + 1)
+        red[tid] = 0u;  // counter sums and the root step cursor
+    __syncthreads();
+
+    // the row tables' address space is known at compile time (no flat loads)
+    const uint32_t *rs = RowsLds ? r_start : a.row_start;
+    const uint32_t *ri = RowsLds ? r_info : a.row_info;
+    // every row of the segment has its window
+    const bool all_in = uni(row_lo + a.win_rows >= a.n_rows || (uint64_t)rs[row_lo + a.win_rows] >= seg_end ? 1u : 0u) != 0;
+
+    uint32_t rpos = 0, rn = 0;      // buffered dividing roots: entries [rpos, rn) of ent
+    uint32_t roots_done = 0;
+    // limits of the type search (0: never met, for the last type and beyond)
+    uint32_t lim8[8];
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k)
+        lim8[k] = uni(k + 1 < T ? lims[k] : 0u);
+    // Row boundaries of the wavefront's root steps (as in sim_kernel)
+    uint32_t rb = row_lo, bnd = 0, rinfo = 0;
+    auto load_rows = [&]() {
+        const uint32_t r1 = rb + 1 + lane;
+        bnd = r1 <= a.n_rows ? rs[r1] : 0xFFFFFFFFu;
+        rinfo = rb + lane < a.n_rows ? ri[rb + lane] : 0u;
+    };
+    load_rows();
+
+    FilterLane<N> L{};
+    uint64_t redoing = 0;                                     // lanes with a redraw pending
+    uint32_t w_div = 0, w_lost = 0, w_cells = 0, w_pool = 0;  // event counts, scalar
+    unsigned int *n_rej = &red[kRedRejected];                 // refused candidates: rare, counted in LDS
+    const uint32_t idle_limit = a.idle_limit;
+
+    for (;;) {
+        const uint64_t idle = __ballot(L.pend == 0);
+        const uint32_t n_idle = uni((uint32_t)__popcll(idle));
+        // ======== refill once more than idle_limit lanes are idle ========
+        if (n_idle > idle_limit) {
+            // ---- root step: the buffer is empty ----
+            if (rpos >= rn && !roots_done) {
+                uint32_t step = 0;
+                if (lane == 0)
+                    step = atomicAdd(cursor, 1u);
+                const uint64_t c_off = (uint64_t)uni(step) * kWave;
+                if (c_off >= seg_cells)
+                    roots_done = 1;
+                if (!roots_done) {
+                    const uint64_t c_cur = seg_begin + c_off;
+                    const uint32_t n_valid = uni((uint32_t)min<uint64_t>(kWave, seg_cells - c_off));
+                    const bool valid = lane < n_valid;
+                    const uint32_t cell = cell0 + (uint32_t)c_off + lane;
+                    // rows of the step's cells (cell ids < 2^32): move rb to the
+                    // row of c_cur, then count the boundaries inside the step
+                    const uint32_t c32 = (uint32_t)c_cur;
+                    for (uint64_t le = __ballot(bnd <= c32); le; le = __ballot(bnd <= c32)) {
+                        rb = uni(rb + (uint32_t)__popcll(le));
+                        load_rows();
+                    }
+                    const uint32_t nb = uni((uint32_t)__popcll(__ballot((uint64_t)bnd < c_cur + n_valid)));
+                    uint32_t rrel = 0;  // boundaries at or below this lane's cell
+                    uint32_t info = uni(rinfo);
+                    if (nb) {
+                        for (uint32_t j = 0; j < nb; ++j)
+                            rrel += lane >= (uint32_t)__builtin_amdgcn_readlane((int)bnd, (int)j) - c32 ? 1u : 0u;
+                        info = (uint32_t)__shfl(rinfo, (int)rrel);
+                    }
+                    const uint32_t row = rb + rrel;
+                    const uint32_t kc = info & 0xFFu;
+                    const bool ge_phi = (info >> 8) & 1u;
+                    // one block per initial cell: type uniform (word 0), phase
+                    // (word 1) and the first timer's Box-Muller pair (words 2, 3)
+                    const Words w = dev::draw_block(seed, cell, 0, 0);
+                    // first type with w 2^-32 < cumulative proportion
+                    // (cell.cu:90-101): scanning from the highest index down, the
+                    // last hit is the first; past the last proportion, the last type
+                    uint32_t jt = T - 1;
+                    if (T > 9) {
+                        for (uint32_t k = T - 2; k >= 8; --k)
+                            jt = w.w0 < lims[k] ? k : jt;
+                    }
+                    if (T > 5) {
+#pragma unroll
+                        for (int k = 7; k >= 4; --k)
+                            jt = w.w0 < lim8[k] ? (uint32_t)k : jt;
+                    }
+#pragma unroll
+                    for (int k = 3; k >= 0; --k)
+                        jt = w.w0 < lim8[k] ? (uint32_t)k : jt;
+                    if (__builtin_expect(__ballot(w.w0 == 0xFFFFFFFFu) != 0, 0)) {
+                        if (w.w0 == 0xFFFFFFFFu)
+                            for (jt = 0; jt + 1 < T && !(dev::uniform_co_hi(w.w0) < a.type_cum[S.type_base + jt]); ++jt) {
+                            }
+                    }
+                    const FilterType ty = types[jt];
+                    const float err = cell_err(kc, ty.err);
+                    const bool quiescent = ty.mean < 0.0f;
+                    const bool live = valid && !quiescent;
+                    // first timer (cell.cu:106-122): two candidates from the root
+                    // block, then node 1's redraw stream (in 64 bits)
+                    float z0, z1;
+                    normal_pair_f32(w.w2, w.w3, z0, z1);
+                    const float u1 = fmaf((float)w.w1, 0x1p-32f, 1.0f);
+                    const float tau0 = fmaf(z0, ty.sd, ty.mean);
+                    float s0 = fmaf(tau0, u1, -t_max32);
+                    const bool sure = (min_abs(tau0, s0) > err) & (tau0 > 0.0f) & pair_sure(w.w2);
+                    if (__builtin_expect(__ballot(live && !sure) != 0, 0)) {
+                        if (live && !sure) {
+                            // the second candidate where the first is surely refused
+                            const float tau1 = fmaf(z1, ty.sd, ty.mean);
+                            s0 = fmaf(tau1, u1, -t_max32);
+                            uint32_t rej = 1;
+                            if (!(pair_sure(w.w2) && tau0 < -err && tau1 > err && fabsf(s0) > err)) {
+                                const ExactTimes e = exact_times(seed, cell, 0, a.type_mean[S.type_base + jt],
+                                                                 a.type_sd[S.type_base + jt], t_max);
+                                s0 = e.l;
+                                rej = e.rej;
+                            }
+                            atomicAdd(n_rej, rej);
+                        }
+                    }
+                    // quiescent or out of time: tallied if its value is in the
+                    // output bin set; in time with f/2 <= phi: dropped; else it
+                    // divides
+                    const bool record = valid && (quiescent || s0 > 0.0f);
+                    const bool rec_ok = record && ge_phi;
+                    const bool divides = valid && !record && kc != 0;
+                    const uint64_t dmask = __ballot(divides);
+                    w_cells += n_valid;
+                    w_lost += (uint32_t)__popcll(__ballot(record && !ge_phi));
+                    w_pool += (uint32_t)__popcll(dmask);
+                    // generation-0 tallies: the window, else one device atomic
+                    // per distinct (row, type) of the step
+                    const uint32_t woff = row - row_lo;
+                    const bool in_win = all_in || woff < a.win_rows;
+                    const uint32_t tb = win_base + __umul24(woff, row_bytes) + ty.file * 4;
+                    if (rec_ok && in_win)
+                        lds_add(tb, 1u);
+                    if (!all_in) {
+                        uint64_t pend = __ballot(rec_ok && !in_win);
+                        while (pend) {
+                            const uint32_t leader = (uint32_t)__builtin_ctzll(pend);
+                            const uint32_t row_l = uni(__shfl(row, (int)leader));
+                            const uint32_t tf_l = uni(__shfl(ty.file, (int)leader));
+                            const uint64_t same = __ballot(rec_ok && !in_win && row == row_l && ty.file == tf_l);
+                            if (lane == leader)
+                                atomicAdd(&a.tally[S.tally_base + (uint64_t)(row_l - S.row_base) * kdim * T + tf_l],
+                                          (unsigned long long)__popcll(same));
+                            pend &= ~same;
+                        }
+                    }
+                    // dividing cells: buffered for the hand-outs
+                    if (divides)
+                        ent[lane_rank(dmask)] = FilterEntry{s0, ty.mean, ty.sd, err, cell, in_win ? tb : kNoWindow,
+                                                            (row - S.row_base) | (jt << 24), kc};
+                    rpos = 0;
+                    rn = uni((uint32_t)__popcll(dmask));
+                    __builtin_amdgcn_wave_barrier();
+                }
+            }
+            // ---- steal pending daughters inside the wavefront ----
+            if (rpos >= rn && roots_done) {
+                // a lane's shallowest pending daughter: the highest bit below
+                // its level-0 bit k
+                const N mine = L.pend & (((N)1 << L.k) - (N)1);
+                const uint64_t donors = __ballot(mine != 0);
+                const uint32_t nd = uni(min((uint32_t)__popcll(donors), n_idle));
+                if (nd) {
+                    const uint32_t my_up = mine ? top_bit(mine) : 0u;
+                    const uint32_t r = lane_rank(idle);
+                    const bool thief = L.pend == 0 && r < nd;
+                    const uint32_t src = thief ? nth_set_bit(donors, r) : lane;
+                    const uint32_t up = __shfl(my_up, (int)src);
+                    const N d_node = __shfl(L.node, (int)src);
+                    const uint32_t d_k = __shfl(L.k, (int)src);
+                    const uint32_t d_cell = __shfl(L.cell, (int)src);
+                    const uint32_t d_kcap = __shfl(L.kcap, (int)src);
+                    const uint32_t d_tb = __shfl(L.tb, (int)src);
+                    const uint32_t d_rowt = __shfl(L.rowt, (int)src);
+                    const float d_mean = __shfl(L.mean, (int)src);
+                    const float d_sd = __shfl(L.sd, (int)src);
+                    const float d_err = __shfl(L.err, (int)src);
+                    if (mine != 0 && lane_rank(donors) < nd)
+                        L.pend &= ~((N)1 << my_up);
+                    if (thief) {
+                        L.k = d_k - up;
+                        L.s = stack[L.k * kWave + src];
+                        L.node = (d_node >> up) | (N)1;
+                        L.pend = (N)1 << L.k;  // its level-0 bit alone
+                        L.cell = d_cell;
+                        L.kcap = d_kcap;
+                        L.tb = d_tb;
+                        L.rowt = d_rowt;
+                        L.mean = d_mean;
+                        L.sd = d_sd;
+                        L.err = d_err;
+                    }
+                }
+            }
+        }
+        // ---- idle lanes take buffered roots, in lane order ----
+        if (rpos < rn) {
+            const uint64_t idle2 = __ballot(L.pend == 0);
+            const uint32_t rank = lane_rank(idle2) + rpos;
+            if (L.pend == 0 && rank < rn) {
+                const FilterEntry e = ent[rank];
+                L.s = e.s0;
+                L.mean = e.mean;
+                L.sd = e.sd;
+                L.err = e.err;
+                L.cell = e.cell;
+                L.tb = e.tb;
+                L.rowt = e.rowt;
+                L.kcap = e.kcap;
+                L.node = (N)1;
+                L.pend = (N)1;
+                L.k = 0u;
+            }
+            rpos = uni(min(rpos + (uint32_t)__popcll(idle2), rn));
+        }
+
+        // ======== division step ========
+        // One Philox block + Box-Muller pair per busy lane and step: either
+        // the pair block of a new division (timers of both daughters) or one
+        // block of a daughter's truncated-normal redraw stream
+        // (cell.cu:106-122); a lane with a redraw pending does not advance its
+        // tree in that step.
+        const uint64_t busy = __ballot(L.pend != 0);
+        if (busy == 0 && roots_done && rpos >= rn)
+            break;
+        w_div += uni((uint32_t)__popcll(busy & ~redoing));
+        bool again = false;  // a redraw pending after this step
+        if (L.pend != 0) {
+            // the completion time a pop at the end of this step takes, read
+            // here so that the LDS round trip overlaps the division (a lane
+            // pops only when the step pushes nothing)
+            const uint32_t fl = low_bit(L.pend);
+            const float sp = *(const float *)(stk + __umul24(L.k - fl, kStride));
+            float sl, sr;
+            bool cmp = true;      // division complete this step
+            bool unsure = false;  // a test of this step is within its error bound
+            if (__builtin_expect(redoing == 0, 1)) {
+                // no redraw pending in the wavefront (the common case)
+                const Words w = dev::draw_block(seed, (uint64_t)L.cell, L.node, 0u);
+                float z0, z1;
+                normal_pair_f32(w.w0, w.w2, z0, z1);
+                const float tl = fmaf(z0, L.sd, L.mean);
+                const float tr = fmaf(z1, L.sd, L.mean);
+                sl = L.s + tl;
+                sr = L.s + tr;
+                const bool fine = (fminf(fminf(tl, tr), min_abs(sl, sr)) > L.err) & pair_sure(w.w0);
+                if (__builtin_expect(__ballot(!fine) != 0, 0)) {
+                    if (!fine) {
+                        // a timer surely < 0: that daughter continues in its
+                        // redraw stream; else surely > 0 and surely in or out
+                        // of time, or the division is evaluated in 64 bits
+                        const uint32_t r0 = tl < 0.0f ? 1u : 0u;
+                        const uint32_t r1 = tr < 0.0f ? 1u : 0u;
+                        if (pair_sure(w.w0) && min_abs(tl, tr) > L.err && (r0 | r1) != 0u) {
+                            *redo = FilterRedo{tl, tr, r0 | (r1 << 1) | 4u, r0 + r1};
+                            cmp = false;
+                        } else {
+                            unsure = true;
+                        }
+                    }
+                }
+            } else {
+                const bool fresh = ((redoing >> lane) & 1ull) == 0;
+                FilterRedo q{0.0f, 0.0f, 4u, 0u};
+                if (!fresh)
+                    q = *redo;
+                const uint32_t att = q.redo >> 2;
+                const bool left = (q.redo & 1u) != 0;  // the left timer is drawn again first
+                const N bnode = fresh ? L.node : (L.node << 1) | (N)(left ? 0u : 1u);
+                const Words w = dev::draw_block(seed, (uint64_t)L.cell, bnode, fresh ? 0u : att);
+                float z0, z1;
+                normal_pair_f32(w.w0, w.w2, z0, z1);
+                const float c0 = fmaf(z0, L.sd, L.mean);
+                const float c1 = fmaf(z1, L.sd, L.mean);
+                const uint32_t r0 = c0 > 0.0f ? 0u : 1u;
+                const uint32_t r1 = c1 > 0.0f ? 0u : 1u;
+                if (fresh) {
+                    q = FilterRedo{c0, c1, r0 | (r1 << 1) | 4u, r0 + r1};
+                } else {
+                    // first candidate > 0 of this block; after 65535 blocks the mean
+                    q.rej += r0 + (r0 & r1);
+                    if ((r0 & r1) == 0u || att >= 65535u) {
+                        const float v = r0 == 0u ? c0 : r1 == 0u ? c1 : L.mean;
+                        (left ? q.tl : q.tr) = v;
+                        q.redo = (q.redo & (left ? 2u : 0u)) | 4u;
+                    } else {
+                        q.redo += 4u;
+                    }
+                }
+                sl = L.s + q.tl;
+                sr = L.s + q.tr;
+                cmp = (q.redo & 3u) == 0;
+                unsure = !pair_sure(w.w0) || !(min_abs(c0, c1) > L.err) || (cmp && !(min_abs(sl, sr) > L.err));
+                // refused candidates are counted when the division completes
+                // (exact_times counts a division's anew)
+                if (!unsure) {
+                    if (cmp && q.rej)
+                        atomicAdd(n_rej, q.rej);
+                    if (!cmp)
+                        *redo = q;
+                }
+            }
+            if (__builtin_expect(__ballot(unsure) != 0, 0)) {
+                if (unsure) {
+                    const uint32_t jt = L.rowt >> 24;
+                    const ExactTimes e = exact_times(seed, L.cell, L.node, a.type_mean[S.type_base + jt],
+                                                     a.type_sd[S.type_base + jt], t_max);
+                    sl = e.l;
+                    sr = e.r;
+                    if (e.rej)
+                        atomicAdd(n_rej, e.rej);
+                    cmp = true;
+                }
+            }
+            again = !cmp;
+
+            if (cmp) {
+                // daughters (proliferation.cu:317-381): out of time ->
+                // tallied, f/2 <= phi -> dropped, else divides later
+                const uint32_t k1 = L.k + 1;
+                const bool rec_l = sl > 0.0f;
+                const bool rec_r = sr > 0.0f;
+                const bool can = k1 < L.kcap;
+                const bool div_l = !rec_l & can;
+                const bool div_r = !rec_r & can;
+                const uint32_t nrec = (uint32_t)rec_l + (uint32_t)rec_r;
+                if (all_in) {
+                    lds_add(L.tb + __umul24(k1, T4), nrec);
+                } else if (L.tb != kNoWindow) {
+                    lds_add(L.tb + __umul24(k1, T4), nrec);
+                } else if (nrec) {
+                    atomicAdd(&a.tally[S.tally_base + (uint64_t)(L.rowt & 0xFFFFFFu) * kdim * T + types[L.rowt >> 24].file +
+                                       (uint64_t)k1 * T],
+                              (unsigned long long)nrec);
+                }
+                // right daughter's completion time, at level k1 (which holds
+                // no pending entry, so the store is harmless when it is not
+                // pushed)
+                *(float *)(stk + __umul24(k1, kStride)) = sr;
+                // next: the left daughter, else the lowest pending level (the
+                // right daughter's if it divides, else fl levels up)
+                const N up = (N)(div_l ? 0u : 1u);
+                const uint32_t sh = (div_l | div_r) ? 0u : fl + 1u;
+                L.node = ((L.node << 1) >> sh) | up;
+                L.pend = (((L.pend << 1) | (N)(div_r ? 1u : 0u)) >> sh) & ~up;
+                L.k = k1 - sh;
+                L.s = div_l ? sl : (div_r ? sr : sp);
+            }
+        }
+        redoing = __ballot(again);
+    }
+
+    Counts n = {0, 0, 0, 0, 0};
+    if (lane == 0) {
+        n.div = w_div;
+        n.lost = w_lost;
+        n.cells = w_cells;
+        n.pool = w_pool;
+    }
+    flush_counts(n, a.counters + (size_t)set * kCounterCopies * kNumCounters, lane, red);
+    const uint64_t gbase = S.tally_base + (uint64_t)(row_lo - S.row_base) * kdim * T;
+    for (uint32_t i = tid; i < win_len; i += bdim) {
+        const uint32_t c = win[i];
+        if (c)
+            atomicAdd(&a.tally[gbase + i], (unsigned long long)c);
+    }
+}
+
 __global__ void debug_draws_kernel(uint64_t seed, const uint64_t *cell, const uint64_t *node,
                                    const uint32_t *attempt, uint64_t n, uint32_t *words, double *z)
 {
@@ -663,14 +1305,22 @@ __global__ void debug_draws_kernel(uint64_t seed, const uint64_t *cell, const ui
 }  // namespace
 
 size_t sim_lds_bytes(uint32_t win_rows, uint32_t kdim, uint32_t n_types, uint32_t stack_levels, uint32_t block_size,
-                     uint32_t lds_rows)
+                     uint32_t lds_rows, bool filter)
 {
-    const size_t tables = kMathTableBytes + (sizeof(dev::Coeffs) + 15) / 16 * 16 + ((size_t)n_types * 28 + 15) / 16 * 16 +
-                          (lds_rows ? ((size_t)(2 * lds_rows + 1) * 4 + 15) / 16 * 16 : 0) + kSimSharedBytes;
-    const size_t waves = (size_t)(block_size / kWave) * sim_wave_lds_bytes();
-    const size_t win = ((size_t)win_rows * kdim * n_types * 4 + 4 + 15) / 16 * 16;
-    const size_t stk = (size_t)stack_levels * block_size * sizeof(double);
-    return tables + waves + win + stk;
+    const size_t types = filter ? filter_type_bytes(n_types)
+                                : kMathTableBytes + (sizeof(dev::Coeffs) + 15) / 16 * 16 + ((size_t)n_types * 28 + 15) / 16 * 16;
+    const size_t rows = lds_rows ? ((size_t)(2 * lds_rows + 1) * 4 + 15) / 16 * 16 : 0;
+    const size_t waves = (size_t)(block_size / kWave) * (filter ? filter_wave_bytes() : sim_wave_lds_bytes());
+    const size_t win = filter ? ((size_t)win_rows * kdim * n_types * 4 + 15) / 16 * 16
+                              : ((size_t)win_rows * kdim * n_types * 4 + 4 + 15) / 16 * 16;
+    const size_t stk = sim_stack_bytes(stack_levels, block_size, filter);
+    return types + rows + kSimSharedBytes + waves + win + stk;
+}
+
+// One workgroup's lane stacks (stack_levels 0: none in LDS).
+size_t sim_stack_bytes(uint32_t stack_levels, uint32_t block_size, bool filter)
+{
+    return (size_t)block_size * stack_levels * (filter ? sizeof(float) : sizeof(double));
 }
 
 hipError_t launch_zero(unsigned long long *p, uint64_t n, hipStream_t st)
@@ -684,29 +1334,34 @@ hipError_t launch_zero(unsigned long long *p, uint64_t n, hipStream_t st)
     return hipGetLastError();
 }
 
-template <bool GStack>
-void launch_sim_as(const RunArgs &a, const LaunchShape &ls, hipStream_t st)
+// The kernel of a launch: filtered tests or not, row tables in LDS, 32-bit
+// heap indices and level masks (trees of at most 31 generations), lane stacks
+// in device memory.
+template <bool RowsLds, typename N, bool GStack>
+auto sim_kernel_as(bool filter)
 {
-    const dim3 g(ls.blocks), b(ls.block_size);
-    const bool narrow = a.kdim <= 32;  // heap indices and level masks fit 32 bits
-    if (a.rows_in_lds && narrow)
-        hipLaunchKernelGGL((sim_kernel<true, uint32_t, GStack>), g, b, ls.lds_bytes, st, a);
-    else if (a.rows_in_lds)
-        hipLaunchKernelGGL((sim_kernel<true, uint64_t, GStack>), g, b, ls.lds_bytes, st, a);
-    else if (narrow)
-        hipLaunchKernelGGL((sim_kernel<false, uint32_t, GStack>), g, b, ls.lds_bytes, st, a);
-    else
-        hipLaunchKernelGGL((sim_kernel<false, uint64_t, GStack>), g, b, ls.lds_bytes, st, a);
+    return filter ? sim_filter_kernel<RowsLds, N, GStack> : sim_kernel<RowsLds, N, GStack>;
+}
+
+template <bool GStack>
+auto sim_kernel_as(bool filter, bool rows_in_lds, bool narrow)
+{
+    if (rows_in_lds)
+        return narrow ? sim_kernel_as<true, uint32_t, GStack>(filter) : sim_kernel_as<true, uint64_t, GStack>(filter);
+    return narrow ? sim_kernel_as<false, uint32_t, GStack>(filter) : sim_kernel_as<false, uint64_t, GStack>(filter);
+}
+
+auto sim_kernel_of(bool rows_in_lds, uint32_t kdim, bool gstack, bool filter)
+{
+    return gstack ? sim_kernel_as<true>(filter, rows_in_lds, kdim <= 32) : sim_kernel_as<false>(filter, rows_in_lds, kdim <= 32);
 }
 
 hipError_t launch_sim(const RunArgs &a, const LaunchShape &ls, hipStream_t st)
 {
     if (a.n_cells == 0)
         return hipSuccess;
-    if (a.gstack)
-        launch_sim_as<true>(a, ls, st);
-    else
-        launch_sim_as<false>(a, ls, st);
+    hipLaunchKernelGGL(sim_kernel_of(a.rows_in_lds != 0, a.kdim, a.gstack != nullptr, a.filter != 0), dim3(ls.blocks),
+                       dim3(ls.block_size), ls.lds_bytes, st, a);
     return hipGetLastError();
 }
 
@@ -721,28 +1376,11 @@ hipError_t launch_debug_draws(uint64_t seed, const uint64_t *cell, const uint64_
     return hipGetLastError();
 }
 
-template <bool GStack>
-hipError_t sim_occupancy_as(int block_size, size_t lds_bytes, bool rows_in_lds, uint32_t kdim, int *blocks_per_cu)
-{
-    const bool narrow = kdim <= 32;
-    if (rows_in_lds && narrow)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, sim_kernel<true, uint32_t, GStack>,
-                                                            block_size, lds_bytes);
-    if (rows_in_lds)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, sim_kernel<true, uint64_t, GStack>,
-                                                            block_size, lds_bytes);
-    if (narrow)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, sim_kernel<false, uint32_t, GStack>,
-                                                            block_size, lds_bytes);
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, sim_kernel<false, uint64_t, GStack>,
-                                                        block_size, lds_bytes);
-}
-
-hipError_t sim_occupancy(int block_size, size_t lds_bytes, bool rows_in_lds, uint32_t kdim, bool gstack,
+hipError_t sim_occupancy(int block_size, size_t lds_bytes, bool rows_in_lds, uint32_t kdim, bool gstack, bool filter,
                          int *blocks_per_cu)
 {
-    return gstack ? sim_occupancy_as<true>(block_size, lds_bytes, rows_in_lds, kdim, blocks_per_cu)
-                  : sim_occupancy_as<false>(block_size, lds_bytes, rows_in_lds, kdim, blocks_per_cu);
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, sim_kernel_of(rows_in_lds, kdim, gstack, filter),
+                                                        block_size, lds_bytes);
 }
 
 }  // namespace procell

@@ -174,6 +174,21 @@ double row_cost(const Setup &s, uint32_t row)
     return w;
 }
 
+// row_cost of every row.  It depends on the row through its generation cap
+// alone, so it is evaluated once per cap (at 1024 rows, 5 types and 11 caps:
+// 0.3 ms of erfc evaluations -> 4 us, twice per plan).
+static std::vector<double> row_costs(const Setup &s)
+{
+    std::vector<double> by_cap(256, -1.0), w(s.v.size());
+    for (uint32_t r = 0; r < (uint32_t)w.size(); ++r) {
+        double &c = by_cap[s.row_info[r] & 0xFFu];
+        if (c < 0.0)
+            c = row_cost(s, r);
+        w[r] = c;
+    }
+    return w;
+}
+
 // Split the initial cells into contiguous segments whose cumulative costs end
 // at the fractions cum[0] < cum[1] < ... < cum[g-1] = 1 of the total.
 void split_segments(const Setup &s, const std::vector<double> &cum, std::vector<uint64_t> &begin,
@@ -184,12 +199,10 @@ void split_segments(const Setup &s, const std::vector<double> &cum, std::vector<
     begin.assign(g + 1, s.n_cells);
     row_of.assign(g, n_rows ? n_rows - 1 : 0);
     begin[0] = 0;
-    std::vector<double> w(n_rows);
+    const std::vector<double> w = row_costs(s);
     double total = 0.0;
-    for (uint32_t r = 0; r < n_rows; ++r) {
-        w[r] = row_cost(s, r);
+    for (uint32_t r = 0; r < n_rows; ++r)
         total += w[r] * (double)(s.start[r + 1] - s.start[r]);
-    }
     uint32_t next = 1;
     double acc = 0.0;
     for (uint32_t r = 0; r < n_rows && next < g; ++r) {
@@ -215,10 +228,11 @@ void split_segments(const Setup &s, const std::vector<double> &cum, std::vector<
 // Expected work of a set (sum of row costs over its cells).
 double set_cost(const Setup &s)
 {
-    double w = 0.0;
+    const std::vector<double> w = row_costs(s);
+    double total = 0.0;
     for (uint32_t r = 0; r < (uint32_t)s.v.size(); ++r)
-        w += row_cost(s, r) * (double)(s.start[r + 1] - s.start[r]);
-    return w;
+        total += w[r] * (double)(s.start[r + 1] - s.start[r]);
+    return total;
 }
 
 void fill_stats(const unsigned long long *cnt, const int64_t *tally, size_t tally_len, procell_stats &st)
