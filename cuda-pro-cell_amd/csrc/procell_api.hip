@@ -149,14 +149,15 @@ bool filter_covers(const std::vector<Setup> &sets)
 
 // Segments per resident workgroup of a single set, from the expected
 // lane-steps per resident workgroup.  Filtered kernel, 3 workgroups of 512 per
-// CU, the five-type histogram at 1e6 cells (4.6e3 lane-steps), 1e7 (4.6e4)
-// and 1e8 (4.6e5), microseconds per run with 1 / 2 / 3 / 4 segments:
-// 39 / 44 / 51 / 58, 154 / 143 / 153 / 160, 1292 / 1213 / 1103 / 1099.
+// CU, the five-type histogram at 1e6 cells (4.6e3 lane-steps), 3e6 (1.4e4),
+// 1e7 (4.6e4) and 1e8 (4.6e5), microseconds per run with 1 / 2 / 3 / 4
+// segments: 36 / 38 / 45 / 51, 66 / 59 / 66 / 74, 172 / 139 / 141 / 147,
+// 1484 / 1185 / 1094 / 1096.
 uint32_t segments_per_workgroup(double lane_steps, bool filter)
 {
     if (!filter)
         return kSegmentsPerWorkgroup;
-    return lane_steps < 1.5e4 ? 1 : lane_steps < 1.5e5 ? 2 : 4;
+    return lane_steps < 8e3 ? 1 : lane_steps < 1.5e5 ? 2 : 3;
 }
 
 // A plan over n_sets parameter sets (1: a plain run).  Rows, cells, type
@@ -313,6 +314,14 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     const size_t row_bytes = (size_t)kdim * T * 4;
     uint32_t win_rows = budget > base + 16 ? (uint32_t)((budget - base - 16) / row_bytes) : 0;
 
+    // the sets in the order their cells are simulated: the filtered kernel's
+    // rows by decreasing cost, so that the runs end with short trees
+    std::vector<Setup> ordered(filter ? n_sets : 0);
+    std::vector<std::vector<uint32_t>> file_row(filter ? n_sets : 0);
+    for (uint32_t i = 0; i < n_sets && filter; ++i)
+        ordered[i] = order_rows(pl->setups[i], file_row[i]);
+    const std::vector<Setup> &lay = filter ? ordered : pl->setups;
+
     // ---- segments: one per workgroup, each within one set ----
     // `per_wg` segments per resident workgroup in total, of about equal
     // expected work: workgroups beyond the resident ones start as others
@@ -321,17 +330,17 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     // least one).
     const uint32_t resident = (uint32_t)((int64_t)n_cu * occ);
     const uint32_t per_wg = tu.segments   ? std::min<uint32_t>(tu.segments, 64)
-                            : n_sets == 1 ? segments_per_workgroup(set_cost(pl->setups[0]) / resident, filter)
+                            : n_sets == 1 ? segments_per_workgroup(set_cost(lay[0]) / resident, filter)
                                           : kBatchSegmentsPerWorkgroup;
     std::vector<uint32_t> g_set(n_sets, 1);
     if (n_sets == 1) {
         g_set[0] = (uint32_t)std::min<uint64_t>((uint64_t)resident * per_wg,
-                                                std::max<uint64_t>(1, (pl->setups[0].n_cells + 63) / 64));
+                                                std::max<uint64_t>(1, (lay[0].n_cells + 63) / 64));
     } else {
         std::vector<double> w(n_sets);
         double wt = 0.0;
         for (uint32_t i = 0; i < n_sets; ++i) {
-            w[i] = set_cost(pl->setups[i]);
+            w[i] = set_cost(lay[i]);
             wt += w[i];
         }
         const double target = (double)per_wg * (double)resident;
@@ -361,7 +370,7 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     };
     std::vector<Seg> segs;
     for (uint32_t i = 0; i < n_sets; ++i) {
-        const Setup &s = pl->setups[i];
+        const Setup &s = lay[i];
         const uint32_t gi = g_set[i];
         std::vector<double> wseg(gi, 1.0);
         if (n_sets == 1 && per_wg > 1 && gi == resident * per_wg) {
@@ -400,7 +409,7 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     // no more window rows than a segment spans
     uint32_t span = 1;
     for (uint32_t k = 0; k < g; ++k) {
-        const Setup &s = pl->setups[seg_set[k]];
+        const Setup &s = lay[seg_set[k]];
         const SetInfo &si = info[seg_set[k]];
         if (!s.n_cells)
             continue;
@@ -414,7 +423,7 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     win_rows = std::min(win_rows, span);
     // u32 window counters must not overflow: bound the leaves any window can see
     for (uint32_t k = 0; k < g && win_rows; ++k) {
-        const Setup &s = pl->setups[seg_set[k]];
+        const Setup &s = lay[seg_set[k]];
         const uint32_t r0 = seg_row[k] - info[seg_set[k]].row_base;
         const uint32_t nr = (uint32_t)s.v.size();
         double bound = 0.0;
@@ -447,6 +456,7 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     off = align_up(off, 256);
     const size_t o_rs = off; off = align_up(off + (size_t)(n_rows + 1) * 4, 256);
     const size_t o_ri = off; off = align_up(off + (size_t)(n_rows + 1) * 4, 256);
+    const size_t o_rc = off; off = align_up(off + (filter ? (size_t)n_rows * 4 : 0), 256);
     const size_t o_cum = off; off = align_up(off + (size_t)n_types_tot * 8, 256);
     const size_t o_mean = off; off = align_up(off + (size_t)n_types_tot * 8, 256);
     const size_t o_sd = off; off = align_up(off + (size_t)n_types_tot * 8, 256);
@@ -488,6 +498,7 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
 
     a.row_start = (const uint32_t *)(dbase + o_rs);
     a.row_info = (const uint32_t *)(dbase + o_ri);
+    a.row_cell = (const uint32_t *)(dbase + o_rc);
     a.type_cum = (const double *)(dbase + o_cum);
     a.type_mean = (const double *)(dbase + o_mean);
     a.type_sd = (const double *)(dbase + o_sd);
@@ -500,15 +511,21 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     a.set_seed = (const uint64_t *)(dbase + o_seed);
     pl->d_seeds = (uint64_t *)(dbase + o_seed);
     // concatenated host tables (cells < 2^32)
-    std::vector<uint32_t> start32, info32;
+    std::vector<uint32_t> start32, info32, cell32;
     std::vector<double> cum, mean, sd;
     std::vector<uint32_t> tfile;
     start32.reserve(n_rows + 1);
     for (uint32_t i = 0; i < n_sets; ++i) {
-        const Setup &s = pl->setups[i];
+        const Setup &s = lay[i];
         for (size_t r = 0; r < s.v.size(); ++r) {
             start32.push_back((uint32_t)(info[i].cell_base + s.start[r]));
-            info32.push_back(s.row_info[r]);
+            if (!filter) {
+                info32.push_back(s.row_info[r]);
+                continue;
+            }
+            const uint32_t fr = file_row[i][r];
+            info32.push_back(row_word(s.row_info[r] & 0xFFu, (s.row_info[r] >> 8) & 1u, fr));
+            cell32.push_back((uint32_t)(pl->setups[i].start[fr] - s.start[r]));
         }
         const uint32_t Ti = info[i].n_types;
         for (uint32_t j = 0; j < Ti; ++j) {
@@ -524,6 +541,7 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
         return bytes == 0 || hipMemcpyAsync(dbase + o, src, bytes, hipMemcpyHostToDevice, pl->stream) == hipSuccess;
     };
     if (!up(o_rs, start32.data(), start32.size() * 4) || !up(o_ri, info32.data(), info32.size() * 4) ||
+        !up(o_rc, cell32.data(), cell32.size() * 4) ||
         !up(o_cum, cum.data(), cum.size() * 8) || !up(o_mean, mean.data(), mean.size() * 8) ||
         !up(o_sd, sd.data(), sd.size() * 8) || !up(o_tf, tfile.data(), tfile.size() * 4) ||
         !up(o_sb, seg_begin.data(), seg_begin.size() * 8) || !up(o_se, seg_end.data(), seg_end.size() * 8) || !up(o_sr, seg_row.data(), seg_row.size() * 4) ||

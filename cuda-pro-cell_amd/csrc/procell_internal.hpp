@@ -75,7 +75,8 @@ struct RunArgs {
     const uint64_t *set_seed;    // [n_sets] seeds of a batch run (n_sets > 1)
     const uint32_t *seg_set;     // [segments] set of each segment
     const uint32_t *row_start;   // [n_rows + 1] first cell of each nonzero row (cells < 2^32)
-    const uint32_t *row_info;    // [n_rows]: generation cap | (value >= phi) << 8
+    const uint32_t *row_info;    // [n_rows]: generation cap | (value >= phi) << 8; sim_filter_kernel: row_word()
+    const uint32_t *row_cell;    // [n_rows] (sim_filter_kernel) cell id of a cell in the set minus its place in row order
     const double *type_cum;      // [n_types] sorted order
     const double *type_mean;
     const double *type_sd;
@@ -90,6 +91,14 @@ struct RunArgs {
 
 // Most threads of a workgroup of sim_filter_kernel.
 constexpr uint32_t kFilterThreads = 512;
+
+// A row of sim_filter_kernel, which takes a set's rows in order of decreasing
+// cost: generation cap (at most 62), (value >= phi), and the row's place in
+// the file order of its set (below 2^24).
+inline uint32_t row_word(uint32_t cap, bool ge_phi, uint32_t file_row)
+{
+    return cap | (ge_phi ? 1u : 0u) << 6 | file_row << 7;
+}
 
 struct LaunchShape {
     int blocks;             // = segments

@@ -787,6 +787,9 @@ __device__ __forceinline__ ExactTimes exact_times(uint64_t seed, uint32_t cell, 
 // instead of 4 gave 1.24 -> 1.09 ms, which holds it to 80 registers (the
 // 64-bit evaluation spills a few, in its own branch only).  The tree logic is
 // arranged for few instructions and few values carried round the loop:
+//  * a set's rows come in order of decreasing cost (the host's order_rows), so
+//    the last trees of a segment, and of the run, are its shallowest: 0.143 ->
+//    0.136 ms at 1e7 cells.
 //  * a lane's pending right daughters are a mask relative to its level (bit i:
 //    level k - i), with one more bit for level 0 that no daughter uses.  Going
 //    down shifts the mask up by one; "the left daughter does not divide" takes
@@ -832,7 +835,7 @@ struct FilterLane {
     float err;          // bound of |s - its 64-bit value| at any level of the tree
     uint32_t cell;      // initial cell, relative to its set
     uint32_t tb;        // LDS address of the window entry (row, generation 0, type), or kNoWindow
-    uint32_t rowt;      // row relative to the set's first row | sorted type << 24
+    uint32_t rowt;      // row in the set's file order | sorted type << 24
     uint32_t k, kcap;
 };
 
@@ -932,11 +935,12 @@ __global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a
     for (uint32_t k = 0; k < 8; ++k)
         lim8[k] = uni(k + 1 < T ? lims[k] : 0u);
     // Row boundaries of the wavefront's root steps (as in sim_kernel)
-    uint32_t rb = row_lo, bnd = 0, rinfo = 0;
+    uint32_t rb = row_lo, bnd = 0, rinfo = 0, rcell = 0;
     auto load_rows = [&]() {
         const uint32_t r1 = rb + 1 + lane;
         bnd = r1 <= a.n_rows ? rs[r1] : 0xFFFFFFFFu;
         rinfo = rb + lane < a.n_rows ? ri[rb + lane] : 0u;
+        rcell = rb + lane < a.n_rows ? a.row_cell[rb + lane] : 0u;
     };
     load_rows();
 
@@ -963,7 +967,6 @@ __global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a
                     const uint64_t c_cur = seg_begin + c_off;
                     const uint32_t n_valid = uni((uint32_t)min<uint64_t>(kWave, seg_cells - c_off));
                     const bool valid = lane < n_valid;
-                    const uint32_t cell = cell0 + (uint32_t)c_off + lane;
                     // rows of the step's cells (cell ids < 2^32): move rb to the
                     // row of c_cur, then count the boundaries inside the step
                     const uint32_t c32 = (uint32_t)c_cur;
@@ -973,15 +976,17 @@ __global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a
                     }
                     const uint32_t nb = uni((uint32_t)__popcll(__ballot((uint64_t)bnd < c_cur + n_valid)));
                     uint32_t rrel = 0;  // boundaries at or below this lane's cell
-                    uint32_t info = uni(rinfo);
+                    uint32_t info = uni(rinfo), dcell = uni(rcell);
                     if (nb) {
                         for (uint32_t j = 0; j < nb; ++j)
                             rrel += lane >= (uint32_t)__builtin_amdgcn_readlane((int)bnd, (int)j) - c32 ? 1u : 0u;
                         info = (uint32_t)__shfl(rinfo, (int)rrel);
+                        dcell = (uint32_t)__shfl(rcell, (int)rrel);
                     }
-                    const uint32_t row = rb + rrel;
-                    const uint32_t kc = info & 0xFFu;
-                    const bool ge_phi = (info >> 8) & 1u;
+                    const uint32_t row = rb + rrel, file_row = info >> 7;
+                    const uint32_t kc = info & 63u;
+                    const bool ge_phi = (info >> 6) & 1u;
+                    const uint32_t cell = cell0 + (uint32_t)c_off + lane + dcell;
                     // one block per initial cell: type uniform (word 0), phase
                     // (word 1) and the first timer's Box-Muller pair (words 2, 3)
                     const Words w = dev::draw_block(seed, cell, 0, 0);
@@ -1054,11 +1059,11 @@ __global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a
                         uint64_t pend = __ballot(rec_ok && !in_win);
                         while (pend) {
                             const uint32_t leader = (uint32_t)__builtin_ctzll(pend);
-                            const uint32_t row_l = uni(__shfl(row, (int)leader));
+                            const uint32_t row_l = uni(__shfl(file_row, (int)leader));
                             const uint32_t tf_l = uni(__shfl(ty.file, (int)leader));
-                            const uint64_t same = __ballot(rec_ok && !in_win && row == row_l && ty.file == tf_l);
+                            const uint64_t same = __ballot(rec_ok && !in_win && file_row == row_l && ty.file == tf_l);
                             if (lane == leader)
-                                atomicAdd(&a.tally[S.tally_base + (uint64_t)(row_l - S.row_base) * kdim * T + tf_l],
+                                atomicAdd(&a.tally[S.tally_base + (uint64_t)row_l * kdim * T + tf_l],
                                           (unsigned long long)__popcll(same));
                             pend &= ~same;
                         }
@@ -1066,7 +1071,7 @@ __global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a
                     // dividing cells: buffered for the hand-outs
                     if (divides)
                         ent[lane_rank(dmask)] = FilterEntry{s0, ty.mean, ty.sd, err, cell, in_win ? tb : kNoWindow,
-                                                            (row - S.row_base) | (jt << 24), kc};
+                                                            file_row | (jt << 24), kc};
                     rpos = 0;
                     rn = uni((uint32_t)__popcll(dmask));
                     __builtin_amdgcn_wave_barrier();
@@ -1269,6 +1274,9 @@ __global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a
         redoing = __ballot(again);
     }
 
+    // places of the first 64 window rows, read ahead of the barrier
+    const uint32_t n_win = min(a.win_rows, a.n_rows - row_lo);
+    uint32_t place = lane < n_win ? ri[row_lo + lane] >> 7 : 0u;
     Counts n = {0, 0, 0, 0, 0};
     if (lane == 0) {
         n.div = w_div;
@@ -1277,11 +1285,20 @@ __global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a
         n.pool = w_pool;
     }
     flush_counts(n, a.counters + (size_t)set * kCounterCopies * kNumCounters, lane, red);
-    const uint64_t gbase = S.tally_base + (uint64_t)(row_lo - S.row_base) * kdim * T;
-    for (uint32_t i = tid; i < win_len; i += bdim) {
-        const uint32_t c = win[i];
-        if (c)
-            atomicAdd(&a.tally[gbase + i], (unsigned long long)c);
+    // one wavefront per window row, to the row's place in file order
+    const uint32_t row_len = kdim * T;
+    for (uint32_t r0 = 0; r0 < n_win; r0 += kWave) {
+        if (r0)
+            place = r0 + lane < n_win ? ri[row_lo + r0 + lane] >> 7 : 0u;
+        for (uint32_t r = r0 + wave; r < min(r0 + kWave, n_win); r += n_waves) {
+            unsigned long long *row =
+                &a.tally[S.tally_base + (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)place, (int)(r - r0)) * row_len];
+            for (uint32_t i = lane; i < row_len; i += kWave) {
+                const uint32_t c = win[r * row_len + i];
+                if (c)
+                    atomicAdd(&row[i], (unsigned long long)c);
+            }
+        }
     }
 }
 

@@ -189,6 +189,26 @@ static std::vector<double> row_costs(const Setup &s)
     return w;
 }
 
+Setup order_rows(const Setup &s, std::vector<uint32_t> &file_row)
+{
+    const std::vector<double> w = row_costs(s);
+    const size_t n = w.size();
+    file_row.resize(n);
+    for (size_t i = 0; i < n; ++i)
+        file_row[i] = (uint32_t)i;
+    std::stable_sort(file_row.begin(), file_row.end(), [&](uint32_t x, uint32_t y) { return w[x] > w[y]; });
+    Setup o = s;
+    uint64_t at = 0;
+    for (size_t i = 0; i < n; ++i) {
+        const uint32_t r = file_row[i];
+        o.v[i] = s.v[r];
+        o.row_info[i] = s.row_info[r];
+        o.start[i] = at;
+        at += s.start[r + 1] - s.start[r];
+    }
+    return o;
+}
+
 // Split the initial cells into contiguous segments whose cumulative costs end
 // at the fractions cum[0] < cum[1] < ... < cum[g-1] = 1 of the total.
 void split_segments(const Setup &s, const std::vector<double> &cum, std::vector<uint64_t> &begin,

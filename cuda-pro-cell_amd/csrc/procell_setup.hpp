@@ -55,6 +55,10 @@ int build_setup(const procell_params *p, Setup &s, bool want_bins);
 // Expected lane-steps of one initial cell of row `row` and of a whole set.
 double row_cost(const Setup &s, uint32_t row);
 double set_cost(const Setup &s);
+// The same problem with its rows in order of decreasing cost per cell (file
+// order among equals): values, starts and row_info permuted, file_row[i] the
+// place of the i-th row in s.  Cell starts count the cells in the new order.
+Setup order_rows(const Setup &s, std::vector<uint32_t> &file_row);
 // Contiguous segments of initial cells whose cumulative expected costs end
 // at the fractions cum[0] < ... < cum[g-1] = 1: begin[g+1], row_of[g].
 void split_segments(const Setup &s, const std::vector<double> &cum, std::vector<uint64_t> &begin,
