@@ -61,6 +61,18 @@ struct procell_plan {
     bool timed = false;            // a run has recorded its events
     uint64_t batch_runs = 0;
     bool ran = false;
+    // results: bins of the tally entries, made at a set's first result, and
+    // pinned memory for downloads, made at the plan's second (a plan used once
+    // would pay for it more than it gains); `stage` holds the sets
+    // [stage_set, stage_end) of run `stage_run`
+    std::mutex result_mu;
+    std::vector<std::vector<int32_t>> bin_of;
+    uint64_t results = 0, run_id = 0, stage_run = 0;
+    uint32_t stage_set = 0, stage_end = 0;
+    uint64_t next_run = 0;             // a download of set next_set of this run brings next_n sets
+    uint32_t next_set = 0, next_n = 1;
+    void *stage = nullptr;
+    size_t stage_bytes = 0;
     // copies of the inputs (the autotuner re-creates the layout from them)
     std::vector<procell_params> params;
     std::vector<std::vector<procell_row>> rows;
@@ -124,6 +136,8 @@ void destroy_plan(procell_plan *pl)
             (void)hipEventDestroy(e);
     if (pl->h_seeds)
         (void)hipHostFree(pl->h_seeds);
+    if (pl->stage)
+        (void)hipHostFree(pl->stage);
     if (pl->d_block && pl->own_block)
         (void)hipFree(pl->d_block);
     if (pl->own_stream && pl->stream)
@@ -421,15 +435,25 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
         span = std::max(span, lr - (seg_row[k] - si.row_base) + 1);
     }
     win_rows = std::min(win_rows, span);
-    // u32 window counters must not overflow: bound the leaves any window can see
+    // u32 window counters must not overflow: bound the leaves any window can
+    // see.  leaves[]: those of the rows before each row, one sum per set (a row
+    // counts for 1e10 at most, which is over the limit by itself and keeps the
+    // differences of the sums exact enough)
+    std::vector<double> leaves;
+    for (uint32_t i = 0; i < n_sets; ++i) {
+        const Setup &s = lay[i];
+        double sum = 0.0;
+        for (size_t r = 0; r < s.v.size(); ++r) {
+            leaves.push_back(sum);
+            sum += std::min(1e10, (double)(s.start[r + 1] - s.start[r]) * ldexp(1.0, (int)(s.row_info[r] & 0xFFu)));
+        }
+        leaves.push_back(sum);
+    }
     for (uint32_t k = 0; k < g && win_rows; ++k) {
-        const Setup &s = lay[seg_set[k]];
+        const uint32_t nr = (uint32_t)lay[seg_set[k]].v.size();
         const uint32_t r0 = seg_row[k] - info[seg_set[k]].row_base;
-        const uint32_t nr = (uint32_t)s.v.size();
-        double bound = 0.0;
-        for (uint32_t r = r0; r < std::min<uint32_t>(nr, r0 + win_rows); ++r)
-            bound += (double)(s.start[r + 1] - s.start[r]) * ldexp(1.0, (int)(s.row_info[r] & 0xFFu));
-        if (bound >= 4.0e9)
+        const double *before = &leaves[info[seg_set[k]].row_base + seg_set[k]];
+        if (before[std::min<uint32_t>(nr, r0 + win_rows)] - before[std::min(nr, r0)] >= 4.0e9)
             win_rows = 0;
     }
     // the window must not cost a resident workgroup (LDS allocation granularity)
@@ -537,15 +561,26 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     }
     start32.push_back((uint32_t)n_cells);
     info32.push_back(0u);
-    auto up = [&](size_t o, const void *src, size_t bytes) {
-        return bytes == 0 || hipMemcpyAsync(dbase + o, src, bytes, hipMemcpyHostToDevice, pl->stream) == hipSuccess;
+    // one copy for all tables (as separate copies of a few hundred bytes to a
+    // few KB each, twelve of them took 52 us; one takes 14)
+    std::vector<char> image(o_seed - o_rs, 0);
+    auto put = [&](size_t o, const void *src, size_t bytes) {
+        if (bytes)
+            memcpy(&image[o - o_rs], src, bytes);
     };
-    if (!up(o_rs, start32.data(), start32.size() * 4) || !up(o_ri, info32.data(), info32.size() * 4) ||
-        !up(o_rc, cell32.data(), cell32.size() * 4) ||
-        !up(o_cum, cum.data(), cum.size() * 8) || !up(o_mean, mean.data(), mean.size() * 8) ||
-        !up(o_sd, sd.data(), sd.size() * 8) || !up(o_tf, tfile.data(), tfile.size() * 4) ||
-        !up(o_sb, seg_begin.data(), seg_begin.size() * 8) || !up(o_se, seg_end.data(), seg_end.size() * 8) || !up(o_sr, seg_row.data(), seg_row.size() * 4) ||
-        !up(o_ss, seg_set.data(), seg_set.size() * 4) || !up(o_info, info.data(), info.size() * sizeof(SetInfo)))
+    put(o_rs, start32.data(), start32.size() * 4);
+    put(o_ri, info32.data(), info32.size() * 4);
+    put(o_rc, cell32.data(), cell32.size() * 4);
+    put(o_cum, cum.data(), cum.size() * 8);
+    put(o_mean, mean.data(), mean.size() * 8);
+    put(o_sd, sd.data(), sd.size() * 8);
+    put(o_tf, tfile.data(), tfile.size() * 4);
+    put(o_sb, seg_begin.data(), seg_begin.size() * 8);
+    put(o_se, seg_end.data(), seg_end.size() * 8);
+    put(o_sr, seg_row.data(), seg_row.size() * 4);
+    put(o_ss, seg_set.data(), seg_set.size() * 4);
+    put(o_info, info.data(), info.size() * sizeof(SetInfo));
+    if (hipMemcpyAsync(dbase + o_rs, image.data(), image.size(), hipMemcpyHostToDevice, pl->stream) != hipSuccess)
         return fail(PROCELL_E_HIP);
     if (hipStreamSynchronize(pl->stream) != hipSuccess)
         return fail(PROCELL_E_HIP);
@@ -650,7 +685,76 @@ int run_plan(procell_plan *pl, const uint64_t *seeds, uint64_t seed, bool use_gr
         pl->timed = true;
     }
     ++pl->runs;
+    ++pl->run_id;
     pl->ran = true;
+    return PROCELL_OK;
+}
+
+// Downloads one set's counter copies and tally.  A batch's sets are usually
+// read one after the other, so a set that follows the last download brings
+// twice as many along, up to kStageBytes; they serve later calls until the
+// next run.  (512 sets one by one: two copies and a wait, about 35 us, each.)
+constexpr size_t kStageBytes = 8u << 20;
+
+int download_set(procell_plan *pl, uint32_t set, std::vector<unsigned long long> &counters, std::vector<int64_t> &tally)
+{
+    constexpr size_t kCntBytes = (size_t)kCounterCopies * kNumCounters * 8;
+    const uint32_t n_sets = pl->args.n_sets;
+    counters.resize(kCntBytes / 8);
+    tally.resize(pl->tally_len[set]);
+    auto fetch = [&](char *cnt, char *tal, uint32_t a, uint32_t b) -> int {
+        const size_t tal_bytes = (pl->tally_base[b - 1] + pl->tally_len[b - 1] - pl->tally_base[a]) * 8;
+        const char *d_cnt = (const char *)pl->args.counters + a * kCntBytes;
+        const char *d_tal = (const char *)(pl->args.tally + pl->tally_base[a]);
+        if (n_sets == 1 && tal == cnt + kCntBytes) {  // (a single set's counters and tally lie together)
+            HIP_TRY(hipMemcpyAsync(cnt, d_cnt, kCntBytes + tal_bytes, hipMemcpyDeviceToHost, pl->stream));
+        } else {
+            HIP_TRY(hipMemcpyAsync(cnt, d_cnt, (b - a) * kCntBytes, hipMemcpyDeviceToHost, pl->stream));
+            if (tal_bytes)
+                HIP_TRY(hipMemcpyAsync(tal, d_tal, tal_bytes, hipMemcpyDeviceToHost, pl->stream));
+        }
+        HIP_TRY(hipStreamSynchronize(pl->stream));
+        return PROCELL_OK;
+    };
+    std::lock_guard<std::mutex> lk(pl->result_mu);
+    if (n_sets == 1 || pl->stage_run != pl->run_id || set < pl->stage_set || set >= pl->stage_end) {  // (runs count from 1)
+        auto bytes_of = [&](uint32_t n) {
+            return n * kCntBytes + (pl->tally_base[set + n - 1] + pl->tally_len[set + n - 1] - pl->tally_base[set]) * 8;
+        };
+        uint32_t want = pl->next_run == pl->run_id && set == pl->next_set ? std::min(pl->next_n, n_sets - set) : 1;
+        while (want > 1 && bytes_of(want) > kStageBytes)
+            want /= 2;
+        const size_t need = bytes_of(want);
+        pl->next_run = pl->run_id;
+        pl->next_set = set + want;
+        pl->next_n = 2 * want;
+        pl->stage_run = 0;
+        if (pl->own_block && pl->results++ > 0 && need <= kStageBytes && need > pl->stage_bytes) {
+            if (pl->stage)
+                (void)hipHostFree(pl->stage);
+            pl->stage_bytes = n_sets > 1 ? kStageBytes : need;
+            if (hipHostMalloc(&pl->stage, pl->stage_bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                pl->stage = nullptr;
+                pl->stage_bytes = 0;
+            }
+        }
+        if (need > pl->stage_bytes) {  // no pinned memory: this set, straight to the caller's buffers
+            pl->next_set = set + 1;
+            return fetch((char *)counters.data(), (char *)tally.data(), set, set + 1);
+        }
+        const int rc = fetch((char *)pl->stage, (char *)pl->stage + want * kCntBytes, set, set + want);
+        if (rc != PROCELL_OK)
+            return rc;
+        pl->stage_run = pl->run_id;
+        pl->stage_set = set;
+        pl->stage_end = set + want;
+    }
+    const uint32_t n = pl->stage_end - pl->stage_set, i = set - pl->stage_set;
+    memcpy(counters.data(), (const char *)pl->stage + i * kCntBytes, kCntBytes);
+    if (!tally.empty())
+        memcpy(tally.data(), (const char *)pl->stage + n * kCntBytes + (pl->tally_base[set] - pl->tally_base[pl->stage_set]) * 8,
+               tally.size() * 8);
     return PROCELL_OK;
 }
 
@@ -663,14 +767,11 @@ int plan_result(procell_plan *pl, uint32_t set, procell_result *r)
     if (r->capacity && !(r->value && r->count))
         return PROCELL_E_INVALID;
     HIP_TRY(hipSetDevice(pl->device));
-    std::vector<unsigned long long> cnt_all((size_t)kCounterCopies * kNumCounters), cnt(kNumCounters, 0);
-    std::vector<int64_t> tally(tally_len);
-    HIP_TRY(hipMemcpyAsync(cnt_all.data(), pl->args.counters + (size_t)set * kCounterCopies * kNumCounters,
-                           cnt_all.size() * 8, hipMemcpyDeviceToHost, pl->stream));
-    if (tally_len)
-        HIP_TRY(hipMemcpyAsync(tally.data(), pl->args.tally + pl->tally_base[set], tally_len * 8,
-                               hipMemcpyDeviceToHost, pl->stream));
-    HIP_TRY(hipStreamSynchronize(pl->stream));
+    std::vector<unsigned long long> cnt_all, cnt(kNumCounters, 0);
+    std::vector<int64_t> tally;
+    const int rc = download_set(pl, set, cnt_all, tally);
+    if (rc != PROCELL_OK)
+        return rc;
     for (size_t i = 0; i < cnt_all.size(); ++i)
         cnt[i % kNumCounters] += cnt_all[i];
     procell_stats &st = r->stats;
@@ -690,7 +791,55 @@ int plan_result(procell_plan *pl, uint32_t set, procell_result *r)
             return PROCELL_E_CAPACITY;
         memcpy(r->raw_tally, tally.data(), tally_len * 8);
     }
-    return merge_tally(s, tally.data(), r);
+    const std::vector<int32_t> *bin_of = nullptr;
+    {
+        std::lock_guard<std::mutex> lk(pl->result_mu);
+        if (pl->bin_of.empty())
+            pl->bin_of.resize(pl->args.n_sets);
+        if (pl->bin_of[set].empty())
+            pl->bin_of[set] = index_bins(s);
+        bin_of = &pl->bin_of[set];
+    }
+    return merge_tally(s, *bin_of, tally.data(), r);
+}
+
+// Streams of procell_simulate calls: making and destroying one took 58 us of
+// a small call's 190.  Up to kKeptStreams idle ones per device wait for the
+// next call; a call takes one for itself and gives it back once its work has
+// ended, so concurrent calls never share one.
+constexpr int kKeptDevices = 64, kKeptStreams = 4;
+std::mutex g_stream_mu;
+hipStream_t g_streams[kKeptDevices][kKeptStreams];
+int g_n_streams[kKeptDevices];
+
+hipStream_t borrow_stream(int device)
+{
+    if (device < 0 || device >= kKeptDevices)
+        return nullptr;
+    {
+        std::lock_guard<std::mutex> lk(g_stream_mu);
+        if (g_n_streams[device] > 0)
+            return g_streams[device][--g_n_streams[device]];
+    }
+    int n_cu = 0;
+    hipStream_t st = nullptr;
+    if (check_device(device, &n_cu) != PROCELL_OK || hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess)
+        return nullptr;  // (the plan reports what is wrong)
+    return st;
+}
+
+void return_stream(int device, hipStream_t st)
+{
+    if (!st)
+        return;
+    if (hipSetDevice(device) == hipSuccess && hipStreamSynchronize(st) == hipSuccess) {
+        std::lock_guard<std::mutex> lk(g_stream_mu);
+        if (g_n_streams[device] < kKeptStreams) {
+            g_streams[device][g_n_streams[device]++] = st;
+            return;
+        }
+    }
+    (void)hipStreamDestroy(st);
 }
 
 // In host code `scratch` names a host-side stand-in, not device memory: the
@@ -930,15 +1079,16 @@ int procell_simulate(const procell_params *p, procell_result *r)
     if (!p || !r)
         return PROCELL_E_INVALID;
     procell_params q = *p;
-    q.stream = nullptr;
+    q.stream = borrow_stream(p->device);  // NULL: the plan makes its own
     procell_plan *pl = nullptr;
     int rc = create_plan(&q, 1, &pl);
-    if (rc != PROCELL_OK)
-        return rc;
-    rc = run_plan(pl, nullptr, p->seed);
-    if (rc == PROCELL_OK)
-        rc = plan_result(pl, 0, r);
-    destroy_plan(pl);
+    if (rc == PROCELL_OK) {
+        rc = run_plan(pl, nullptr, p->seed);
+        if (rc == PROCELL_OK)
+            rc = plan_result(pl, 0, r);
+        destroy_plan(pl);
+    }
+    return_stream(p->device, (hipStream_t)q.stream);
     return rc;
 }
 

@@ -1022,7 +1022,7 @@ __global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a
                     const float u1 = fmaf((float)w.w1, 0x1p-32f, 1.0f);
                     const float tau0 = fmaf(z0, ty.sd, ty.mean);
                     float s0 = fmaf(tau0, u1, -t_max32);
-                    const bool sure = (min_abs(tau0, s0) > err) & (tau0 > 0.0f) & pair_sure(w.w2);
+                    const bool sure = (int)(min_abs(tau0, s0) > err) & (int)(tau0 > 0.0f) & (int)pair_sure(w.w2);
                     if (__builtin_expect(__ballot(live && !sure) != 0, 0)) {
                         if (live && !sure) {
                             // the second candidate where the first is surely refused
@@ -1167,7 +1167,7 @@ __global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a
                 const float tr = fmaf(z1, L.sd, L.mean);
                 sl = L.s + tl;
                 sr = L.s + tr;
-                const bool fine = (fminf(fminf(tl, tr), min_abs(sl, sr)) > L.err) & pair_sure(w.w0);
+                const bool fine = (int)(fminf(fminf(tl, tr), min_abs(sl, sr)) > L.err) & (int)pair_sure(w.w0);
                 if (__builtin_expect(__ballot(!fine) != 0, 0)) {
                     if (!fine) {
                         // a timer surely < 0: that daughter continues in its
@@ -1245,8 +1245,8 @@ __global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a
                 const bool rec_l = sl > 0.0f;
                 const bool rec_r = sr > 0.0f;
                 const bool can = k1 < L.kcap;
-                const bool div_l = !rec_l & can;
-                const bool div_r = !rec_r & can;
+                const bool div_l = (int)!rec_l & (int)can;
+                const bool div_r = (int)!rec_r & (int)can;
                 const uint32_t nrec = (uint32_t)rec_l + (uint32_t)rec_r;
                 if (all_in) {
                     lds_add(L.tb + __umul24(k1, T4), nrec);
@@ -1264,7 +1264,7 @@ __global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a
                 // next: the left daughter, else the lowest pending level (the
                 // right daughter's if it divides, else fl levels up)
                 const N up = (N)(div_l ? 0u : 1u);
-                const uint32_t sh = (div_l | div_r) ? 0u : fl + 1u;
+                const uint32_t sh = ((int)div_l | (int)div_r) ? 0u : fl + 1u;
                 L.node = ((L.node << 1) >> sh) | up;
                 L.pend = (((L.pend << 1) | (N)(div_r ? 1u : 0u)) >> sh) & ~up;
                 L.k = k1 - sh;

@@ -845,7 +845,7 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
     c.n_sets = n;
     c.setups.resize(n);
     for (uint32_t i = 0; i < n; ++i) {
-        const int rc = build_setup(&ps[i], c.setups[i], want_bins);
+        const int rc = build_setup(&ps[i], c.setups[i], want_bins, false);
         if (rc != PROCELL_OK)
             return rc;
     }

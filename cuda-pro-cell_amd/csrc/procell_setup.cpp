@@ -46,7 +46,84 @@ double resolve_phi(const procell_params *p)
     return best;
 }
 
-int build_setup(const procell_params *p, Setup &s, bool want_bins)
+// Bits, biased exponent and mantissa of a double.
+static uint64_t double_bits(double x)
+{
+    uint64_t u;
+    memcpy(&u, &x, 8);
+    return u;
+}
+static uint64_t exponent(double x) { return double_bits(x) >> 52; }
+static uint64_t mantissa(double x) { return double_bits(x) & ((1ull << 52) - 1); }
+
+// Rows with value >= phi by mantissa.  Halving a normal number keeps its
+// mantissa, so the values v / 2^k of one exponent come in this order.
+static std::vector<std::pair<uint64_t, uint32_t>> rows_by_mantissa(const Setup &s)
+{
+    std::vector<std::pair<uint64_t, uint32_t>> rows;  // mantissa, row
+    rows.reserve(s.v.size());
+    for (size_t r = 0; r < s.v.size(); ++r)
+        if (s.v[r] >= s.phi)
+            rows.emplace_back(mantissa(s.v[r]), (uint32_t)r);
+    std::sort(rows.begin(), rows.end());
+    return rows;
+}
+
+// Output bin set (parser.cu:126-151): every v / 2^k >= phi, exact halving,
+// distinct, ascending.
+static void build_bins(Setup &s)
+{
+    if (exponent(s.phi) == 0) {
+        // phi below the smallest normal number: sorted as they come
+        for (double v : s.v) {
+            double f = v;
+            while (f >= s.phi) {
+                s.bins.push_back(f);
+                f = f / 2;
+            }
+        }
+        std::sort(s.bins.begin(), s.bins.end());
+        s.bins.erase(std::unique(s.bins.begin(), s.bins.end()), s.bins.end());
+        return;
+    }
+    // one exponent after the other, each in the order of the distinct
+    // mantissas (sorting the rows, not the several bins of each: 175 -> 50 us
+    // at 796 rows and 3706 bins)
+    std::vector<std::pair<uint64_t, uint64_t>> values;  // mantissa, largest exponent
+    uint64_t top = 0;
+    for (const auto &mr : rows_by_mantissa(s)) {
+        const uint64_t e = exponent(s.v[mr.second]);
+        top = std::max(top, e);
+        if (values.empty() || values.back().first != mr.first)
+            values.emplace_back(mr.first, e);
+        else
+            values.back().second = std::max(values.back().second, e);
+    }
+    const uint64_t first = exponent(s.phi);
+    for (uint64_t e = first; e <= top; ++e)
+        for (const auto &me : values)
+            if (me.second >= e && (e > first || me.first >= mantissa(s.phi))) {
+                const uint64_t u = e << 52 | me.first;
+                double f;
+                memcpy(&f, &u, 8);
+                s.bins.push_back(f);
+            }
+}
+
+// row_cost of every row depends on the row through its generation cap alone, so
+// it is evaluated once per cap (1024 rows, 5 types, 11 caps: 0.3 ms
+// of erfc evaluations -> 30 us, needed four times per plan).
+static void cost_caps(Setup &s)
+{
+    s.cap_cost.assign((size_t)s.kmax + 1, -1.0);
+    for (uint32_t r = 0; r < (uint32_t)s.v.size(); ++r) {
+        double &c = s.cap_cost[s.row_info[r] & 0xFFu];
+        if (c < 0.0)
+            c = row_cost(s, r);
+    }
+}
+
+int build_setup(const procell_params *p, Setup &s, bool want_bins, bool want_costs)
 {
     if (!p || (p->n_rows && !p->rows) || (p->n_types && !p->types))
         return PROCELL_E_INVALID;
@@ -125,18 +202,10 @@ int build_setup(const procell_params *p, Setup &s, bool want_bins)
         s.type_mean.push_back(t.mean);
         s.type_sd.push_back(t.sd);
     }
-    if (want_bins) {
-        // parser.cu:126-151: every v / 2^k >= phi, exact halving, distinct.
-        for (double v : s.v) {
-            double f = v;
-            while (f >= phi) {
-                s.bins.push_back(f);
-                f = f / 2;
-            }
-        }
-        std::sort(s.bins.begin(), s.bins.end());
-        s.bins.erase(std::unique(s.bins.begin(), s.bins.end()), s.bins.end());
-    }
+    if (want_costs)
+        cost_caps(s);
+    if (want_bins)
+        build_bins(s);
     return PROCELL_OK;
 }
 
@@ -174,18 +243,11 @@ double row_cost(const Setup &s, uint32_t row)
     return w;
 }
 
-// row_cost of every row.  It depends on the row through its generation cap
-// alone, so it is evaluated once per cap (at 1024 rows, 5 types and 11 caps:
-// 0.3 ms of erfc evaluations -> 4 us, twice per plan).
 static std::vector<double> row_costs(const Setup &s)
 {
-    std::vector<double> by_cap(256, -1.0), w(s.v.size());
-    for (uint32_t r = 0; r < (uint32_t)w.size(); ++r) {
-        double &c = by_cap[s.row_info[r] & 0xFFu];
-        if (c < 0.0)
-            c = row_cost(s, r);
-        w[r] = c;
-    }
+    std::vector<double> w(s.v.size());
+    for (uint32_t r = 0; r < (uint32_t)w.size(); ++r)
+        w[r] = s.cap_cost[s.row_info[r] & 0xFFu];
     return w;
 }
 
@@ -272,51 +334,92 @@ void fill_stats(const unsigned long long *cnt, const int64_t *tally, size_t tall
     st.pool = cnt[kPoolCount];
 }
 
+std::vector<int32_t> index_bins(const Setup &s)
+{
+    const uint64_t n_rows = s.v.size();
+    const uint32_t kdim = (uint32_t)s.kmax + 1;
+    std::vector<int32_t> bin_of(n_rows * kdim, -1);
+    if (s.bins.empty())
+        return bin_of;
+    if (exponent(s.bins.front()) == 0) {
+        // subnormal bins (phi below the smallest normal number): searched
+        for (uint64_t r = 0; r < n_rows; ++r) {
+            double f = s.v[r];
+            for (uint32_t k = 0; k < kdim; ++k, f = f / 2) {
+                auto it = std::lower_bound(s.bins.begin(), s.bins.end(), f);
+                if (it != s.bins.end() && *it == f)
+                    bin_of[r * kdim + k] = (int32_t)(it - s.bins.begin());
+            }
+        }
+        return bin_of;
+    }
+    // the bins of each exponent beside the rows, both by mantissa (a search per
+    // entry took most of the merge)
+    const auto rows = rows_by_mantissa(s);
+    for (size_t b = 0; b < s.bins.size();) {
+        const uint64_t e = exponent(s.bins[b]);
+        size_t end = b;
+        while (end < s.bins.size() && exponent(s.bins[end]) == e)
+            ++end;
+        for (const auto &mr : rows) {
+            const uint64_t er = exponent(s.v[mr.second]);
+            if (er < e || er - e >= kdim)
+                continue;
+            while (b < end && mantissa(s.bins[b]) < mr.first)
+                ++b;
+            if (b < end && mantissa(s.bins[b]) == mr.first)
+                bin_of[(uint64_t)mr.second * kdim + (er - e)] = (int32_t)b;
+        }
+        b = end;
+    }
+    return bin_of;
+}
+
 int merge_tally(const Setup &s, const int64_t *tally, procell_result *r)
+{
+    return merge_tally(s, index_bins(s), tally, r);
+}
+
+int merge_tally(const Setup &s, const std::vector<int32_t> &bin_of, const int64_t *tally, procell_result *r)
 {
     const uint32_t T = s.n_types ? s.n_types : 1;
     const uint32_t kdim = (uint32_t)s.kmax + 1;
-    const uint64_t n_rows = s.v.size();
+    const uint64_t n_ent = s.v.size() * kdim;
     const uint64_t n_bins = s.bins.size();
     if (!r || (r->capacity && !(r->value && r->count)))
         return PROCELL_E_INVALID;
     // (row, generation) -> output value row_value * 2^-generation, exact
     // equality merge into the bin set (proliferation.cu:353-380 searches the
     // same set by exact equality).
-    std::vector<int64_t> bc(n_bins, 0), bt((size_t)n_bins * T, 0);
-    for (uint64_t row = 0; row < n_rows; ++row) {
-        double f = s.v[row];
-        for (uint32_t k = 0; k < kdim; ++k, f = f / 2) {
-            const int64_t *cell = &tally[((size_t)row * kdim + k) * T];
-            int64_t tot = 0;
-            for (uint32_t j = 0; j < T; ++j)
-                tot += cell[j];
-            if (!tot)
-                continue;
-            auto it = std::lower_bound(s.bins.begin(), s.bins.end(), f);
-            if (it == s.bins.end() || *it != f)
-                continue;  // cannot happen: recorded values are >= phi
-            const size_t b = (size_t)(it - s.bins.begin());
-            bc[b] += tot;
-            for (uint32_t j = 0; j < T; ++j)
-                bt[b * T + j] += cell[j];
-        }
+    std::vector<int64_t> bt((size_t)n_bins * (T + 1), 0);  // per bin: all types, then each
+    for (uint64_t e = 0; e < n_ent; ++e) {
+        const int64_t *cell = &tally[(size_t)e * T];
+        int64_t tot = 0;
+        for (uint32_t j = 0; j < T; ++j)
+            tot += cell[j];
+        if (!tot || bin_of[e] < 0)  // (recorded values are >= phi)
+            continue;
+        int64_t *bin = &bt[(size_t)bin_of[e] * (T + 1)];
+        bin[0] += tot;
+        for (uint32_t j = 0; j < T; ++j)
+            bin[1 + j] += cell[j];
     }
     uint64_t n_out = 0;
     for (uint64_t b = 0; b < n_bins; ++b)
-        n_out += bc[b] > 0;
+        n_out += bt[b * (T + 1)] > 0;
     r->n_out = n_out;
     if (n_out > r->capacity)
         return PROCELL_E_CAPACITY;
     uint64_t o = 0;
     for (uint64_t b = 0; b < n_bins; ++b) {
-        if (bc[b] <= 0)
+        const int64_t *bin = &bt[b * (T + 1)];
+        if (bin[0] <= 0)
             continue;
         r->value[o] = s.bins[b];
-        r->count[o] = bc[b];
+        r->count[o] = bin[0];
         if (r->type_count)
             for (uint32_t j = 0; j < s.n_types; ++j)
-                r->type_count[o * s.n_types + j] = bt[b * T + j];
+                r->type_count[o * s.n_types + j] = bin[1 + j];
         ++o;
     }
     return PROCELL_OK;
@@ -333,7 +436,7 @@ int procell_output_capacity(const procell_params *p, uint64_t *capacity)
     if (!capacity)
         return PROCELL_E_INVALID;
     Setup s;
-    const int rc = build_setup(p, s, true);
+    const int rc = build_setup(p, s, true, false);
     if (rc != PROCELL_OK)
         return rc;
     *capacity = s.bins.size();
@@ -345,7 +448,7 @@ int procell_tally_shape(const procell_params *p, uint64_t *nonzero_rows, uint32_
     if (!nonzero_rows || !kdim)
         return PROCELL_E_INVALID;
     Setup s;
-    const int rc = build_setup(p, s, false);
+    const int rc = build_setup(p, s, false, false);
     if (rc != PROCELL_OK)
         return rc;
     *nonzero_rows = s.v.size();

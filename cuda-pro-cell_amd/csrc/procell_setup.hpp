@@ -46,11 +46,14 @@ struct Setup {
     double t_max = 0.0;
     int kmax = 0;
     std::vector<double> bins;       // output bin set, ascending, distinct
+    std::vector<double> cap_cost;   // row_cost by generation cap (-1: no such row)
 };
 
 int generation_cap(double v, double phi);
 double resolve_phi(const procell_params *p);
-int build_setup(const procell_params *p, Setup &s, bool want_bins);
+// want_bins: bins; want_costs: cap_cost (what set_cost, order_rows and
+// split_segments work from).
+int build_setup(const procell_params *p, Setup &s, bool want_bins, bool want_costs = true);
 
 // Expected lane-steps of one initial cell of row `row` and of a whole set.
 double row_cost(const Setup &s, uint32_t row);
@@ -67,8 +70,13 @@ void split_segments(const Setup &s, const std::vector<double> &cum, std::vector<
 // Event statistics from the summed counters (kNumCounters) and the raw
 // tally; the launch fields of `st` are left zero.
 void fill_stats(const unsigned long long *cnt, const int64_t *tally, size_t tally_len, procell_stats &st);
+// Bin of every (row, generation) of the raw tally: index into s.bins of
+// value * 2^-generation, or -1 where that is below phi.
+std::vector<int32_t> index_bins(const Setup &s);
 // Merge a raw tally [rows][kmax+1][max(T,1)] (file type order) into r's
 // output histogram; PROCELL_E_CAPACITY when r->capacity is too small.
 int merge_tally(const Setup &s, const int64_t *tally, procell_result *r);
+// The same with index_bins(s) at hand.
+int merge_tally(const Setup &s, const std::vector<int32_t> &bin_of, const int64_t *tally, procell_result *r);
 
 }  // namespace procell
