@@ -29,22 +29,19 @@
 //   dL/dp_j    += g W (1 - d)
 // for the cotangent g = dL/dh of each recorded entry.
 //
-// Kernel shape: one wavefront per workgroup, a static range of (cell,
-// proliferating type) walks per wavefront balanced by an estimate of their
-// cost, one walk per lane at a time.  A lane runs its walk depth first and
-// evaluates both daughters of a node as it expands it, so every loop step of
-// every busy lane is one expansion (one Philox block, one Box-Muller pair,
-// two sigmoids); expandable right daughters wait in a per-lane stack in
-// device memory, one 64-byte line per frame laid out [wavefront][lane][level]
-// (lanes of a wavefront sit at different levels, so a field-major layout
-// would write a partial line per field and lane).  Recorded weights
-// go to an LDS window over the rows of the wavefront's range (the cotangent
-// window in the backward pass) and reach the tally with FP64 atomics at the
-// end.
+// Kernel shape (walk_kernel): a workgroup of four wavefronts takes a segment
+// of a set's initial cells, every proliferating type of each; its wavefronts
+// claim root steps, which draw 64 roots at once into a buffer, and one walk
+// per lane runs depth first.  A lane evaluates both daughters of a node as it
+// expands it, so every step of every busy lane is one expansion (one Philox
+// block, one Box-Muller pair, two sigmoids); expandable right daughters wait in
+// a per-lane stack in device memory, the newest in registers.  Recorded
+// weights go to an LDS window over the segment's rows (the cotangent's window
+// in the backward pass) and reach the tally with FP64 atomics at the end.
 //
 // A plan covers one parameter set (procell_relaxed_*) or many (the batched
 // calibration, procell_calib_*): sets' rows, cells and tally blocks are
-// concatenated and every wavefront's range lies in one set.  A cell stride k
+// concatenated and every segment lies in one set.  A cell stride k
 // (a power of two) restricts a pass to the initial cells of one residue
 // class mod k.  A calibration step -- fill, forward pass, loss and cotangent,
 // adjoint pass, Adam -- is captured once into a hipGraph and replayed.
@@ -73,39 +70,41 @@ constexpr uint32_t kWalkBudget = 1u << 22;
 // (for untruncated normal timers it would diverge beyond sd / mean = 0.85,
 // where mean^2 / (2 sd^2) = ln 2), so the bound keeps the walks cheap.
 constexpr double kLogMaxSdRatio = -0.22314355131420976;
-// A stacked node: s, W, d (both passes), b, dlogW/dmean, dlogW/dsd (adjoint),
-// padded to one 64-byte line so that a push or a pop of a lane moves one line.
-constexpr uint32_t kFrameDoubles = 8;
-// The adjoint pass (without a cell stride) keeps its two most recently pushed
-// frames (the six tangent fields) in LDS, field-major so that a wavefront's
-// accesses are bank-conflict free; only older frames reach the device stack.
-// Its cotangent window is smaller, so that window and cache fit the LDS of
-// four wavefronts per SIMD.  256 sets x 2e5 cells: adjoint 13.4 -> 12.6 ms,
-// calibration step 23.3 -> 22.5 ms (one slot measured slower).  The Jacobian
-// pass without a stride keeps one frame beside a 768-double window: HBM
-// written per expansion 26.5 -> 10.6 B, read 25.7 -> 8.7 B, for 1% more time
-// (14.09 -> 14.24 ms; two slots beside 384 doubles measured 2% slower, the
-// cache in the stride-4 Jacobian pass 7% slower).
-// Idle lanes a wavefront tolerates before it claims walks for them: a claim
-// costs the wavefront about 50 instructions, so claiming for every idle lane
-// at every step costs more than the idle lanes.  256 sets x 2e5 cells
-// (with the merged redraw loop): calibration step 23.96 ms (0), 23.38 (4),
-// 23.33 (8), 24.06 (16).
-constexpr uint32_t kRefillIdle = 8;
-constexpr uint32_t kTanFields = 6;
-constexpr uint32_t kTanSlots = 2;  // adjoint
-constexpr uint32_t kJacSlots = 1;  // Jacobian pass
-constexpr uint32_t kWindowDoubles = 1024;  // LDS window of a wavefront (8 KB)
-constexpr uint32_t kWindowAdj = 384;       // window of the adjoint pass beside its frame cache (3 KB)
-constexpr uint32_t kWindowJac = 768;       // window of the Jacobian pass beside its frame cache (6 KB)
-constexpr uint32_t kRowCap = 64;           // rows of a wavefront's range staged in LDS
-// Wavefronts of a plan over several sets, in resident wavefronts: short
-// ranges cover few rows, so the tallies stay in the LDS window (the
-// Jacobian pass keeps three), and the dispatcher evens out the cost
-// estimate's errors.  256 sets x 2e5 cells, 8x against 2x: forward pass
-// 12.9 -> 9.8 ms, adjoint 15.9 -> 13.2 ms, Jacobian pass 17.5 -> 13.5 ms,
-// calibration step 29.8 -> 23.3 ms; 16x measured level with 8x.
-constexpr uint32_t kMultiSetWaveFactor = 8;
+// A workgroup: one wavefront per SIMD, a quarter of a CU's LDS.  128 registers
+// and four wavefronts per SIMD; five (the forward pass: six) gained nothing,
+// the walks in flight then being more and the end of a launch longer.
+constexpr uint32_t kWalkThreads = 256;
+constexpr uint32_t kWalkWaves = kWalkThreads / 64;
+constexpr size_t kWalkLds = 40960;
+// Idle lanes a wavefront tolerates before it draws roots (some 220
+// instructions) or shares walks.  1e6 cells of 256 rows and 256 sets x 2e5
+// cells: 231 us and 9.93 ms (8), 232 and 10.0 (12), 232 and 10.0 (16), 235
+// and 10.3 (24).
+constexpr uint32_t kWalkIdle = 12;
+constexpr uint32_t kNoWindow = 0xFFFFFFFFu;
+constexpr uint32_t kMaxCopies = 8;   // of a workgroup's window
+constexpr uint32_t kGradSums = 384;  // gradient sums of a workgroup, all copies
+
+// What a pass of the walk computes.
+enum WalkMode : int {
+    kForward = 0,   // h
+    kAdjoint = 1,   // gradient of <g, h>
+    kJacobian = 2,  // h and its derivatives in each type's mean and sd
+};
+
+// Expected expansions of a walk from which the last root steps of a segment
+// are claimed in parts: a root step of short walks costs more than the
+// wavefronts' uneven ends.
+constexpr double kDeepWalk = 16.0;
+// Least walks of a workgroup.
+constexpr uint32_t kMinWalks = 256;
+// Workgroups of a plan in resident workgroups.  One set: all resident at
+// once, with equal shares of the estimated cost, so that none starts late
+// (1e6 cells: 232 us; two 250).  Many sets: short segments cover few rows, so
+// that the tallies stay in the LDS window.  256 sets x 2e5 cells and 64 sets:
+// 11.1 and 2.31 ms (4), 10.0 and 2.32 (8), 9.66 and 2.55 (16); quarter of the
+// cells 18.5 (8), 20.6 (16).
+constexpr uint32_t kMultiSetFactor = 8;
 
 // One parameter set of a relaxed plan (a single-set plan has one).  Rows,
 // initial cells, tally entries and type blocks of the sets are concatenated.
@@ -123,26 +122,28 @@ struct RelaxSet {
     uint32_t n_prolif;     // proliferating types (mean >= 0 when the plan was made)
     uint32_t quiet_base;
     uint32_t n_quiet;
-    uint32_t pad[3];
+    uint32_t deep;         // nonzero: walks of kDeepWalk expansions or more are expected
+    uint32_t pad[2];
 };
 
 struct RelaxArgs {
     double beta;
     uint32_t n_sets;
     uint32_t n_rows;           // all sets
-    uint32_t kdim_max;         // stack levels per lane
-    uint32_t pad;
+    uint32_t kdim_max;         // most generations + 1 of any set
+    uint32_t even_ends;        // nonzero: every segment is resident at once
+    uint32_t win_doubles[3];   // LDS window of a workgroup, per WalkMode
     const RelaxSet *sets;
-    const uint32_t *wave_set;  // [n_waves] set of each wavefront
-    const uint64_t *wave_unit; // [n_waves][2] first and end walk of the range (set-local)
-    const uint32_t *wave_row;  // [n_waves][2] first and last (global) row of the range
+    const uint32_t *seg_set;   // [segments] set of each segment
+    const uint32_t *seg_cell;  // [segments][2] first and end initial cell (set-local)
+    const uint32_t *seg_row;   // [segments][2] first and last (global) row
+    const uint32_t *seg_win;   // [3 modes][segments] first (global) row of the window
     const uint32_t *row_start; // [n_rows + 1] first initial cell of each row (all sets)
     const uint32_t *row_info;  // [n_rows] generation cap | (value >= phi) << 8
-    const uint32_t *row_set;   // [n_rows] set of each row
     const uint32_t *prolif;    // file index of each proliferating type, per set
     const uint32_t *quiet;     // file index of each quiescent type, per set
     const double *theta;       // per set [3][n_types]: mean, sd, proportion, file order
-    double *stack;             // [n_waves][64 lanes][kdim_max] frames of kFrameDoubles
+    double *stack;             // per segment and wavefront [64 lanes][kdim_max + 1] frames
     double *h;                 // per set [rows][kdim][n_types] relaxed tally (forward)
     const double *g;           // cotangent, layout of h (backward)
     double *grad;              // per set [3][n_types] gradient (backward)
@@ -161,545 +162,920 @@ struct RelaxArgs {
     uint64_t h_total;
 };
 
-// What a pass of the walk computes.
-enum WalkMode : int {
-    kForward = 0,   // h
-    kAdjoint = 1,   // gradient of <g, h>
-    kJacobian = 2,  // h and its derivatives in each type's mean and sd
+// The FP64 constants of the walk, held in scalar registers: left to itself the
+// compiler puts each 64-bit literal into a register again at every use, one
+// or two scalar and often a vector instruction (0.45 to 0.56 scalar
+// instructions per vector instruction, and half of the vector registers).
+// An FP64 operation reads one scalar operand at no cost.  The log, sin/cos
+// and exp polynomials share the factorials' reciprocals.
+struct WalkConst {
+    double r3, r5, r6, r7;              // 1/3, 1/5, 1/6, 1/7
+    double f4, f5, f6, f7;              // 1/4!, 1/5!, 1/6!, 1/7!
+    double f8, f9, f10, f11, f12;
+    double ln2_hi, ln2_lo, two_pi_hi, two_pi_lo;
+    double log2e;
+    double p53;                         // 2^-53
 };
 
-// 1 / x for x >= 1: the hardware reciprocal estimate refined by two Newton
-// steps (each squares the relative error), within an ulp or two of the
-// quotient.
+__device__ __forceinline__ double in_sgpr(double x)
+{
+    asm("" : "+s"(x));
+    return x;
+}
+
+__device__ __forceinline__ WalkConst walk_const()
+{
+    constexpr dev::Coeffs C = dev::coeffs();
+    static_assert(C.lp[0] == -0.5 && C.lp[2] == -0.25 && C.lp[4] == C.s1 && C.c1 == -0.5, "shared coefficients");
+    return WalkConst{in_sgpr(C.lp[1]), in_sgpr(C.lp[3]), in_sgpr(-C.lp[4]), in_sgpr(C.lp[5]),
+                     in_sgpr(C.c2), in_sgpr(C.s2), in_sgpr(-C.c3), in_sgpr(-C.s3),
+                     in_sgpr(2.48015873015873e-05), in_sgpr(2.7557319223985893e-06), in_sgpr(2.755731922398589e-07),
+                     in_sgpr(2.505210838544172e-08), in_sgpr(2.08767569878681e-09),
+                     in_sgpr(C.ln2_hi), in_sgpr(C.ln2_lo), in_sgpr(C.two_pi_hi), in_sgpr(C.two_pi_lo),
+                     in_sgpr(1.4426950408889634), in_sgpr(0x1p-53)};
+}
+
+// The stream's coefficients from the shared ones.
+__device__ __forceinline__ dev::Coeffs stream_coeffs(const WalkConst &c)
+{
+    return dev::Coeffs{{-0.5, c.r3, -0.25, c.r5, -c.r6, c.r7}, c.ln2_hi, c.ln2_lo, c.two_pi_hi, c.two_pi_lo,
+                       -c.r6, c.f5, -c.f7, -0.5, c.f4, -c.f6};
+}
+
+// The stream's Box-Muller pair (dev::normal_pair) with the walk's constants:
+// the same log and sin/cos; the square root by Goldschmidt's method from the
+// hardware's estimate (Markstein, 1990) where the stream's, which a host must
+// be able to repeat, starts from an integer estimate with three Newton steps.
+__device__ __forceinline__ void walk_pair(const dev::Words &w, double &z0, double &z1, const WalkConst &c,
+                                          const dev::Coeffs &K, const dev::Tables &tb)
+{
+    const double u = fma((double)w.w0, 0x1p-32, fma((double)(w.w1 >> 11), c.p53, c.p53));
+    const uint32_t jl = dev::log_index(u);
+    const double invc = tb.log[jl][0], logc = tb.log[jl][1];
+    // the nearest 1/256 turn t and what is left of the turns: both exact
+    const uint32_t t = w.w2 + 0x800000u;
+    const uint32_t js = t >> 24;
+    const double sa = tb.sincos[js][0], ca = tb.sincos[js][1];
+    const double d = fma((double)(int32_t)(w.w2 - (t & 0xFF000000u)), 0x1p-32, (double)(w.w3 >> 11) * c.p53);
+    const double a = fma(d, K.two_pi_hi, d * K.two_pi_lo);
+    const double a2 = a * a;
+    double ps = fma(a2, K.s3, K.s2);
+    ps = fma(a2, ps, K.s1);
+    const double st = fma(a * a2, ps, a);
+    const double cm = a2 * fma(a2, fma(a2, K.c3, K.c2), K.c1);
+    const double sn = sa + fma(sa, cm, ca * st), cs = ca + fma(ca, cm, -(sa * st));
+    // (u = 1: log 0, for which the least normal number keeps rho finite and 0 in effect)
+    const double x = fmax(-2.0 * dev::log_with_entry(u, jl, invc, logc, K), 0x1p-1022);
+    const double y = __builtin_amdgcn_rsq(x);
+    const double h = 0.5 * y;
+    double g = x * y;
+    g = fma(g, fma(-h, g, 0.5), g);
+    const double rho = fma(fma(-g, g, x), h, g);
+    z0 = rho * cs;
+    z1 = rho * sn;
+}
+
 // exp(x) for -40 <= x <= 700 (below -40, 1 + exp(x) rounds to 1): x = k ln 2
 // + r with |r| <= ln 2 / 2 (Cody-Waite reduction, ln 2 in two parts), exp(r)
 // by its Taylor polynomial of degree 12 (truncation below 2e-16 relative),
-// times 2^k.  Horner steps p = fma(p, r, c) keep each coefficient in its
-// register (no copy before a two-address fma).
-// p r + c as one three-address fma (the compiler otherwise ties the result
-// to a copy of the loop-invariant coefficient)
-__device__ __forceinline__ double horner(double p, double r, double c)
+// times 2^k.
+__device__ __forceinline__ double exp_sig(double x, const WalkConst &c)
 {
-    double out;
-    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(out) : "v"(p), "v"(r), "v"(c));
-    return out;
-}
-
-__device__ __forceinline__ double exp_sig(double x)
-{
-    const double k = __builtin_rint(x * 1.4426950408889634);
-    double r = fma(k, -6.93147180369123816490e-01, x);
-    r = fma(k, -1.90821492927058770002e-10, r);
-    double p = 2.08767569878681e-09;
-    p = horner(p, r, 2.505210838544172e-08);
-    p = horner(p, r, 2.755731922398589e-07);
-    p = horner(p, r, 2.7557319223985893e-06);
-    p = horner(p, r, 2.48015873015873e-05);
-    p = horner(p, r, 0.0001984126984126984);
-    p = horner(p, r, 0.001388888888888889);
-    p = horner(p, r, 0.008333333333333333);
-    p = horner(p, r, 0.041666666666666664);
-    p = horner(p, r, 0.16666666666666666);
+    const double k = __builtin_rint(x * c.log2e);
+    double r = fma(-k, c.ln2_hi, x);
+    r = fma(-k, c.ln2_lo, r);
+    double p = fma(c.f12, r, c.f11);
+    p = fma(p, r, c.f10);
+    p = fma(p, r, c.f9);
+    p = fma(p, r, c.f8);
+    p = fma(p, r, c.f7);
+    p = fma(p, r, c.f6);
+    p = fma(p, r, c.f5);
+    p = fma(p, r, c.f4);
+    p = fma(p, r, c.r6);
     p = fma(p, r, 0.5);
     p = fma(p, r, 1.0);
     p = fma(p, r, 1.0);
     return __builtin_ldexp(p, (int)k);
 }
 
+// 1 / x for x >= 1: the hardware estimate r (relative error e < 2^-24) and
+// one cubic step r + r (e + e^2), which leaves e^3 and the last rounding.
 __device__ __forceinline__ double recip_ge1(double x)
 {
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(fma(-x, r, 1.0), r, r);
-    return fma(fma(-x, r, 1.0), r, r);
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, r, 1.0);
+    return fma(r, fma(e, e, e), r);
 }
 
 // sigmoid(y / beta) with ib = 1 / beta.  The exponent is capped at 700 so
 // that 1 + e stays finite (an infinite one would turn the Newton steps into
 // inf x 0); there the sigmoid is below 1e-304 either way.
-__device__ __forceinline__ double sigmoid_scaled(double y, double ib)
+__device__ __forceinline__ double sigmoid_scaled(double y, double ib, const WalkConst &c)
 {
-    return recip_ge1(1.0 + exp_sig(fmin(fmax(-(y * ib), -40.0), 700.0)));
+    return recip_ge1(1.0 + exp_sig(fmin(fmax(-(y * ib), -40.0), 700.0), c));
 }
 
-template <int Mode, bool Strided>
-__device__ __forceinline__ void relaxed_walks(const RelaxArgs &a)
+// A root walk buffered in LDS between a root step and the hand-out to an idle
+// lane: completion time and sigmoid of the root and (tangent passes) 1 + U of
+// its phase and ds/dsd.
+template <bool Tan>
+struct WalkEntry;
+template <>
+struct alignas(16) WalkEntry<false> {
+    double s, d;
+    uint32_t cell;  // set-local id
+    uint32_t tb;    // LDS address of the window entry (row, generation 0, type), or kNoWindow
+    uint32_t rowt;  // row relative to the set's first row | type << 24
+    uint32_t kcap;
+};
+template <>
+struct alignas(16) WalkEntry<true> {
+    double s, d;
+    double u1, b;
+    uint32_t cell, tb, rowt, kcap;
+};
+
+// Stacked right daughter: completion time and W d; tangent passes also ds/dsd
+// and its daughters' dlogW/dmean, dlogW/dsd (padded to 16-byte words).
+template <bool Tan>
+struct WalkFrame;
+template <>
+struct alignas(16) WalkFrame<false> {
+    double s, w;
+};
+template <>
+struct alignas(16) WalkFrame<true> {
+    double s, w, b, gm, gs, pad;
+};
+constexpr uint32_t kFrameBytes = sizeof(WalkFrame<true>);
+
+typedef __attribute__((address_space(3))) double LdsDouble;
+typedef __attribute__((address_space(3))) uint32_t LdsWord;
+__device__ __forceinline__ void lds_add(uint32_t at, double v)
 {
-    constexpr bool Grad = Mode == kAdjoint;
-    constexpr bool Jac = Mode == kJacobian;
-    constexpr bool Tan = Grad || Jac;  // path tangents carried (six-field frames)
-    // LDS: [kWindowDoubles] window | [3][T] gradient sums | [3][T] theta of the set |
-    //      u32 [kRowCap + 1] row starts | [kRowCap] row info | [T] proliferating types
-    extern __shared__ double lds[];
-    const uint32_t lane = threadIdx.x;
-    const uint32_t w = blockIdx.x;
-    const uint32_t set_id = a.wave_set[w];
-    const RelaxSet S = a.sets[set_id];
-    const uint32_t T = S.n_types;
-    const uint32_t KT = S.kdim * T;
-    uint64_t next = a.wave_unit[2 * w];
-    uint64_t u_end = a.wave_unit[2 * w + 1];
-    if (next >= u_end)
-        return;
-    const uint32_t r_lo = a.wave_row[2 * w], r_hi = a.wave_row[2 * w + 1];
-    const uint32_t win_n = (r_hi - r_lo + 1) * KT;
-    // window: h (forward), g (adjoint) or h | dh/dmean | dh/dsd (Jacobian)
-    const uint32_t win_t = Jac ? 3 * win_n : win_n;
-    constexpr bool kLdsCache = (Grad || Jac) && !Strided;  // frames cached in LDS
-    constexpr uint32_t kWin = kLdsCache ? (Jac ? kWindowJac : kWindowAdj) : kWindowDoubles;
-    constexpr uint32_t kSlots = Jac ? kJacSlots : kTanSlots;
-    const bool in_lds = win_t <= kWin;
-    const uint64_t hw0 = S.h_base + (uint64_t)(r_lo - S.row_base) * KT;  // tally index of the window
-    double *gsum = lds + kWin;
-    double *theta = gsum + 3 * T;
-    uint32_t *rs = (uint32_t *)(theta + 3 * T);
-    uint32_t *ri = rs + kRowCap + 1;
-    uint32_t *prolif = ri + kRowCap;
-    const uint32_t nr = r_hi - r_lo + 1;
-    const bool rows_lds = nr <= kRowCap;
-    if (in_lds)
-        for (uint32_t i = lane; i < win_t; i += 64)
-            lds[i] = Grad ? a.g[hw0 + i] : 0.0;
-    for (uint32_t i = lane; i < 3 * T; i += 64) {
-        gsum[i] = 0.0;
+    __hip_atomic_fetch_add((LdsDouble *)(uintptr_t)at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ uint32_t uni(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+__device__ __forceinline__ uint32_t lane_rank(uint64_t mask)
+{
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+__device__ __forceinline__ uint32_t low_bit(uint32_t m) { return (uint32_t)__builtin_ctz(m); }
+__device__ __forceinline__ uint32_t low_bit(uint64_t m) { return (uint32_t)__builtin_ctzll(m); }
+__device__ __forceinline__ uint32_t top_bit(uint32_t m) { return 31u - (uint32_t)__builtin_clz(m); }
+__device__ __forceinline__ uint32_t top_bit(uint64_t m) { return 63u - (uint32_t)__builtin_clzll(m); }
+// Index of the r-th set bit of m (r < popcount(m)).
+__device__ __forceinline__ uint32_t nth_set_bit(uint64_t m, uint32_t r)
+{
+    for (; r; --r)
+        m &= m - 1;
+    return (uint32_t)__builtin_ctzll(m);
+}
+
+// LDS of a workgroup before its window: log and sin/cos tables | theta [3][T]
+// | (adjoint) gradient sums, up to 16 copies of [3][T] | proliferating types
+// u32 [T] | cursor of the root steps u32 [4] | entries, per wavefront [64]
+// (once the roots are done: the walks' expansions by origin lane, u32 [64],
+// and each lane's origin, u32 [64]) | redraws' timers, per lane.  16 bytes
+// more for the gap behind the window's last copy.
+__host__ __device__ constexpr size_t walk_lds_fixed(uint32_t n_types, int mode)
+{
+    const size_t theta = 3 * (size_t)n_types, sums = mode == kAdjoint ? (theta > kGradSums ? theta : kGradSums) : 0;
+    return 384 * 16 + (theta + sums) * 8 + ((size_t)n_types * 4 + 15) / 16 * 16 + 16 +
+           kWalkThreads * (16 + (mode == kForward ? sizeof(WalkEntry<false>) : sizeof(WalkEntry<true>))) + 16;
+}
+
+__device__ __forceinline__ uint64_t again_value(uint64_t x)
+{
+    asm volatile("" : "+s"(x));
+    return x;
+}
+typedef __attribute__((address_space(4))) RelaxArgs ConstArgs;
+typedef __attribute__((address_space(4))) RelaxSet ConstSet;
+template <typename P>
+__device__ __forceinline__ P *again(P *p)
+{
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
+// ======================================================================
+// walk_kernel: one workgroup walks the trees of one segment of a set's initial
+// cells, every proliferating type of each.  As in sim_filter_kernel, its
+// wavefronts claim root steps (64 walks: 64 / n_prolif cells, the lane's type
+// fixed) from an LDS cursor, draw those roots on all lanes into an LDS buffer,
+// hand them to idle lanes, and every busy lane expands one node per step:
+// both daughters' timers, sigmoids and records; it goes on with the left
+// daughter, else the right, else the lowest pending level of its mask.  At the
+// end of the segment idle lanes take the shallowest pending daughter of busy
+// lanes.
+//
+// What bounds it is the vector unit's issue rate (4 cycles per SIMD for nearly
+// every FP64 and integer instruction): the forward pass takes 285 of them per
+// step, root steps and hand-outs included, with 64 of 64 lanes in work, and a
+// CU 320 cycles per step; the Jacobian pass, 5 LDS and up to 6 memory accesses
+// more, is at 0.75 of that rate.  One static range of walks per wavefront,
+// roots drawn in the walks' own steps and no sharing at the end kept 40 to 45
+// lanes busy at 0.71-0.73.  1e6 cells: 330 -> 223 us, adjoint 424 -> 260;
+// Jacobian of 64 sets x 2e5 cells 3.63 -> 2.32 ms, calibration step of 256
+// sets 14.0 -> 9.75 ms, with a quarter of the cells 7.4 -> 4.4 ms.
+//  * constants, arguments: see WalkConst and args_again; 285 against 330
+//    instructions per step with the compiler's own choice.
+//  * the most recently pushed daughter stays in registers (the frame F): it is
+//    the next one popped.  A push writes an F that is not in memory yet to its
+//    level's frame (lane-major in device memory); a pop lets the next step
+//    begin with the read of the next F.  A second frame in LDS halved the
+//    memory traffic and took as long (the LDS then has more to do).
+//  * a node's frame holds what its own expansion needs, W d and its daughters'
+//    tangents, rather than W, d and its own tangents: the sigmoid is not kept.
+//  * p_j multiplies the sums, not the records (h is linear in p_j).
+//  * a timer <= 0 waits for the next steps, which draw from its redraw stream
+//    on that lane beside the other lanes' expansions.
+//  * the window is kept in up to 8 copies where it is small: the adds of 64
+//    lanes meet in some 30 entries (Jacobian pass of 64 sets 2.58 -> 2.31 ms).
+//  * the quiescent types' records are written here too and everything is
+//    cleared in one launch: four launches per pass became two (5000 cells: 20
+//    -> 14 us).
+//  * where all segments run at once, the hardware prefers the older of a
+//    SIMD's wavefronts, so that the youngest ends alone, at a third of the
+//    rate; a wavefront of a segment with more left to claim takes a higher
+//    priority (242 -> 232 us).
+// LDS: see walk_lds_fixed; the window follows.
+// ======================================================================
+template <int Mode, typename N>
+__global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
+{
+    constexpr bool Grad = Mode == kAdjoint, Jac = Mode == kJacobian, Tan = Mode != kForward;
+    constexpr uint32_t kParts = Jac ? 3 : 1;  // values of a window entry
+    using Entry = WalkEntry<Tan>;
+    using Frame = WalkFrame<Tan>;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = uni(tid >> 6);
+    const uint32_t seg = blockIdx.x;
+    const uint32_t set_id = args.seg_set[seg];
+    // The arguments and the set's values are read again (scalar loads) where
+    // they are rarely used: held through the loop they would take the scalar
+    // registers of the walk's constants.
+    const ConstArgs *ap = (const ConstArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    const ConstSet *sp = (const ConstSet *)(uintptr_t)(args.sets + set_id);
+    auto args_again = [&]() -> const ConstArgs & { return *again(ap); };
+    auto set_again = [&]() -> const ConstSet & { return *again(sp); };
+    const ConstArgs &a = *ap;
+    const ConstSet &S = *sp;
+    const uint32_t T = S.n_types, T8 = T * 8, TW = T8 * kParts, KT = S.kdim * T;
+    const uint32_t r_lo = a.seg_row[2 * seg], r_hi = a.seg_row[2 * seg + 1];
+    const uint32_t w_lo = a.seg_win[Mode * gridDim.x + seg];  // first row of the window
+    // selected cells of the segment: first, first + stride, ... (set-local)
+    const uint32_t sshift = (uint32_t)__popc(a.stride_mask);
+    const uint32_t phase = ((a.step ? (uint32_t)a.step[0] : 0u) + a.phase) & a.stride_mask;
+    const uint32_t c_begin = a.seg_cell[2 * seg], c_end = a.seg_cell[2 * seg + 1];
+    const uint32_t first = uni(c_begin + ((0u - (c_begin + phase)) & a.stride_mask));
+    const uint32_t n_sel = uni(first >= c_begin && c_end > first ? ((c_end - 1u - first) >> sshift) + 1u : 0u);
+
+    double(*m_log)[2] = (double(*)[2])lds_raw;
+    double(*m_sc)[2] = (double(*)[2])(lds_raw + 128 * 16);
+    double *theta = (double *)(lds_raw + 384 * 16);
+    double *gsum = theta + 3 * T;
+    uint32_t *prolif = (uint32_t *)(gsum + (Grad ? max(kGradSums, 3 * T) : 0u));
+    uint32_t *cursor = (uint32_t *)((unsigned char *)prolif + ((size_t)T * 4 + 15) / 16 * 16);
+    Entry *ent = (Entry *)(cursor + 4) + wave * 64;
+    double *held = (double *)((Entry *)(cursor + 4) + kWalkThreads) + tid * 2;  // a waiting lane's timers
+    uint32_t *origin_exp = (uint32_t *)ent, *origin = origin_exp + 64;  // (steals)
+    double *win = (double *)((Entry *)(cursor + 4) + kWalkThreads) + kWalkThreads * 2;
+    const uint32_t win_base = (uint32_t)(uintptr_t)(LdsDouble *)win;
+    const uint32_t n_win = min(r_hi - w_lo + 1, a.win_doubles[Mode] / (KT * kParts));  // rows with a window
+    const uint32_t win_n = n_win * KT;
+    // copies of the window, a lane adding to one of them: 64 lanes meet in a few
+    // entries, and adds to one address take turns
+    const uint32_t win_stride = kParts * win_n + 1u;
+    uint32_t copies = 1;
+    if constexpr (!Grad)
+        while (copies < kMaxCopies && 2 * copies * win_stride <= a.win_doubles[Mode])
+            copies *= 2;
+    const uint32_t lane_copy = (lane & (copies - 1u)) * win_stride * 8u;
+    const bool all_in = w_lo == r_lo && n_win == r_hi - r_lo + 1;
+    const uint64_t h0 = S.h_base + (uint64_t)(w_lo - S.row_base) * KT;  // tally index of the window
+    for (uint32_t i = tid; i < 128; i += kWalkThreads) {
+        m_log[i][0] = dev::procell_log_table[i][0];
+        m_log[i][1] = dev::procell_log_table[i][1];
+    }
+    for (uint32_t i = tid; i < 256; i += kWalkThreads) {
+        m_sc[i][0] = dev::procell_sincos_table[i][0];
+        m_sc[i][1] = dev::procell_sincos_table[i][1];
+    }
+    for (uint32_t i = tid; i < 3 * T; i += kWalkThreads) {
         theta[i] = a.theta[S.theta_base + i];
     }
-    for (uint32_t i = lane; i < S.n_prolif; i += 64)
+    // copies of the gradient sums, as of the window
+    uint32_t sums = 1;
+    if constexpr (Grad) {
+        while (sums < 16 && 2 * sums * 3 * T <= kGradSums)
+            sums *= 2;
+        for (uint32_t i = tid; i < sums * 3 * T; i += kWalkThreads)
+            gsum[i] = 0.0;
+    }
+    const uint32_t lane_sums = (uint32_t)(uintptr_t)(LdsDouble *)gsum + (lane & (sums - 1u)) * 3 * T8;
+    for (uint32_t i = tid; i < S.n_prolif; i += kWalkThreads)
         prolif[i] = a.prolif[S.prolif_base + i];
-    if (rows_lds) {
-        for (uint32_t i = lane; i <= nr; i += 64)
-            rs[i] = a.row_start[r_lo + i];
-        for (uint32_t i = lane; i < nr; i += 64)
-            ri[i] = a.row_info[r_lo + i];
-    }
+    for (uint32_t i = tid; i < (Grad ? win_n : copies * win_stride); i += kWalkThreads)
+        win[i] = Grad ? a.g[h0 + i] : 0.0;
+    if (tid == 0)
+        *cursor = 0u;
     __syncthreads();
-    // row r's start and info are row_start[r - roff], row_info[r - roff]
-    const uint32_t roff = rows_lds ? r_lo : 0u;
-    const uint32_t *row_start = rows_lds ? rs : a.row_start;
-    const uint32_t *row_info = rows_lds ? ri : a.row_info;
-    const bool small_units = u_end <= 0xFFFFFFFFull;
 
-    const dev::Coeffs K = dev::coeffs();
-    const dev::Tables tb = dev::global_tables();
-    const double t_max = S.t_max, ib = 1.0 / a.beta;
-    const uint32_t n_prolif = S.n_prolif;
-    double *stk = a.stack + ((uint64_t)w * 64 + lane) * a.kdim_max * kFrameDoubles;
-    // LDS frame cache of the adjoint pass: field f of slot q of this lane
-    double *fc = (double *)(((uintptr_t)(prolif + T) + 7) & ~(uintptr_t)7) + lane;
-    auto fcp = [&](uint32_t q, uint32_t f) -> double & { return fc[(q * kTanFields + f) * 64]; };
-
-    bool active = false;
-    uint64_t cell = 0, node = 0, pending = 0;
-    uint32_t row = r_lo, j = 0, kcap = 0, k = 0;
-    bool ge_phi = false;
-    double pj = 0.0, mean = 0.0, sd = 0.0, u1 = 0.0;  // u1 = 1 + U of the walk's cell
-    double s = 0.0, b = 0.0, W = 0.0, d = 0.0, gm = 0.0, gs = 0.0;
-    double acc_m = 0.0, acc_s = 0.0, acc_p = 0.0;
-    uint32_t row_cursor = r_lo;  // row of the first walk not yet taken (wave-uniform)
-    uint32_t n_exp = 0, n_cut = 0, walk_exp = 0;
-    // The most recently pushed frame stays in registers until another push
-    // spills it: it is always the deepest pending level, i.e. the next one
-    // popped, so most push/pop pairs never touch memory (a store would also
-    // hold up the wavefront's next wait on its loads).
-    // (forward pass only: the adjoint's six-field frame would cost it a
-    // wavefront per SIMD in registers)
-    constexpr bool kCache = !Tan;
-    bool c_ok = false;
-    uint32_t c_lvl = 0;
-    double c_s = 0.0, c_W = 0.0, c_d = 0.0;
-    // adjoint and Jacobian passes: frames cached in LDS slots (c_n of them, c_top the
-    // deepest); the levels of slots 0 and 1 in t_lvl0, t_lvl1
-    static_assert(kSlots == 1 || kSlots == 2, "one or two cached frames");
-    uint32_t c_n = 0, c_top = 0, t_lvl0 = 0, t_lvl1 = 0;
-    const uint32_t smask = Strided ? a.stride_mask : 0u;
-    const uint32_t sphase = Strided ? ((a.step ? (uint32_t)a.step[0] : 0u) + a.phase) & smask : 0u;
-    // With a cell stride the range is enumerated over the selected cells only:
-    // walk index v stands for local cell soff + stride * (v / n_prolif), type
-    // v mod n_prolif (soff: the first cell c with (c + phase) a multiple of
-    // the stride), so every claim takes a walk.
-    const uint32_t sshift = Strided ? (uint32_t)__popc(smask) : 0u;
-    const uint64_t soff = Strided ? (uint64_t)((0u - sphase) & smask) : 0ull;
-    if (Strided) {
-        auto compress = [&](uint64_t u) -> uint64_t {
-            const uint64_t c = u / n_prolif, t = u - c * n_prolif;
-            const uint64_t below = c > soff ? (c - soff + smask) >> sshift : 0ull;  // selected cells < c
-            return below * n_prolif + ((((uint32_t)c + sphase) & smask) == 0u ? t : 0ull);
-        };
-        next = compress(next);
-        u_end = compress(u_end);
+    // Quiescent types: each initial cell of a row with value >= phi records p_j
+    // at generation 0 (cell.cu:104-108 gives them timer -1, always out of
+    // time).  A row's are this segment's if its first cell is.  One wavefront
+    // takes them while the others draw roots.
+    if (S.n_quiet && wave == kWalkWaves - 1) {
+        const uint32_t row0 = r_lo + (a.row_start[r_lo] < (uint32_t)S.cell_base + c_begin ? 1u : 0u);
+        for (uint32_t row = row0 + lane; row <= r_hi; row += 64) {
+            if (((a.row_info[row] >> 8) & 1u) == 0)
+                continue;
+            // selected cells of the row: local ids c in [lo, hi) with c + phase
+            // a multiple of the stride
+            const uint64_t lo = a.row_start[row] - S.cell_base + phase, hi = a.row_start[row + 1] - S.cell_base + phase;
+            const double cnt = (double)(((hi + a.stride_mask) >> sshift) - ((lo + a.stride_mask) >> sshift));
+            const uint64_t e = S.h_base + (uint64_t)(row - S.row_base) * KT;
+            for (uint32_t q = 0; q < S.n_quiet; ++q) {
+                const uint32_t j = a.quiet[S.quiet_base + q];
+                if constexpr (Grad)
+                    lds_add(lane_sums + 2 * T8 + j * 8, cnt * a.g[e + j]);
+                else
+                    a.h[e + j] = cnt * theta[2 * T + j];
+            }
+        }
     }
+
+    const WalkConst C = walk_const();
+    const dev::Coeffs K = stream_coeffs(C);
+    const dev::Tables tb{m_log, m_sc};
+    const uint64_t seed = again_value(S.seed);
+    const double t_max = in_sgpr(S.t_max), ib = 1.0 / a.beta;
+    // root steps: cells of `n_prolif` types each, lanes in (cell, type) order,
+    // or 64 types of one cell of several chunks
+    const uint32_t n_prolif = max(1u, S.n_prolif);
+    const uint32_t chunks = uni((n_prolif + 63) / 64);
+    const uint32_t per_step = uni(chunks > 1 ? 1u : 64u / n_prolif);  // cells of a full step
+    const uint32_t lane_cell = chunks > 1 ? 0u : lane / n_prolif, lane_type = chunks > 1 ? lane : lane % n_prolif;
+    const uint32_t n_units = uni(S.n_prolif ? n_sel * chunks : 0u);
+    // the last walks are claimed as they are needed, so that the wavefronts end together
+    const uint32_t tail = uni(S.deep ? n_units - min(n_units, per_step * kWalkWaves) : n_units);
+
+    uint32_t rpos = 0, rn = 0, roots_done = 0;
+    uint32_t rb = r_lo, bnd = 0, rinfo = 0;  // row boundaries, as in sim_kernel
+    auto load_rows = [&]() {
+        const uint32_t r1 = rb + 1 + lane;
+        bnd = r1 <= args_again().n_rows ? args_again().row_start[r1] : 0xFFFFFFFFu;
+        rinfo = rb + lane < args_again().n_rows ? args_again().row_info[rb + lane] : 0u;
+    };
+    load_rows();
+    const uint32_t frame0 = sizeof(Frame);
+    // the lane's frames: level l at stk + l * frame0 (level 0: a redraw's
+    // timers of a root's daughters never lie there; it is read, not used)
+    const size_t lane_frames = (size_t)(args_again().kdim_max + 1);
+    unsigned char *const stk0 = (unsigned char *)args_again().stack + ((size_t)seg * kWalkThreads + wave * 64) * lane_frames * kFrameBytes;
+    unsigned char *const stk = stk0 + (size_t)lane * lane_frames * frame0;
+
+    // lane state: the node to expand
+    N node = 0, pend = 0;  // pend: pending levels relative to k and the level-0 bit; 0: idle
+    uint32_t k = 0, kcap = 0, cell = 0, tbl = 0, rowt = 0;
+    uint32_t redo = 0;   // redraw pending: timers still to draw (bits 0, 1) | attempt << 16
+    uint32_t since = 0;  // step at which the walk started, and one more per step spent waiting for a redraw
+    double mean = 0.0, sd = 0.0, s = 0.0, W = 0.0, u1 = 0.0, b = 0.0, gm = 0.0, gs = 0.0;
+    double F_s = 0.0, F_w = 0.0, F_b = 0.0, F_gm = 0.0, F_gs = 0.0;
+    double acc_m = 0.0, acc_s = 0.0, acc_p = 0.0;
+    uint64_t dirty = 0;     // lanes whose F is not in memory
+    uint64_t popped = 0;    // lanes that took their F in the last step: the next one is read
+    uint64_t redoing = 0;   // lanes with a redraw pending
+    uint64_t w_exp = 0;     // expansions
+    uint32_t n_cut = 0, steps = 0;
+    uint32_t check = kWalkBudget - 1u;  // first step at which a walk may be near its budget
+    bool shared = false, counted = false;  // steals have begun; walks are counted in origin_exp
+
+    // a frame to its level, F into `below` and back
+    auto store_frame = [&](uint32_t level, double fs, double fw, double fb, double fgm, double fgs) {
+        Frame *f = (Frame *)(stk + (size_t)level * frame0);
+        f->s = fs;
+        f->w = fw;
+        if constexpr (Tan) {
+            f->b = fb;
+            f->gm = fgm;
+            f->gs = fgs;
+        }
+    };
+    // Reads of frames have arrived (vmcnt 0), on every path and before the
+    // step's stores: where the compiler has to wait by itself, stores may
+    // follow the reads, and it waits for those as well.
+    auto frames_read = []() { __builtin_amdgcn_s_waitcnt(0x0F70); };
+    // the adjoint's sums of a walk, or of the part of it that ran on this lane
+    auto end_walk = [&]() {
+        if constexpr (Grad) {
+            const uint32_t at = lane_sums + (rowt >> 24) * 8;
+            lds_add(at, acc_m);
+            lds_add(at + T8, acc_s);
+            lds_add(at + 2 * T8, acc_p);
+            acc_m = acc_s = acc_p = 0.0;
+        }
+    };
 
     for (;;) {
-        // ---- refill idle lanes from the wavefront's range once more than
-        //      kRefillIdle are idle (or all are) ----
-        {
-            const uint64_t idle = __ballot(!active);
-            const bool refill = idle && next < u_end && (__popcll(idle) > kRefillIdle || ~idle == 0);
-            if (refill && !active) {
-                const uint64_t u = next + (uint64_t)__popcll(idle & ((1ull << lane) - 1ull));
-                const uint64_t wi = small_units ? (uint64_t)((uint32_t)u / n_prolif) : u / n_prolif;
-                if (u < u_end) {
-                    cell = Strided ? soff + (wi << sshift) : wi;
-                    j = prolif[(uint32_t)(u - wi * n_prolif)];
-                    const uint64_t gcell = S.cell_base + cell;
-                    row = row_cursor;
-                    while (row_start[row + 1 - roff] <= gcell)
-                        ++row;
-                    const uint32_t info = row_info[row - roff];
-                    kcap = info & 255u;
-                    ge_phi = ((info >> 8) & 1u) != 0;
-                    mean = theta[j];
-                    sd = theta[T + j];
-                    pj = theta[2 * T + j];
-                    node = 0;  // the next step draws the root from block (cell, 0, 0)
-                    pending = 0;
-                    c_ok = false;
-                    c_n = 0;
-                    walk_exp = 0;
-                    active = true;
+        const uint64_t idle = __ballot(pend == 0);
+        const uint32_t n_idle = uni((uint32_t)__popcll(idle));
+        if (n_idle > kWalkIdle) {
+            // ---- root step: the buffer is empty ----
+            if (rpos >= rn && !roots_done) {
+                uint32_t unit = 0, want = per_step;
+                if (lane == 0) {
+                    if (__hip_atomic_load((LdsWord *)cursor, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >= tail)
+                        want = min(per_step, max((n_idle + n_prolif - 1) / n_prolif, (per_step + 3) / 4));
+                    unit = atomicAdd(cursor, want);
                 }
-            }
-            if (refill) {
-                next = next + (uint64_t)__popcll(idle);
-                if (next > u_end)
-                    next = u_end;
-                if (next < u_end) {
-                    const uint64_t wi = small_units ? (uint64_t)((uint32_t)next / n_prolif) : next / n_prolif;
-                    const uint64_t c = S.cell_base + (Strided ? soff + (wi << sshift) : wi);
-                    while (row_start[row_cursor + 1 - roff] <= c)
-                        ++row_cursor;
+                unit = uni(unit);
+                want = uni(want);
+                if (unit >= n_units)
+                    roots_done = 1;
+                if (args_again().even_ends) {
+                    const uint32_t left = n_units - min(unit, n_units);
+                    if (left > n_units / 2)
+                        __builtin_amdgcn_s_setprio(3);
+                    else if (left > n_units / 4)
+                        __builtin_amdgcn_s_setprio(2);
+                    else if (left > n_units / 8)
+                        __builtin_amdgcn_s_setprio(1);
+                    else
+                        __builtin_amdgcn_s_setprio(0);
                 }
-            }
-        }
-        if (__ballot(active) == 0)
-            break;
-        if (!active)
-            continue;
-
-        // ---- one expansion: the root (node 0 stands for "not drawn yet") or
-        //      both daughters of the current node ----
-        const bool pre = node == 0;
-        ++n_exp;
-        ++walk_exp;
-        dev::Words wd = dev::draw_block(S.seed, cell, node, 0u);
-        if (pre) {
-            u1 = 1.0 + dev::uniform_oc(wd.w1, 0u);
-            wd = dev::Words{wd.w2, 0u, wd.w3, 0u};
-        }
-        double z0, z1;
-        dev::normal_pair(wd, z0, z1, K, tb);
-        // the plain method's timers (cell.cu:106-122): a candidate <= 0 gives
-        // way to the first candidate > 0 of a redraw stream -- the root's to
-        // its second candidate, then node 1's stream; a daughter's to its own
-        // node's stream; after 65535 blocks the timer is the mean (z = 0)
-        {
-            bool redoA = !(fma(z0, sd, mean) > 0.0);
-            const bool redoB = !pre && !(fma(z1, sd, mean) > 0.0);
-            if (__builtin_expect(__ballot(redoA || redoB) != 0, 0)) {
-                // the root's second candidate first
-                if (pre && redoA && fma(z1, sd, mean) > 0.0) {
-                    z0 = z1;
-                    redoA = false;
-                }
-                // one loop for both daughters: each round draws one block per
-                // lane, of A's stream while A is pending, then of B's (a lane
-                // needing both takes them in turn; the values do not depend on
-                // the order); a stream gives up after 65535 blocks (z = 0)
-                uint32_t need = (redoA ? 1u : 0u) | (redoB ? 2u : 0u);
-                uint32_t att = 1;
-                while (__ballot(need != 0) != 0) {
-                    if (need != 0) {
-                        const bool onA = (need & 1u) != 0;
-                        const uint64_t rnode = onA ? (pre ? 1ull : 2 * node) : 2 * node + 1;
-                        const dev::Words wr = dev::draw_block(S.seed, cell, rnode, att);
-                        double y0, y1;
-                        dev::normal_pair(wr, y0, y1, K, tb);
-                        const bool ok0 = fma(y0, sd, mean) > 0.0;
-                        const bool ok1 = fma(y1, sd, mean) > 0.0;
-                        const bool done = ok0 || ok1 || att == 65535u;
-                        const double v = ok0 ? y0 : (ok1 ? y1 : 0.0);
-                        if (done) {
-                            if (onA)
-                                z0 = v;
+                if (!roots_done) {
+                    const uint32_t i0 = chunks > 1 ? unit / chunks : unit;
+                    const uint32_t type = chunks > 1 ? (unit % chunks) * 64 + lane_type : lane_type;
+                    const bool valid = lane_cell < want && i0 + lane_cell < n_sel && type < n_prolif;
+                    const uint32_t c = first + ((valid ? i0 + lane_cell : i0) << sshift);
+                    const uint32_t gcell = (uint32_t)set_again().cell_base + c;  // (cells of all sets < 2^32)
+                    const uint32_t g_first = uni((uint32_t)set_again().cell_base + first + (i0 << sshift));
+                    const uint32_t g_last = uni((uint32_t)set_again().cell_base + first + ((min(i0 + want, n_sel) - 1u) << sshift));
+                    for (uint64_t le = __ballot(bnd <= g_first); le; le = __ballot(bnd <= g_first)) {
+                        rb = uni(rb + (uint32_t)__popcll(le));
+                        load_rows();
+                    }
+                    const uint32_t nb = uni((uint32_t)__popcll(__ballot(bnd <= g_last)));
+                    uint32_t row = rb, info = uni(rinfo);
+                    if (nb == 64) {  // (a cell stride over short rows) beyond the boundaries at hand
+                        uint32_t lo = rb, hi = r_hi;
+                        while (lo < hi) {
+                            const uint32_t mid = lo + (hi - lo + 1) / 2;
+                            if (args_again().row_start[mid] <= gcell)
+                                lo = mid;
                             else
-                                z1 = v;
-                            need &= onA ? ~1u : ~2u;
-                            att = 1;
+                                hi = mid - 1;
+                        }
+                        row = lo;
+                        info = args_again().row_info[row];
+                    } else if (nb) {
+                        for (uint32_t j = 0; j < nb; ++j)
+                            row += gcell >= (uint32_t)__builtin_amdgcn_readlane((int)bnd, (int)j) ? 1u : 0u;
+                        info = (uint32_t)__shfl(rinfo, (int)(row - rb));
+                    }
+                    const uint32_t cap = info & 255u;
+                    const bool ge_phi = ((info >> 8) & 1u) != 0;
+                    const uint32_t j = prolif[valid ? type : 0u];
+                    const double m_j = theta[j], sd_j = theta[T + j];
+                    const dev::Words w = dev::draw_block(set_again().seed, c, 0, 0u);
+                    const double U1 = 1.0 + dev::uniform_oc(w.w1, 0u);
+                    double z0, z1;
+                    walk_pair(dev::Words{w.w2, 0u, w.w3, 0u}, z0, z1, C, K, tb);
+                    // the plain method's timer (cell.cu:106-122): the second
+                    // candidate, then node 1's redraw stream; after 65535
+                    // blocks the timer is the mean (z = 0)
+                    if (__builtin_expect(__ballot(valid && !(fma(z0, sd_j, m_j) > 0.0)) != 0, 0)) {
+                        if (valid && !(fma(z0, sd_j, m_j) > 0.0)) {
+                            z0 = z1;
+                            if (!(fma(z0, sd_j, m_j) > 0.0)) {
+                                z0 = 0.0;
+                                for (uint32_t att = 1; att < 65536u; ++att) {
+                                    double y0, y1;
+                                    walk_pair(dev::draw_block(set_again().seed, c, 1, att), y0, y1, C, K, tb);
+                                    if (fma(y0, sd_j, m_j) > 0.0) { z0 = y0; break; }
+                                    if (fma(y1, sd_j, m_j) > 0.0) { z0 = y1; break; }
+                                }
+                            }
+                        }
+                    }
+                    const double s0 = fma(z0, sd_j, m_j) * U1;
+                    const double d0 = sigmoid_scaled(t_max - s0, ib, C);
+                    const double e0 = 1.0 - d0, b0 = z0 * U1;
+                    const uint32_t wrow = row - w_lo;
+                    const uint32_t at = win_base + lane_copy + (__umul24(min(wrow, n_win), KT) + j) * (8 * kParts);
+                    const bool in_win = wrow < n_win;
+                    const uint64_t e = set_again().h_base + (uint64_t)(row - set_again().row_base) * KT + j;
+                    if (valid && ge_phi) {
+                        const double q = d0 * e0 * ib;
+                        const double vm = q * U1, vs = q * b0;
+                        if (Grad) {
+                            const double gv = in_win ? *(LdsDouble *)(uintptr_t)at : args_again().g[e];
+                            lds_add(lane_sums + j * 8, gv * vm);
+                            lds_add(lane_sums + T8 + j * 8, gv * vs);
+                            lds_add(lane_sums + 2 * T8 + j * 8, gv * e0);
+                        } else if (in_win) {
+                            lds_add(at, e0);
+                            if (Jac) {
+                                lds_add(at + 8, vm);
+                                lds_add(at + 16, vs);
+                            }
                         } else {
-                            ++att;
+                            const double p = theta[2 * T + j];
+                            unsafeAtomicAdd(args_again().h + e, p * e0);
+                            if (Jac) {
+                                unsafeAtomicAdd(args_again().jac + e, p * vm);
+                                unsafeAtomicAdd(args_again().jac + args_again().h_total + e, p * vs);
+                            }
+                        }
+                    }
+                    const uint64_t vmask = __ballot(valid);
+                    w_exp += (uint64_t)__popcll(vmask);
+                    const bool grows = valid && cap > 0 && d0 >= kRelaxEps;
+                    const uint64_t gmask = __ballot(grows);
+                    if (grows) {
+                        Entry &q = ent[lane_rank(gmask)];
+                        q.s = s0;
+                        q.d = d0;
+                        if constexpr (Tan) {
+                            q.u1 = U1;
+                            q.b = b0;
+                        }
+                        q.cell = c;
+                        q.tb = in_win ? at : kNoWindow;
+                        q.rowt = (row - set_again().row_base) | (j << 24);
+                        q.kcap = cap;
+                    }
+                    rpos = 0;
+                    rn = uni((uint32_t)__popcll(gmask));
+                    __builtin_amdgcn_wave_barrier();
+                }
+            }
+            // ---- steals: the walks left share the wavefront ----
+            if (rpos >= rn && roots_done && !counted) {
+                const N real = pend & (((N)1 << k) - (N)1);
+                const uint64_t donors = __ballot(real != 0);
+                const uint32_t nd = uni(min((uint32_t)__popcll(donors), n_idle));
+                if (nd) {
+                    if (!shared) {
+                        shared = true;
+                        check = min(check, steps + (kWalkBudget - 1u - min(steps, kWalkBudget - 1u)) / 64u);
+                        origin_exp[lane] = 0u;
+                        origin[lane] = lane;
+                        __builtin_amdgcn_wave_barrier();
+                    }
+                    // every F into memory, then the thieves read theirs
+                    if (real != 0 && __builtin_amdgcn_inverse_ballot_w64(dirty))
+                        store_frame(k - low_bit(pend), F_s, F_w, F_b, F_gm, F_gs);
+                    dirty = 0;
+                    frames_read();  // (and written: vmcnt counts both)
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                    const uint32_t my_up = real ? top_bit(real) : 0u;
+                    const uint32_t r = lane_rank(idle);
+                    const bool thief = pend == 0 && r < nd;
+                    const uint32_t src = thief ? nth_set_bit(donors, r) : lane;
+                    const uint32_t up = __shfl(my_up, (int)src);
+                    const N d_node = __shfl(node, (int)src);
+                    const uint32_t d_k = __shfl(k, (int)src), d_cell = __shfl(cell, (int)src);
+                    const uint32_t d_kcap = __shfl(kcap, (int)src), d_tb = __shfl(tbl, (int)src);
+                    const uint32_t d_rowt = __shfl(rowt, (int)src);
+                    const double d_mean = __shfl(mean, (int)src), d_sd = __shfl(sd, (int)src);
+                    const double d_u1 = Tan ? __shfl(u1, (int)src) : 0.0;
+                    const uint32_t d_origin = origin[src];
+                    if (real != 0 && lane_rank(donors) < nd)
+                        pend &= ~((N)1 << my_up);
+                    if (thief) {
+                        k = d_k - up;
+                        const Frame *f = (const Frame *)(stk0 + ((size_t)src * lane_frames + k) * frame0);
+                        s = f->s;
+                        W = f->w;
+                        if constexpr (Tan) {
+                            b = f->b;
+                            gm = f->gm;
+                            gs = f->gs;
+                            u1 = d_u1;
+                        }
+                        node = (d_node >> up) | (N)1;
+                        pend = (N)1 << k;
+                        cell = d_cell;
+                        kcap = d_kcap;
+                        tbl = d_tb;
+                        rowt = d_rowt;
+                        mean = d_mean;
+                        sd = d_sd;
+                        origin[lane] = d_origin;
+                        since = steps;
+                    }
+                    frames_read();
+                }
+            }
+        }
+        // ---- idle lanes take buffered walks ----
+        if (rpos < rn) {
+            const uint64_t idle2 = __ballot(pend == 0);
+            const uint32_t rank = lane_rank(idle2) + rpos;
+            if (pend == 0 && rank < rn) {
+                const Entry q = ent[rank];
+                s = q.s;
+                W = q.d;
+                if constexpr (Tan) {
+                    const double f = (1.0 - q.d) * ib;
+                    u1 = q.u1;
+                    b = q.b;
+                    gm = -(f * u1);
+                    gs = -(f * b);
+                }
+                cell = q.cell;
+                tbl = q.tb;
+                rowt = q.rowt;
+                kcap = q.kcap;
+                mean = theta[rowt >> 24];
+                sd = theta[T + (rowt >> 24)];
+                node = (N)1;
+                pend = (N)1;
+                k = 0;
+                since = steps - 1u;  // (the root counts)
+            }
+            rpos = uni(min(rpos + (uint32_t)__popcll(idle2), rn));
+        }
+        const uint64_t busy = __ballot(pend != 0);
+        if (busy == 0 && roots_done && rpos >= rn)
+            break;
+        ++steps;
+        // A walk past its budget is cut short (counted; the call reports it).
+        // A lane's walk has taken steps - since expansions after this step; no
+        // walk can be near the budget before that many steps, or a 64th of
+        // them once its parts run on several lanes.
+        uint64_t over = 0;
+        if (__builtin_expect(steps >= check, 0)) {
+            if (!shared) {
+                over = __ballot(pend != 0 && steps - since > kWalkBudget);
+            } else {
+                // exact: every walk's expansions summed by origin lane
+                if (!counted) {
+                    counted = true;
+                    if (pend != 0)
+                        atomicAdd(&origin_exp[origin[lane]], steps - 1u - since + (redo ? 1u : 0u));
+                }
+                bool past = false;
+                if (pend != 0 && redo == 0) {
+                    const uint32_t n = atomicAdd(&origin_exp[origin[lane]], 1u);
+                    past = n >= kWalkBudget;
+                    n_cut += n == kWalkBudget ? 1u : 0u;
+                }
+                over = __ballot(past);
+            }
+            if (over) {
+                if (__builtin_amdgcn_inverse_ballot_w64(over)) {
+                    n_cut += shared ? 0u : 1u;
+                    end_walk();
+                    pend = 0;
+                    redo = 0;
+                }
+                redoing &= ~over;
+                dirty &= ~over;
+            }
+        }
+
+        // ======== one expansion per busy lane ========
+        bool expanded = false, push = false, pop = false;
+        if (pend != 0) {
+            // the next F, for this step's end (level 0 when no level is
+            // pending: read, not used)
+            if (__builtin_amdgcn_inverse_ballot_w64(popped)) {
+                const Frame *f = (const Frame *)(stk + (size_t)(k - low_bit(pend)) * frame0);
+                F_s = f->s;
+                F_w = f->w;
+                if constexpr (Tan) {
+                    F_b = f->b;
+                    F_gm = f->gm;
+                    F_gs = f->gs;
+                }
+            }
+            N bnode = node;
+            if (__builtin_expect(redoing != 0, 0))
+                bnode = redo == 0 ? node : (node << 1) | (N)((redo & 1u) ? 0u : 1u);
+            // (the round keys by scalar adds: held, they would not all fit)
+            const dev::Words wd = dev::draw_block(again_value(seed), cell, bnode, redo >> 16);
+            double z0, z1;
+            walk_pair(wd, z0, z1, C, K, tb);
+            // the plain method's timers (cell.cu:106-122): a candidate <= 0
+            // gives way to the first candidate > 0 of the daughter's redraw
+            // stream (the left daughter's first); after 65535 blocks the timer
+            // is the mean (z = 0)
+            double tauA = fma(z0, sd, mean), tauB = fma(z1, sd, mean);
+            expanded = true;
+            if (__builtin_expect(redoing != 0 || __ballot(!(tauA > 0.0) || !(tauB > 0.0)) != 0, 0)) {
+                const bool okA = tauA > 0.0, okB = tauB > 0.0;
+                // the timers of a lane that waits lie in LDS
+                if (redo == 0) {
+                    redo = (okA ? 0u : 1u) | (okB ? 0u : 2u);
+                    if (redo) {
+                        held[0] = z0;
+                        held[1] = z1;
+                        redo |= 0x10000u;
+                        expanded = false;
+                    }
+                } else {
+                    const uint32_t left = redo & 1u;
+                    expanded = false;
+                    if (okA || okB || (redo >> 16) >= 65535u) {
+                        const double v = okA ? z0 : okB ? z1 : 0.0;
+                        z0 = left ? v : held[0];
+                        z1 = left ? held[1] : v;
+                        redo = (redo & (left ? 2u : 0u)) | 0x10000u;
+                        if ((redo & 3u) == 0u) {
+                            redo = 0u;
+                            expanded = true;
+                            tauA = fma(z0, sd, mean);
+                            tauB = fma(z1, sd, mean);
+                        } else {
+                            held[0] = z0;
+                        }
+                    } else {
+                        redo += 0x10000u;
+                    }
+                }
+                since += expanded ? 0u : 1u;
+            }
+            const uint32_t k1 = k + 1;
+            const double sA = s + tauA, sB = s + tauB;
+            const uint32_t at = tbl + __umul24(k1, TW);
+            double gv = 0.0;
+            if (Grad && (all_in || tbl != kNoWindow))
+                gv = *(LdsDouble *)(uintptr_t)at;
+            const double dA = sigmoid_scaled(t_max - sA, ib, C), dB = sigmoid_scaled(t_max - sB, ib, C);
+            const double eA = 1.0 - dA, eB = 1.0 - dB, e2 = eA + eB;
+            double a1 = 0.0, bA = 0.0, bB = 0.0, fA = 0.0, fB = 0.0, vm = 0.0, vs = 0.0;
+            const double vh = W * e2;
+            if constexpr (Tan) {
+                // the recorded W (1 - d) in mean_j, sd_j:
+                // W ((1 - d) dlogW/dtheta + d (1 - d) / beta ds/dtheta)
+                a1 = u1 + (double)k1;
+                bA = b + z0;
+                bB = b + z1;
+                fA = eA * ib;
+                fB = eB * ib;
+                const double qA = dA * fA, qB = dB * fB;
+                vm = W * fma(e2, gm, (qA + qB) * a1);
+                vs = W * fma(e2, gs, fma(qA, bA, qB * bB));
+            }
+            frames_read();
+            if (expanded) {
+                if (all_in || tbl != kNoWindow) {
+                    if constexpr (!Grad) {
+                        lds_add(at, vh);
+                        if constexpr (Jac) {
+                            lds_add(at + 8, vm);
+                            lds_add(at + 16, vs);
+                        }
+                    }
+                } else {
+                    const uint64_t e = set_again().h_base + (uint64_t)(rowt & 0xFFFFFFu) * KT + (rowt >> 24) + (uint64_t)k1 * T;
+                    if constexpr (Grad) {
+                        gv = args_again().g[e];
+                    } else {
+                        const double p = theta[2 * T + (rowt >> 24)];
+                        unsafeAtomicAdd(args_again().h + e, p * vh);
+                        if constexpr (Jac) {
+                            unsafeAtomicAdd(args_again().jac + e, p * vm);
+                            unsafeAtomicAdd(args_again().jac + args_again().h_total + e, p * vs);
                         }
                     }
                 }
-            }
-        }
-
-        double sA, bA, WA, gmA, gsA, sB = 0.0, bB = 0.0;
-        uint32_t kA;
-        if (pre) {
-            const double tau0 = fma(z0, sd, mean);
-            sA = tau0 * u1;
-            bA = z0 * u1;
-            WA = 1.0;
-            gmA = 0.0;
-            gsA = 0.0;
-            kA = 0;
-        } else {
-            const double f = (1.0 - d) * ib;
-            const double a_cur = u1 + (double)k;
-            WA = W * d;
-            gmA = gm - f * a_cur;
-            gsA = gs - f * b;
-            sA = s + fma(z0, sd, mean);
-            sB = s + fma(z1, sd, mean);
-            bA = b + z0;
-            bB = b + z1;
-            kA = k + 1;
-        }
-        const double aA = u1 + (double)kA;
-        const double dA = sigmoid_scaled(t_max - sA, ib);
-        const double dB = pre ? 0.0 : sigmoid_scaled(t_max - sB, ib);
-        const double recA = WA * (1.0 - dA);
-        const double recB = WA * (1.0 - dB);
-        const bool recordA = kA > 0 || ge_phi;
-        const uint32_t col = kA * T + j;
-        if (Mode == kForward) {
-            // both daughters land in the same (row, generation, type) entry
-            const double v = (recordA ? pj * recA : 0.0) + (pre ? 0.0 : pj * recB);
-            if (recordA || !pre) {
-                if (in_lds)
-                    atomicAdd(lds + (row - r_lo) * KT + col, v);
-                else
-                    unsafeAtomicAdd(a.h + S.h_base + (uint64_t)(row - S.row_base) * KT + col, v);
-            }
-        } else if (Jac) {
-            // the recorded p_j W (1 - d) and its derivatives in mean_j, sd_j:
-            // p_j W ((1 - d) dlogW/dtheta + d (1 - d) / beta ds/dtheta)
-            double vh = 0.0, vm = 0.0, vs = 0.0;
-            if (recordA) {
-                const double q = dA * (1.0 - dA) * ib;
-                vh = recA;
-                vm = WA * ((1.0 - dA) * gmA + q * aA);
-                vs = WA * ((1.0 - dA) * gsA + q * bA);
-            }
-            if (!pre) {
-                const double q = dB * (1.0 - dB) * ib;
-                vh += recB;
-                vm += WA * ((1.0 - dB) * gmA + q * aA);
-                vs += WA * ((1.0 - dB) * gsA + q * bB);
-            }
-            if (recordA || !pre) {
-                if (in_lds) {
-                    double *e = lds + (row - r_lo) * KT + col;
-                    atomicAdd(e, pj * vh);
-                    atomicAdd(e + win_n, pj * vm);
-                    atomicAdd(e + 2 * win_n, pj * vs);
-                } else {
-                    const uint64_t e = S.h_base + (uint64_t)(row - S.row_base) * KT + col;
-                    unsafeAtomicAdd(a.h + e, pj * vh);
-                    unsafeAtomicAdd(a.jac + e, pj * vm);
-                    unsafeAtomicAdd(a.jac + a.h_total + e, pj * vs);
+                if constexpr (Grad) {
+                    acc_m = fma(gv, vm, acc_m);
+                    acc_s = fma(gv, vs, acc_s);
+                    acc_p = fma(gv, vh, acc_p);
                 }
-            }
-        } else {
-            const double gv = in_lds ? lds[(row - r_lo) * KT + col]
-                                     : a.g[S.h_base + (uint64_t)(row - S.row_base) * KT + col];
-            if (recordA) {
-                const double q = dA * (1.0 - dA) * ib;
-                acc_m += pj * gv * WA * ((1.0 - dA) * gmA + q * aA);
-                acc_s += pj * gv * WA * ((1.0 - dA) * gsA + q * bA);
-                acc_p += gv * recA;
-            }
-            if (!pre) {
-                const double q = dB * (1.0 - dB) * ib;
-                acc_m += pj * gv * WA * ((1.0 - dB) * gmA + q * aA);
-                acc_s += pj * gv * WA * ((1.0 - dB) * gsA + q * bB);
-                acc_p += gv * recB;
-            }
-        }
-        const bool expA = kA < kcap && WA * dA >= kRelaxEps;
-        const bool expB = !pre && kA < kcap && WA * dB >= kRelaxEps;
-
-        // ---- next node: left daughter (right one stacked), the only
-        //      expandable daughter, or the deepest stacked node ----
-        // a walk past its budget is cut short (counted; the call reports it)
-        const bool over = walk_exp >= kWalkBudget;
-        if (kCache && expA && expB) {
-            if (c_ok) {  // spill the cached frame to its level (no tangents in the forward pass)
-                double2 *f = (double2 *)(stk + (uint64_t)c_lvl * kFrameDoubles);
-                f[0] = make_double2(c_s, c_W);
-                f[1].x = c_d;
-            }
-            c_ok = true;
-            c_lvl = kA;
-            c_s = sB;
-            c_W = WA;
-            c_d = dB;
-            pending |= 1ull << kA;
-        } else if (kLdsCache && expA && expB) {
-            if (c_n == kSlots) {  // spill the oldest cached frame to its level
-                const uint32_t bot = kSlots == 1 ? 0u : c_top ^ 1u;
-                double2 *f = (double2 *)(stk + (uint64_t)(bot ? t_lvl1 : t_lvl0) * kFrameDoubles);
-                f[0] = make_double2(fcp(bot, 0), fcp(bot, 1));
-                f[1] = make_double2(fcp(bot, 2), fcp(bot, 3));
-                f[2] = make_double2(fcp(bot, 4), fcp(bot, 5));
-                --c_n;
-            }
-            c_top = kSlots == 1 ? 0u : c_top ^ 1u;
-            fcp(c_top, 0) = sB;
-            fcp(c_top, 1) = WA;
-            fcp(c_top, 2) = dB;
-            fcp(c_top, 3) = bB;
-            fcp(c_top, 4) = gmA;
-            fcp(c_top, 5) = gsA;
-            t_lvl0 = c_top ? t_lvl0 : kA;
-            t_lvl1 = c_top ? kA : t_lvl1;
-            ++c_n;
-            pending |= 1ull << kA;
-        } else if (expA && expB) {
-            double2 *f = (double2 *)(stk + (uint64_t)kA * kFrameDoubles);
-            f[0] = make_double2(sB, WA);
-            f[1] = make_double2(dB, bB);
-            f[2] = make_double2(gmA, gsA);
-            pending |= 1ull << kA;
-        }
-        if (!over && (expA || expB)) {
-            const bool left = expA;
-            node = pre ? 1ull : 2ull * node + (left ? 0ull : 1ull);
-            k = kA;
-            s = left ? sA : sB;
-            b = left ? bA : bB;
-            d = left ? dA : dB;
-            W = WA;
-            gm = gmA;
-            gs = gsA;
-        } else if (!over && pending) {
-            const uint32_t L = 63u - (uint32_t)__clzll(pending);
-            pending &= ~(1ull << L);
-            node = (node >> (k - L)) | 1ull;
-            k = L;
-            if (kCache && c_ok) {  // the cached frame is level L
-                s = c_s;
-                W = c_W;
-                d = c_d;
-                c_ok = false;
-            } else if (kLdsCache && c_n) {  // the deepest cached frame is level L
-                s = fcp(c_top, 0);
-                W = fcp(c_top, 1);
-                d = fcp(c_top, 2);
-                b = fcp(c_top, 3);
-                gm = fcp(c_top, 4);
-                gs = fcp(c_top, 5);
-                c_top = kSlots == 1 ? 0u : c_top ^ 1u;
-                --c_n;
-            } else {
-                const double2 *f = (const double2 *)(stk + (uint64_t)L * kFrameDoubles);
-                const double2 f0 = f[0];
-                s = f0.x;
-                W = f0.y;
-                if (Tan) {
-                    const double2 f1 = f[1], f2 = f[2];
-                    d = f1.x;
-                    b = f1.y;
-                    gm = f2.x;
-                    gs = f2.y;
+                const double WA = W * dA, WB = W * dB;
+                const bool can = k1 < kcap;
+                const bool expA = can && WA >= kRelaxEps, expB = can && WB >= kRelaxEps;
+                push = expA && expB;
+                // next: the left daughter, else the lowest pending level (the
+                // right daughter's if it is expanded, else F's)
+                const uint32_t fl = low_bit(pend);
+                const N right = (N)(expA ? 0u : 1u);
+                const uint32_t sh = ((int)expA | (int)expB) ? 0u : fl + 1u;
+                node = ((node << 1) >> sh) | right;
+                pend = (((pend << 1) | (N)(expB ? 1u : 0u)) >> sh) & ~right;
+                if (expA) {
+                    asm volatile("");  // (a branch: the moves are masked, where selects take two each)
+                    if (expB) {
+                        if (__builtin_amdgcn_inverse_ballot_w64(dirty)) {
+                            store_frame(k - fl, F_s, F_w, F_b, F_gm, F_gs);  // F to its level
+                        }
+                        F_s = sB;
+                        F_w = WB;
+                        if constexpr (Tan) {
+                            F_b = bB;
+                            F_gm = fma(-fB, a1, gm);
+                            F_gs = fma(-fB, bB, gs);
+                        }
+                    }
+                    s = sA;
+                    W = WA;
+                    if constexpr (Tan) {
+                        gm = fma(-fA, a1, gm);
+                        gs = fma(-fA, bA, gs);
+                        b = bA;
+                    }
+                } else if (expB) {
+                    asm volatile("");
+                    s = sB;
+                    W = WB;
+                    if constexpr (Tan) {
+                        gm = fma(-fB, a1, gm);
+                        gs = fma(-fB, bB, gs);
+                        b = bB;
+                    }
                 } else {
-                    d = f[1].x;
+                    asm volatile("");
+                    s = F_s;
+                    W = F_w;
+                    if constexpr (Tan) {
+                        gm = F_gm;
+                        gs = F_gs;
+                        b = F_b;
+                    }
+                    pop = true;
+                    if (pend == 0) {
+                        end_walk();
+                        if (shared && !counted)
+                            atomicAdd(&origin_exp[origin[lane]], steps - since);
+                    }
                 }
+                k = k1 - sh;
             }
-        } else {
-            n_cut += over && (expA || expB || pending) ? 1u : 0u;
-            if (Grad) {
-                atomicAdd(gsum + j, acc_m);
-                atomicAdd(gsum + T + j, acc_s);
-                atomicAdd(gsum + 2 * T + j, acc_p);
-                acc_m = acc_s = acc_p = 0.0;
-            }
-            active = false;
         }
+        const uint64_t done = __ballot(expanded);
+        redoing = busy & ~over & ~done;
+        popped = __ballot(pop);
+        dirty = (dirty & ~popped) | __ballot(push);
+        w_exp += (uint64_t)__popcll(done);
     }
+
     __syncthreads();
-    for (int o = 32; o > 0; o >>= 1) {
-        n_exp += __shfl_xor(n_exp, o);
+    if (lane == 0)
+        atomicAdd(args_again().expansions, (unsigned long long)w_exp);
+    for (int o = 32; o > 0; o >>= 1)
         n_cut += __shfl_xor(n_cut, o);
+    if (lane == 0 && n_cut) {
+        atomicAdd(args_again().expansions + 1, (unsigned long long)n_cut);
+        if (args_again().set_cuts)
+            atomicAdd(args_again().set_cuts + set_id, (unsigned long long)n_cut);
     }
-    if (lane == 0) {
-        atomicAdd(a.expansions, (unsigned long long)n_exp);
-        if (n_cut) {
-            atomicAdd(a.expansions + 1, (unsigned long long)n_cut);
-            if (a.set_cuts)
-                atomicAdd(a.set_cuts + set_id, (unsigned long long)n_cut);
-        }
-    }
-    if (Mode == kForward) {
-        if (in_lds)
-            for (uint32_t i = lane; i < win_n; i += 64) {
-                const double v = lds[i];
-                if (v != 0.0)
-                    unsafeAtomicAdd(a.h + hw0 + i, v);
-            }
-    } else if (Jac) {
-        if (in_lds)
-            for (uint32_t i = lane; i < win_t; i += 64) {
-                const double v = lds[i];
-                const uint32_t part = i / win_n, e = i - part * win_n;
-                double *dst = part == 0 ? a.h : a.jac + (uint64_t)(part - 1) * a.h_total;
-                if (v != 0.0)
-                    unsafeAtomicAdd(dst + hw0 + e, v);
-            }
-    } else {
-        for (uint32_t i = lane; i < 3 * T; i += 64) {
-            const double v = gsum[i];
+    if constexpr (Grad) {
+        for (uint32_t i = tid; i < 3 * T; i += kWalkThreads) {
+            // dL/dmean and dL/dsd carry p_j
+            double v = gsum[i];
+            for (uint32_t k = 1; k < sums; ++k)
+                v += gsum[k * 3 * T + i];
+            v *= (i < 2 * T ? theta[2 * T + i % T] : 1.0);
             if (v != 0.0)
-                unsafeAtomicAdd(a.grad + S.theta_base + i, v);
+                unsafeAtomicAdd(args_again().grad + set_again().theta_base + i, v);
+        }
+    } else {
+        for (uint32_t i = tid; i < kParts * win_n; i += kWalkThreads) {
+            double v = win[i];
+            for (uint32_t k = 1; k < copies; ++k)
+                v += win[k * win_stride + i];
+            if (v != 0.0) {
+                const uint32_t e = i / kParts, part = i - e * kParts;
+                double *dst = part == 0 ? args_again().h : args_again().jac + (uint64_t)(part - 1) * args_again().h_total;
+                unsafeAtomicAdd(dst + h0 + e, v * theta[2 * T + e % T]);
+            }
         }
     }
 }
 
-template <bool Grad>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void relaxed_kernel(RelaxArgs a)
+// Clears up to three ranges in one launch.
+__global__ __launch_bounds__(256) void relaxed_clear_kernel(unsigned long long *p0, uint64_t n0, unsigned long long *p1,
+                                                            uint64_t n1, unsigned long long *p2, uint64_t n2)
 {
-    relaxed_walks<Grad ? kAdjoint : kForward, false>(a);
-}
-
-// h, dh/dmean and dh/dsd in one pass (optionally with a cell stride).
-template <bool Strided>
-__global__ __launch_bounds__(64) void relaxed_jacobian_kernel(RelaxArgs a)
-{
-    relaxed_walks<kJacobian, Strided>(a);
-}
-
-// With a cell stride; held to four wavefronts per SIMD (the extra refill
-// rounds would otherwise cost the adjoint one).
-template <bool Grad>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void relaxed_strided_kernel(RelaxArgs a)
-{
-    relaxed_walks<Grad ? kAdjoint : kForward, true>(a);
-}
-
-// Quiescent types: each initial cell of a row with value >= phi records p_j
-// at generation 0 (cell.cu:104-108 gives them timer -1, always out of time).
-template <bool Grad>
-__global__ void relaxed_quiescent_kernel(RelaxArgs a)
-{
-    const uint32_t row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= a.n_rows)
-        return;
-    const RelaxSet &S = a.sets[a.row_set[row]];
-    if (S.n_quiet == 0 || ((a.row_info[row] >> 8) & 1u) == 0)
-        return;
-    // cells of the row walked by this pass: local ids c in [lo, hi) with
-    // (c + phase) a multiple of the stride
-    const uint32_t stride = a.stride_mask + 1u;
-    const uint32_t phase = ((a.step ? (uint32_t)a.step[0] : 0u) + a.phase) & a.stride_mask;
-    const uint64_t lo = a.row_start[row] - S.cell_base + phase, hi = a.row_start[row + 1] - S.cell_base + phase;
-    const double cnt = (double)((hi + stride - 1) / stride - (lo + stride - 1) / stride);
-    const uint64_t base = S.h_base + (uint64_t)(row - S.row_base) * S.kdim * S.n_types;
-    for (uint32_t q = 0; q < S.n_quiet; ++q) {
-        const uint32_t j = a.quiet[S.quiet_base + q];
-        if (!Grad)
-            a.h[base + j] = cnt * a.theta[S.theta_base + 2 * S.n_types + j];
+    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n0 + n1 + n2; i += (uint64_t)gridDim.x * 256) {
+        if (i < n0)
+            p0[i] = 0ull;
+        else if (i < n0 + n1)
+            p1[i - n0] = 0ull;
         else
-            unsafeAtomicAdd(a.grad + S.theta_base + 2 * S.n_types + j, cnt * a.g[base + j]);
+            p2[i - n0 - n1] = 0ull;
     }
+}
+
+hipError_t clear_ranges(void *p0, uint64_t n0, void *p1, uint64_t n1, void *p2, uint64_t n2, hipStream_t st)
+{
+    const uint64_t blocks = (n0 + n1 + n2 + 255) / 256;
+    if (blocks == 0)
+        return hipSuccess;
+    hipLaunchKernelGGL(relaxed_clear_kernel, dim3((unsigned)std::min<uint64_t>(blocks, 4096)), dim3(256), 0, st,
+                       (unsigned long long *)p0, n0, (unsigned long long *)p1, n1, (unsigned long long *)p2, n2);
+    return hipGetLastError();
 }
 
 thread_local hipError_t g_relaxed_hip = hipSuccess;
@@ -713,28 +1089,23 @@ thread_local hipError_t g_relaxed_hip = hipSuccess;
         }                                    \
     } while (0)
 
-// mode 0: the forward kernels and the strided passes; 1: the adjoint without
-// a stride; 2: the Jacobian pass without a stride (the last two: smaller
-// window, frame cache)
-size_t relaxed_lds_bytes(uint32_t n_types, int mode)
+// Expected expansions of one walk of a type in a row with this generation
+// cap: its root and, per generation, the nodes whose completion time s lies at
+// most 34.5 beta past t_max (beyond it d < 1e-15).  s_k is taken as normal (as
+// in the plain method's row_cost).  Only used to balance the segments.
+double walk_cost(uint32_t kcap, double t_max, double beta, double mean, double sd)
 {
-    const uint32_t win = mode == 1 ? kWindowAdj : mode == 2 ? kWindowJac : kWindowDoubles;
-    const size_t base = (win + 6ull * n_types) * sizeof(double) + (2ull * kRowCap + 1 + n_types) * sizeof(uint32_t);
-    const uint32_t slots = mode == 1 ? kTanSlots : mode == 2 ? kJacSlots : 0u;
-    return slots ? (base + 7) / 8 * 8 + (size_t)slots * kTanFields * 64 * sizeof(double) : base;
-}
-
-// Expected expansions of one walk of a type with this mean in a row with
-// this generation cap: a full binary tree down to the generation the mean
-// timer reaches by t_max, plus the relaxed fringe.  Only used to balance the
-// wavefronts' ranges.
-double walk_cost(uint32_t kcap, double t_max, double mean)
-{
-    double g = mean > 0.0 ? floor(t_max / mean) : (double)kcap;
-    if (!(g >= 0.0))
-        g = 0.0;
-    g = std::min(g, (double)kcap);
-    return ldexp(1.0, (int)g + 1) + 1.0;
+    double e = 1.0;
+    for (uint32_t k = 0; k < kcap; ++k) {
+        const double mu = (1.5 + k) * mean;
+        const double var = (7.0 / 3.0 + k) * sd * sd + mean * mean / 12.0;
+        const double z = (t_max + 34.5 * beta - mu) / sqrt(var > 0.0 ? var : 1e-300);
+        const double prob = 0.5 * erfc(-z * 0.70710678118654752);
+        e += ldexp(prob, (int)k);
+        if (!(prob >= 1e-12))
+            break;
+    }
+    return e;
 }
 
 int relaxed_device(int device, int *n_cu)
@@ -751,6 +1122,19 @@ int relaxed_device(int device, int *n_cu)
     return PROCELL_OK;
 }
 
+using WalkKernel = void (*)(RelaxArgs);
+
+// The kernel of a pass: 32-bit heap indices and level masks for trees of at
+// most 31 generations.
+WalkKernel walk_kernel_of(int mode, uint32_t kdim)
+{
+    static const WalkKernel narrow[3] = {walk_kernel<kForward, uint32_t>, walk_kernel<kAdjoint, uint32_t>,
+                                         walk_kernel<kJacobian, uint32_t>};
+    static const WalkKernel wide[3] = {walk_kernel<kForward, uint64_t>, walk_kernel<kAdjoint, uint64_t>,
+                                       walk_kernel<kJacobian, uint64_t>};
+    return kdim <= 32 ? narrow[mode] : wide[mode];
+}
+
 // Device tables of a relaxed plan over n parameter sets.
 struct RelaxCore {
     int device = 0;
@@ -758,15 +1142,8 @@ struct RelaxCore {
     std::vector<Setup> setups;
     std::vector<RelaxSet> sets;
     std::vector<uint32_t> quiet_flag;  // per type of every set: 1 = quiescent
-    uint32_t n_waves = 0;
-    size_t lds_bytes = 0;  // every walk kernel but the two below
-    size_t lds_adj = 0;    // the adjoint without a stride
-    size_t lds_jac = 0;    // the Jacobian pass without a stride
-    // the wavefront layout of the strided and Jacobian passes (equal-cost ranges)
-    const uint32_t *eq_set = nullptr;
-    const uint64_t *eq_unit = nullptr;
-    const uint32_t *eq_row = nullptr;
-    bool any_prolif = false, any_quiet = false;
+    uint32_t n_segments = 0;
+    size_t lds_bytes[3] = {0, 0, 0};  // of the walk kernel, per WalkMode
     uint64_t h_total = 0;      // tally entries of all sets
     uint32_t types_total = 0;  // types of all sets
     RelaxArgs args{};
@@ -785,55 +1162,52 @@ void core_free(RelaxCore &c)
     c.d_stack = nullptr;
 }
 
-// Splits walks [0, n_units) of one set into n_w ranges of equal estimated
-// cost (unit u = cell u / n_prolif, type prolif[u % n_prolif]).
-void split_set(const Setup &s, const std::vector<double> &unit_cost, uint32_t n_prolif, uint32_t n_w,
-               uint32_t row_base, uint64_t *unit_out, uint32_t *row_out, const double *cumw = nullptr)
+// One workgroup's initial cells.
+struct Segment {
+    uint32_t set;
+    uint32_t c0, c1;  // first and end initial cell (set-local)
+    uint32_t r0, r1;  // first and last row (global)
+};
+
+// Splits the initial cells of one set into `n_seg` segments of equal cost
+// (fewer where a cell costs more than that).
+void split_set(const Setup &s, const std::vector<double> &cell_cost, uint64_t n_seg, uint32_t set, uint32_t row_base,
+               std::vector<Segment> &out)
 {
     const uint32_t n_rows = (uint32_t)s.v.size();
-    const uint64_t n_units = s.n_cells * (uint64_t)n_prolif;
     double total = 0.0;
     for (uint32_t i = 0; i < n_rows; ++i)
-        total += unit_cost[i] * (double)(s.start[i + 1] - s.start[i]) * n_prolif;
-    std::vector<uint64_t> cut(n_w + 1, n_units);
-    cut[0] = 0;
-    uint32_t wv = 1;
-    double acc = 0.0;
-    for (uint32_t i = 0; i < n_rows && wv < n_w; ++i) {
-        const uint64_t u0 = s.start[i] * n_prolif, u1 = s.start[i + 1] * n_prolif;
-        const double per = unit_cost[i];
-        while (wv < n_w) {
-            const double need = (total * (cumw ? cumw[wv - 1] : (double)wv / (double)n_w) - acc) / per;
-            if (need >= (double)(u1 - u0))
-                break;
-            uint64_t c = u0 + (uint64_t)std::max(0.0, ceil(need));
-            c = std::min(c, u1);
-            cut[wv] = std::max(c, cut[wv - 1]);
-            ++wv;
-        }
-        acc += per * (double)(u1 - u0);
-    }
-    for (uint32_t v = 1; v <= n_w; ++v)
-        cut[v] = std::max(cut[v], cut[v - 1]);
+        total += cell_cost[i] * (double)(s.start[i + 1] - s.start[i]);
     auto row_of = [&](uint64_t cell) {
-        return (uint32_t)(std::upper_bound(s.start.begin(), s.start.end() - 1, cell) - s.start.begin() - 1);
+        return row_base + (uint32_t)(std::upper_bound(s.start.begin(), s.start.end() - 1, cell) - s.start.begin() - 1);
     };
-    for (uint32_t v = 0; v < n_w; ++v) {
-        unit_out[2 * v] = cut[v];
-        unit_out[2 * v + 1] = cut[v + 1];
-        row_out[2 * v] = row_out[2 * v + 1] = row_base;
-        if (cut[v] < cut[v + 1]) {
-            row_out[2 * v] = row_base + row_of(cut[v] / n_prolif);
-            row_out[2 * v + 1] = row_base + row_of((cut[v + 1] - 1) / n_prolif);
+    uint32_t row = 0;
+    double acc = 0.0;  // cost of the rows before `row`
+    uint64_t c0 = 0;
+    for (uint64_t v = 1; v <= n_seg; ++v) {
+        uint64_t c1 = s.n_cells;
+        if (v < n_seg) {
+            const double want = total * ((double)v / (double)n_seg);
+            for (; row < n_rows; ++row) {
+                const double rc = cell_cost[row] * (double)(s.start[row + 1] - s.start[row]);
+                if (acc + rc > want)
+                    break;
+                acc += rc;
+            }
+            if (row < n_rows) {
+                c1 = s.start[row] + (uint64_t)std::max(0.0, ceil((want - acc) / cell_cost[row]));
+                c1 = std::max(c0, std::min<uint64_t>(c1, s.start[row + 1]));
+            }
         }
+        if (c1 > c0)
+            out.push_back(Segment{set, (uint32_t)c0, (uint32_t)c1, row_of(c0), row_of(c1 - 1)});
+        c0 = c1;
     }
 }
 
-// Validates the sets, sizes the launch (resident wavefronts of the plan's
-// device, `wave_factor` times more, so that the dispatcher evens out the
-// cost estimate's errors between sets) and uploads the tables.
-int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, bool want_bins,
-               uint32_t wave_factor)
+// Validates the sets, cuts their initial cells into the workgroups' segments
+// and uploads the tables.
+int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, bool want_bins)
 {
     if (!ps || n == 0)
         return PROCELL_E_INVALID;
@@ -858,7 +1232,7 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
     c.device = ps[0].device;
 
     // ---- concatenation ----
-    std::vector<uint32_t> prolif, quiet, row_start, row_info, row_set;
+    std::vector<uint32_t> prolif, quiet, row_start, row_info;
     c.sets.resize(n);
     uint64_t cells = 0;
     uint32_t rows = 0, kdim_max = 1, t_max_types = 1;
@@ -887,12 +1261,9 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
             c.quiet_flag.push_back(1u);
         S.n_prolif = (uint32_t)prolif.size() - S.prolif_base;
         S.n_quiet = (uint32_t)quiet.size() - S.quiet_base;
-        c.any_prolif = c.any_prolif || (S.n_prolif && s.n_cells);
-        c.any_quiet = c.any_quiet || S.n_quiet;
         for (uint32_t r = 0; r < S.n_rows; ++r) {
             row_start.push_back((uint32_t)(cells + s.start[r]));
             row_info.push_back(s.row_info[r]);
-            row_set.push_back(i);
         }
         units[i] = s.n_cells * (uint64_t)S.n_prolif;
         cells += s.n_cells;
@@ -906,120 +1277,108 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
     }
     row_start.push_back((uint32_t)cells);
 
-    // ---- wavefronts ----
-    c.lds_bytes = relaxed_lds_bytes(t_max_types, 0);
-    c.lds_adj = relaxed_lds_bytes(t_max_types, 1);
-    c.lds_jac = relaxed_lds_bytes(t_max_types, 2);
-    int occ = 0, occ_f = 0;
-    int occ_s = 0, occ_sf = 0, occ_j = 0, occ_js = 0;
-    RELAX_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, relaxed_kernel<true>, 64, c.lds_adj));
-    RELAX_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_f, relaxed_kernel<false>, 64, c.lds_bytes));
-    RELAX_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_s, relaxed_strided_kernel<true>, 64, c.lds_bytes));
-    RELAX_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_sf, relaxed_strided_kernel<false>, 64, c.lds_bytes));
-    RELAX_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_j, relaxed_jacobian_kernel<false>, 64, c.lds_jac));
-    RELAX_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_js, relaxed_jacobian_kernel<true>, 64, c.lds_bytes));
-    occ = std::min(std::min(std::min(occ, occ_f), std::min(occ_s, occ_sf)), std::min(occ_j, occ_js));
+    // ---- segments ----
+    // Windows: what is left of a workgroup's share of the LDS beside its
+    // fixed part (kept to the rows that a segment has, below)
+    uint32_t win_cap[3];
+    int occ = 0;
+    for (int m = 0; m < 3; ++m) {
+        const size_t fixed = walk_lds_fixed(t_max_types, m);
+        win_cap[m] = fixed < kWalkLds ? (uint32_t)((kWalkLds - fixed) / 8) : 0u;
+        int o = 0;
+        RELAX_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, walk_kernel_of(m, kdim_max), (int)kWalkThreads,
+                                                               fixed + win_cap[m] * 8));
+        occ = m == 0 ? o : std::min(occ, o);
+    }
     if (occ < 1)
         return PROCELL_E_HIP;
     if (ps[0].tuning.blocks_per_cu)
         occ = std::min(occ, (int)ps[0].tuning.blocks_per_cu);
-    const uint64_t budget = (uint64_t)occ * (uint64_t)n_cu * std::max(1u, wave_factor);
-    std::vector<std::vector<double>> ucost(n);
+    const uint32_t factor = n > 1 ? kMultiSetFactor : 1u;
+    const uint64_t budget = (uint64_t)occ * (uint64_t)n_cu * factor;
+    std::vector<std::vector<double>> cell_cost(n);
     std::vector<double> set_cost(n, 0.0);
     double all_cost = 0.0;
     for (uint32_t i = 0; i < n; ++i) {
         const Setup &s = c.setups[i];
         const RelaxSet &S = c.sets[i];
-        ucost[i].assign(S.n_rows, 1.0);
+        cell_cost[i].assign(S.n_rows, 1.0);
         if (!units[i])
             continue;
+        std::vector<double> by_cap(S.kdim, -1.0);
         for (uint32_t r = 0; r < S.n_rows; ++r) {
-            double cr = 0.0;
-            for (uint32_t q = 0; q < S.n_prolif; ++q)
-                cr += walk_cost(s.row_info[r] & 255u, ps[i].t_max, ps[i].types[prolif[S.prolif_base + q]].mean);
-            ucost[i][r] = cr / S.n_prolif;
-            set_cost[i] += ucost[i][r] * (double)(s.start[r + 1] - s.start[r]) * S.n_prolif;
+            const uint32_t cap = s.row_info[r] & 255u;
+            double &cr = by_cap[cap];
+            if (cr < 0.0) {
+                cr = 0.0;
+                for (uint32_t q = 0; q < S.n_prolif; ++q) {
+                    const procell_type &ty = ps[i].types[prolif[S.prolif_base + q]];
+                    cr += walk_cost(cap, ps[i].t_max, beta, ty.mean, ty.sd);
+                }
+            }
+            cell_cost[i][r] = cr;
+            set_cost[i] += cr * (double)(s.start[r + 1] - s.start[r]);
         }
         all_cost += set_cost[i];
+        c.sets[i].deep = set_cost[i] >= kDeepWalk * (double)units[i] ? 1u : 0u;
     }
-    std::vector<uint32_t> waves_of(n, 0);
-    uint64_t n_waves = 0;
+    std::vector<Segment> segs;
     for (uint32_t i = 0; i < n; ++i) {
-        if (!units[i])
+        const Setup &s = c.setups[i];
+        if (!units[i]) {
+            // no walks: the quiescent types' records alone, 4096 rows a segment
+            for (size_t r = 0; r < s.v.size(); r += 4096) {
+                const size_t r1 = std::min(r + 4096, s.v.size());
+                segs.push_back(Segment{i, (uint32_t)s.start[r], (uint32_t)(r1 < s.v.size() ? s.start[r1] : s.n_cells),
+                                       c.sets[i].row_base + (uint32_t)r, c.sets[i].row_base + (uint32_t)r1 - 1});
+            }
             continue;
-        double share = all_cost > 0.0 ? set_cost[i] / all_cost * (double)budget : 1.0;
-        uint64_t wv = (uint64_t)std::max(1.0, floor(share + 0.5));
-        wv = std::min<uint64_t>(wv, (units[i] + 63) / 64);
-        waves_of[i] = (uint32_t)std::max<uint64_t>(1, wv);
-        n_waves += waves_of[i];
+        }
+        const double share = all_cost > 0.0 ? set_cost[i] / all_cost * (double)budget : 1.0;
+        const uint64_t most = (units[i] + kMinWalks - 1) / kMinWalks;
+        split_set(s, cell_cost[i], std::max<uint64_t>(1, std::min((uint64_t)floor(share + 0.5), most)), i,
+                  c.sets[i].row_base, segs);
     }
-    if (n_waves > 0x7FFFFFFFull)
+    if (segs.size() > 0x7FFFFFFFull)
         return PROCELL_E_TOO_MANY_CELLS;
-    c.n_waves = (uint32_t)n_waves;
-    const uint32_t NW = std::max(1u, c.n_waves);
-    std::vector<uint32_t> wave_set(NW, 0), wave_row(2 * NW, 0);
-    std::vector<uint64_t> wave_unit(2 * NW, 0);
-    // Two layouts of the same number of wavefronts.  Passes with a cell
-    // stride and the Jacobian pass take ranges of equal cost, set by set;
-    // the full forward and adjoint passes take ranges that shrink
-    // geometrically over rounds (the last 1/8 of the first), launched round
-    // by round over all sets, so that the wavefronts dispatched last are
-    // short.  256 sets x 2e5 cells: calibration step 23.26 -> 22.48 ms,
-    // forward 10.50 -> 10.28, adjoint 13.17 -> 13.03 (the strided passes
-    // measured 12 % slower and the Jacobian pass 3 % slower with it: their
-    // per-wavefront set-up weighs more in short ranges).
-    std::vector<uint32_t> eq_set(NW, 0), eq_row(2 * NW, 0);
-    std::vector<uint64_t> eq_unit(2 * NW, 0);
-    {
-        uint32_t wpos = 0;
-        for (uint32_t i = 0; i < n; ++i) {
-            if (!waves_of[i])
-                continue;
-            split_set(c.setups[i], ucost[i], c.sets[i].n_prolif, waves_of[i], c.sets[i].row_base,
-                      &eq_unit[2 * wpos], &eq_row[2 * wpos]);
-            for (uint32_t v = 0; v < waves_of[i]; ++v)
-                eq_set[wpos + v] = i;
-            wpos += waves_of[i];
+    c.n_segments = (uint32_t)segs.size();
+    c.args.even_ends = c.n_segments <= (uint64_t)occ * (uint64_t)n_cu ? 1u : 0u;
+    std::vector<uint32_t> seg_set, seg_cell, seg_row;
+    uint64_t entries = 0;  // most entries of a segment's rows
+    for (const Segment &p : segs) {
+        seg_set.push_back(p.set);
+        seg_cell.insert(seg_cell.end(), {p.c0, p.c1});
+        seg_row.insert(seg_row.end(), {p.r0, p.r1});
+        entries = std::max<uint64_t>(entries, (uint64_t)(p.r1 - p.r0 + 1) * c.sets[p.set].kdim * c.sets[p.set].n_types);
+    }
+    // each segment's window over the rows that take most of its cost
+    std::vector<uint32_t> seg_win;
+    for (int m = 0; m < 3; ++m) {
+        for (const Segment &p : segs) {
+            const Setup &s = c.setups[p.set];
+            const RelaxSet &S = c.sets[p.set];
+            const uint32_t len = std::max(1u, win_cap[m] / (S.kdim * S.n_types * (m == kJacobian ? 3 : 1)));
+            auto cost = [&](uint32_t row) {  // of the segment's cells in a row
+                const uint32_t r = row - S.row_base;
+                return cell_cost[p.set][r] * (double)(std::min<uint64_t>(s.start[r + 1], p.c1) - std::max<uint64_t>(s.start[r], p.c0));
+            };
+            uint32_t at = p.r0;
+            double in = 0.0, best = -1.0;
+            for (uint32_t r = p.r0; r <= p.r1; ++r) {
+                in += cost(r);
+                if (r - p.r0 >= len)
+                    in -= cost(r - len);
+                if (in > best && (r - p.r0 + 1 >= len || r == p.r1)) {
+                    best = in;
+                    at = r - p.r0 + 1 >= len ? r + 1 - len : p.r0;
+                }
+            }
+            seg_win.push_back(at);
         }
     }
-    struct Piece {
-        uint32_t round, set;
-        uint64_t u0, u1;
-        uint32_t r0, r1;
-    };
-    std::vector<Piece> pieces;
-    pieces.reserve(NW);
-    const uint32_t R = std::max(1u, wave_factor);
-    for (uint32_t i = 0; i < n; ++i) {
-        const uint32_t nw = waves_of[i];
-        if (!nw)
-            continue;
-        const uint32_t rounds = std::min(nw, R);
-        const double q = rounds > 1 ? pow(0.125, 1.0 / (double)(rounds - 1)) : 1.0;
-        std::vector<double> wk(nw), cumw(nw);
-        double tot = 0.0;
-        for (uint32_t k = 0; k < nw; ++k) {
-            wk[k] = pow(q, (double)((uint64_t)k * rounds / nw));
-            tot += wk[k];
-        }
-        double acc = 0.0;
-        for (uint32_t k = 0; k < nw; ++k) {
-            acc += wk[k];
-            cumw[k] = k + 1 == nw ? 1.0 : acc / tot;
-        }
-        std::vector<uint64_t> wu(2 * nw);
-        std::vector<uint32_t> wr(2 * nw);
-        split_set(c.setups[i], ucost[i], c.sets[i].n_prolif, nw, c.sets[i].row_base, wu.data(), wr.data(), cumw.data());
-        for (uint32_t k = 0; k < nw; ++k)
-            pieces.push_back(Piece{(uint32_t)((uint64_t)k * rounds / nw), i, wu[2 * k], wu[2 * k + 1], wr[2 * k], wr[2 * k + 1]});
-    }
-    std::stable_sort(pieces.begin(), pieces.end(), [](const Piece &x, const Piece &y) { return x.round < y.round; });
-    for (uint32_t v = 0; v < (uint32_t)pieces.size(); ++v) {
-        wave_set[v] = pieces[v].set;
-        wave_unit[2 * v] = pieces[v].u0;
-        wave_unit[2 * v + 1] = pieces[v].u1;
-        wave_row[2 * v] = pieces[v].r0;
-        wave_row[2 * v + 1] = pieces[v].r1;
+    for (int m = 0; m < 3; ++m) {
+        c.args.win_doubles[m] = (uint32_t)std::min<uint64_t>(win_cap[m], (entries * (m == kJacobian ? 3 : 1) + 1) * (m == kAdjoint ? 1 : 8));
+        c.lds_bytes[m] = walk_lds_fixed(t_max_types, m) + (size_t)c.args.win_doubles[m] * 8;
     }
 
     // ---- upload ----
@@ -1030,10 +1389,10 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
         return o;
     };
     const size_t o_sets = take(c.sets.size() * sizeof(RelaxSet));
-    const size_t o_ws = take(wave_set.size() * 4), o_wu = take(wave_unit.size() * 8);
-    const size_t o_wr = take(wave_row.size() * 4), o_rs = take(row_start.size() * 4);
-    const size_t o_es = take(eq_set.size() * 4), o_eu = take(eq_unit.size() * 8), o_er = take(eq_row.size() * 4);
-    const size_t o_ri = take(row_info.size() * 4 + 4), o_rt = take(row_set.size() * 4 + 4);
+    const size_t o_ss = take(seg_set.size() * 4 + 4), o_sc = take(seg_cell.size() * 4 + 4);
+    const size_t o_sw = take(seg_win.size() * 4 + 4);
+    const size_t o_sr = take(seg_row.size() * 4 + 4), o_rs = take(row_start.size() * 4);
+    const size_t o_ri = take(row_info.size() * 4 + 4);
     const size_t o_pr = take(prolif.size() * 4 + 4), o_qu = take(quiet.size() * 4 + 4);
     const size_t o_ex = take(16 + (size_t)n * 8);  // expansions, walks cut, walks cut per set
     if (hipMalloc(&c.d_block, off) != hipSuccess)
@@ -1043,15 +1402,12 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
         return bytes ? hipMemcpy(base + o, src, bytes, hipMemcpyHostToDevice) : hipSuccess;
     };
     RELAX_TRY(up(o_sets, c.sets.data(), c.sets.size() * sizeof(RelaxSet)));
-    RELAX_TRY(up(o_ws, wave_set.data(), wave_set.size() * 4));
-    RELAX_TRY(up(o_wu, wave_unit.data(), wave_unit.size() * 8));
-    RELAX_TRY(up(o_wr, wave_row.data(), wave_row.size() * 4));
-    RELAX_TRY(up(o_es, eq_set.data(), eq_set.size() * 4));
-    RELAX_TRY(up(o_eu, eq_unit.data(), eq_unit.size() * 8));
-    RELAX_TRY(up(o_er, eq_row.data(), eq_row.size() * 4));
+    RELAX_TRY(up(o_ss, seg_set.data(), seg_set.size() * 4));
+    RELAX_TRY(up(o_sc, seg_cell.data(), seg_cell.size() * 4));
+    RELAX_TRY(up(o_sw, seg_win.data(), seg_win.size() * 4));
+    RELAX_TRY(up(o_sr, seg_row.data(), seg_row.size() * 4));
     RELAX_TRY(up(o_rs, row_start.data(), row_start.size() * 4));
     RELAX_TRY(up(o_ri, row_info.data(), row_info.size() * 4));
-    RELAX_TRY(up(o_rt, row_set.data(), row_set.size() * 4));
     RELAX_TRY(up(o_pr, prolif.data(), prolif.size() * 4));
     RELAX_TRY(up(o_qu, quiet.data(), quiet.size() * 4));
     RelaxArgs &a = c.args;
@@ -1060,22 +1416,19 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
     a.n_rows = rows;
     a.kdim_max = kdim_max;
     a.sets = (const RelaxSet *)(base + o_sets);
-    a.wave_set = (const uint32_t *)(base + o_ws);
-    a.wave_unit = (const uint64_t *)(base + o_wu);
-    a.wave_row = (const uint32_t *)(base + o_wr);
-    c.eq_set = (const uint32_t *)(base + o_es);
-    c.eq_unit = (const uint64_t *)(base + o_eu);
-    c.eq_row = (const uint32_t *)(base + o_er);
+    a.seg_set = (const uint32_t *)(base + o_ss);
+    a.seg_cell = (const uint32_t *)(base + o_sc);
+    a.seg_win = (const uint32_t *)(base + o_sw);
+    a.seg_row = (const uint32_t *)(base + o_sr);
     a.row_start = (const uint32_t *)(base + o_rs);
     a.row_info = (const uint32_t *)(base + o_ri);
-    a.row_set = (const uint32_t *)(base + o_rt);
     a.prolif = (const uint32_t *)(base + o_pr);
     a.quiet = (const uint32_t *)(base + o_qu);
     a.expansions = (unsigned long long *)(base + o_ex);
     a.set_cuts = a.expansions + 2;
     a.h_total = c.h_total;
-    if (c.n_waves) {
-        const size_t stack_bytes = (size_t)c.n_waves * 64 * kdim_max * kFrameDoubles * sizeof(double);
+    if (c.n_segments) {
+        const size_t stack_bytes = (size_t)c.n_segments * kWalkThreads * (kdim_max + 1) * kFrameBytes;
         if (hipMalloc((void **)&c.d_stack, stack_bytes) != hipSuccess)
             return PROCELL_E_OUT_OF_MEMORY;
         a.stack = c.d_stack;
@@ -1083,48 +1436,14 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
     return PROCELL_OK;
 }
 
-// Enqueues one pass of a WalkMode: the walk kernel and the quiescent kernel
-// (the caller has cleared h, the Jacobian or the gradient, and the expansion
-// counter).
-hipError_t core_launch(const RelaxCore &c, const RelaxArgs &a_in, int mode, hipStream_t st)
+// Enqueues one pass of a WalkMode (the caller has cleared h, the Jacobian or
+// the gradient, and the expansion counter).
+hipError_t core_launch(const RelaxCore &c, const RelaxArgs &a, int mode, hipStream_t st)
 {
-    const bool grad = mode == kAdjoint;
-    RelaxArgs a = a_in;
-    if (a.stride_mask || mode == kJacobian) {
-        a.wave_set = c.eq_set;
-        a.wave_unit = c.eq_unit;
-        a.wave_row = c.eq_row;
-    }
-    if (c.any_prolif && c.n_waves) {
-        const dim3 g(c.n_waves), b(64);
-        if (mode == kJacobian) {
-            if (a.stride_mask)
-                hipLaunchKernelGGL(relaxed_jacobian_kernel<true>, g, b, c.lds_bytes, st, a);
-            else
-                hipLaunchKernelGGL(relaxed_jacobian_kernel<false>, g, b, c.lds_jac, st, a);
-        } else if (a.stride_mask) {
-            if (grad)
-                hipLaunchKernelGGL(relaxed_strided_kernel<true>, g, b, c.lds_bytes, st, a);
-            else
-                hipLaunchKernelGGL(relaxed_strided_kernel<false>, g, b, c.lds_bytes, st, a);
-        } else if (grad) {
-            hipLaunchKernelGGL(relaxed_kernel<true>, g, b, c.lds_adj, st, a);
-        } else {
-            hipLaunchKernelGGL(relaxed_kernel<false>, g, b, c.lds_bytes, st, a);
-        }
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess)
-            return e;
-    }
-    if (c.any_quiet && a.n_rows) {
-        const dim3 g((a.n_rows + 255) / 256);
-        if (grad)
-            hipLaunchKernelGGL(relaxed_quiescent_kernel<true>, g, dim3(256), 0, st, a);
-        else
-            hipLaunchKernelGGL(relaxed_quiescent_kernel<false>, g, dim3(256), 0, st, a);
-        return hipGetLastError();
-    }
-    return hipSuccess;
+    if (c.n_segments == 0)
+        return hipSuccess;
+    hipLaunchKernelGGL(walk_kernel_of(mode, a.kdim_max), dim3(c.n_segments), dim3(kWalkThreads), c.lds_bytes[mode], st, a);
+    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -1394,14 +1713,11 @@ int relaxed_call(procell_relaxed *r, int mode, const double *theta, double *h, c
     a.g = g;
     a.grad = gr;
     a.jac = jac;
-    RELAX_TRY(launch_zero(a.expansions, 2ull + a.n_sets, st));
-    if (mode == kAdjoint) {
-        RELAX_TRY(launch_zero((unsigned long long *)gr, 3ull * r->core.types_total, st));
-    } else {
-        RELAX_TRY(launch_zero((unsigned long long *)h, r->core.h_total, st));
-        if (mode == kJacobian)
-            RELAX_TRY(launch_zero((unsigned long long *)jac, 2ull * r->core.h_total, st));
-    }
+    const uint64_t n_h = r->core.h_total;
+    if (mode == kAdjoint)
+        RELAX_TRY(clear_ranges(a.expansions, 2ull + a.n_sets, gr, 3ull * r->core.types_total, nullptr, 0, st));
+    else
+        RELAX_TRY(clear_ranges(a.expansions, 2ull + a.n_sets, h, n_h, jac, mode == kJacobian ? 2 * n_h : 0, st));
     RELAX_TRY(core_launch(r->core, a, mode, st));
     return PROCELL_OK;
 }
@@ -1440,7 +1756,7 @@ int procell_relaxed_create(const procell_params *p, double beta, procell_relaxed
     procell_relaxed *r = new (std::nothrow) procell_relaxed();
     if (!r)
         return PROCELL_E_OUT_OF_MEMORY;
-    const int rc = core_build(r->core, p, 1, beta, false, 1);
+    const int rc = core_build(r->core, p, 1, beta, false);
     if (rc != PROCELL_OK) {
         destroy_relaxed(r);
         return rc;
@@ -1457,7 +1773,7 @@ int procell_relaxed_create_batch(const procell_params *sets, uint32_t n_sets, do
     procell_relaxed *r = new (std::nothrow) procell_relaxed();
     if (!r)
         return PROCELL_E_OUT_OF_MEMORY;
-    const int rc = core_build(r->core, sets, n_sets, beta, false, n_sets > 1 ? kMultiSetWaveFactor : 1u);
+    const int rc = core_build(r->core, sets, n_sets, beta, false);
     if (rc != PROCELL_OK) {
         destroy_relaxed(r);
         return rc;
@@ -1584,7 +1900,7 @@ int procell_calib_create(const procell_params *sets, uint32_t n_sets, double bet
             return fail(PROCELL_E_HIP);       \
         }                                     \
     } while (0)
-    int rc = core_build(c->core, sets, n_sets, beta, true, n_sets > 1 ? kMultiSetWaveFactor : 1u);
+    int rc = core_build(c->core, sets, n_sets, beta, true);
     if (rc != PROCELL_OK)
         return fail(rc);
     RelaxCore &core = c->core;
