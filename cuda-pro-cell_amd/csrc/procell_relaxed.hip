@@ -143,7 +143,7 @@ struct RelaxArgs {
     const uint32_t *prolif;    // file index of each proliferating type, per set
     const uint32_t *quiet;     // file index of each quiescent type, per set
     const double *theta;       // per set [3][n_types]: mean, sd, proportion, file order
-    double *stack;             // per segment and wavefront [64 lanes][kdim_max + 1] frames
+    double *stack;             // per segment and wavefront [kdim_max + 1 levels][64 lanes] frames
     double *h;                 // per set [rows][kdim][n_types] relaxed tally (forward)
     const double *g;           // cotangent, layout of h (backward)
     double *grad;              // per set [3][n_types] gradient (backward)
@@ -377,14 +377,14 @@ __device__ __forceinline__ P *again(P *p)
 // CU 320 cycles per step; the Jacobian pass, 5 LDS and up to 6 memory accesses
 // more, is at 0.75 of that rate.  One static range of walks per wavefront,
 // roots drawn in the walks' own steps and no sharing at the end kept 40 to 45
-// lanes busy at 0.71-0.73.  1e6 cells: 330 -> 223 us, adjoint 424 -> 260;
-// Jacobian of 64 sets x 2e5 cells 3.63 -> 2.32 ms, calibration step of 256
-// sets 14.0 -> 9.75 ms, with a quarter of the cells 7.4 -> 4.4 ms.
+// lanes busy at 0.71-0.73.  1e6 cells: 330 -> 223 us, adjoint 424 -> 249;
+// Jacobian of 64 sets x 2e5 cells 3.63 -> 2.15 ms, calibration step of 256
+// sets 14.0 -> 9.0 ms, with a quarter of the cells 7.4 -> 4.3 ms.
 //  * constants, arguments: see WalkConst and args_again; 285 against 330
 //    instructions per step with the compiler's own choice.
 //  * the most recently pushed daughter stays in registers (the frame F): it is
 //    the next one popped.  A push writes an F that is not in memory yet to its
-//    level's frame (lane-major in device memory); a pop lets the next step
+//    level's frame in device memory; a pop lets the next step
 //    begin with the read of the next F.  A second frame in LDS halved the
 //    memory traffic and took as long (the LDS then has more to do).
 //  * a node's frame holds what its own expansion needs, W d and its daughters'
@@ -531,12 +531,16 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
         rinfo = rb + lane < args_again().n_rows ? args_again().row_info[rb + lane] : 0u;
     };
     load_rows();
-    const uint32_t frame0 = sizeof(Frame);
-    // the lane's frames: level l at stk + l * frame0 (level 0: a redraw's
-    // timers of a root's daughters never lie there; it is read, not used)
-    const size_t lane_frames = (size_t)(args_again().kdim_max + 1);
-    unsigned char *const stk0 = (unsigned char *)args_again().stack + ((size_t)seg * kWalkThreads + wave * 64) * lane_frames * kFrameBytes;
-    unsigned char *const stk = stk0 + (size_t)lane * lane_frames * frame0;
+    // the lane's frames: level l at stk + l * kLevelBytes (level 0 is read, not
+    // used).  By level, then lane: lanes at one level share their lines, and a
+    // line holds no levels that are rarely touched.  By lane, then level (each
+    // lane's levels in its own lines): Jacobian pass of 64 sets 2.26 -> 2.15
+    // ms, calibration step 9.55 -> 9.0, adjoint of 1e6 cells 257 -> 249 us; a
+    // frame's fields apart (16 bytes per lane): 2.44 ms.
+    constexpr uint32_t kLevelBytes = 64 * sizeof(Frame);
+    const size_t levels = (size_t)args_again().kdim_max + 1;
+    unsigned char *const stk0 = (unsigned char *)args_again().stack + ((size_t)seg * kWalkThreads + wave * 64) * levels * kFrameBytes;
+    unsigned char *const stk = stk0 + (size_t)lane * sizeof(Frame);
 
     // lane state: the node to expand
     N node = 0, pend = 0;  // pend: pending levels relative to k and the level-0 bit; 0: idle
@@ -556,7 +560,7 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
 
     // a frame to its level, F into `below` and back
     auto store_frame = [&](uint32_t level, double fs, double fw, double fb, double fgm, double fgs) {
-        Frame *f = (Frame *)(stk + (size_t)level * frame0);
+        Frame *f = (Frame *)(stk + (size_t)level * kLevelBytes);
         f->s = fs;
         f->w = fw;
         if constexpr (Tan) {
@@ -751,7 +755,7 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
                         pend &= ~((N)1 << my_up);
                     if (thief) {
                         k = d_k - up;
-                        const Frame *f = (const Frame *)(stk0 + ((size_t)src * lane_frames + k) * frame0);
+                        const Frame *f = (const Frame *)(stk0 + (size_t)k * kLevelBytes + src * sizeof(Frame));
                         s = f->s;
                         W = f->w;
                         if constexpr (Tan) {
@@ -848,7 +852,7 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
             // the next F, for this step's end (level 0 when no level is
             // pending: read, not used)
             if (__builtin_amdgcn_inverse_ballot_w64(popped)) {
-                const Frame *f = (const Frame *)(stk + (size_t)(k - low_bit(pend)) * frame0);
+                const Frame *f = (const Frame *)(stk + (size_t)(k - low_bit(pend)) * kLevelBytes);
                 F_s = f->s;
                 F_w = f->w;
                 if constexpr (Tan) {
