@@ -171,15 +171,23 @@ struct RelaxArgs {
 struct WalkConst {
     double r3, r5, r6, r7;              // 1/3, 1/5, 1/6, 1/7
     double f4, f5, f6, f7;              // 1/4!, 1/5!, 1/6!, 1/7!
-    double f8, f9, f10, f11, f12;
+    double f8, f9, f10, f12;
     double ln2_hi, ln2_lo, two_pi_hi, two_pi_lo;
     double log2e;
     double p53;                         // 2^-53
+    // of these a polynomial's first step adds: an operation reads one scalar
+    double f11, f4v, f5v, r6v;
 };
 
 __device__ __forceinline__ double in_sgpr(double x)
 {
     asm("" : "+s"(x));
+    return x;
+}
+
+__device__ __forceinline__ double in_vgpr(double x)
+{
+    asm("" : "+v"(x));
     return x;
 }
 
@@ -190,16 +198,42 @@ __device__ __forceinline__ WalkConst walk_const()
     return WalkConst{in_sgpr(C.lp[1]), in_sgpr(C.lp[3]), in_sgpr(-C.lp[4]), in_sgpr(C.lp[5]),
                      in_sgpr(C.c2), in_sgpr(C.s2), in_sgpr(-C.c3), in_sgpr(-C.s3),
                      in_sgpr(2.48015873015873e-05), in_sgpr(2.7557319223985893e-06), in_sgpr(2.755731922398589e-07),
-                     in_sgpr(2.505210838544172e-08), in_sgpr(2.08767569878681e-09),
+                     in_sgpr(2.08767569878681e-09),
                      in_sgpr(C.ln2_hi), in_sgpr(C.ln2_lo), in_sgpr(C.two_pi_hi), in_sgpr(C.two_pi_lo),
-                     in_sgpr(1.4426950408889634), in_sgpr(0x1p-53)};
+                     in_sgpr(1.4426950408889634), in_sgpr(0x1p-53),
+                     in_vgpr(2.505210838544172e-08), in_vgpr(C.c2), in_vgpr(C.s2), in_vgpr(-C.lp[4])};
 }
 
 // The stream's coefficients from the shared ones.
 __device__ __forceinline__ dev::Coeffs stream_coeffs(const WalkConst &c)
 {
-    return dev::Coeffs{{-0.5, c.r3, -0.25, c.r5, -c.r6, c.r7}, c.ln2_hi, c.ln2_lo, c.two_pi_hi, c.two_pi_lo,
-                       -c.r6, c.f5, -c.f7, -0.5, c.f4, -c.f6};
+    return dev::Coeffs{{-0.5, c.r3, -0.25, c.r5, -c.r6v, c.r7}, c.ln2_hi, c.ln2_lo, c.two_pi_hi, c.two_pi_lo,
+                       -c.r6, c.f5v, -c.f7, -0.5, c.f4v, -c.f6};
+}
+
+// dev::log_with_entry, bit for bit: the hardware splits x = m 2^e with m in
+// [0.5, 1), and where m is halved against the table's (j < 64) the entry's
+// 1/c comes doubled (see walk_log_table).
+__device__ __forceinline__ double walk_log(double x, uint32_t j, double invc, double logc, const dev::Coeffs &K)
+{
+    const double r = fma(__builtin_amdgcn_frexp_mant(x), invc, -1.0);
+    const double de = (double)(__builtin_amdgcn_frexp_exp(x) + (int)(j >> 6) - 1);
+    const double r2 = r * r;
+    double p = fma(K.lp[5], r, K.lp[4]);
+    p = fma(p, r, K.lp[3]);
+    p = fma(p, r, K.lp[2]);
+    p = fma(p, r, K.lp[1]);
+    p = fma(p, r, K.lp[0]);
+    const double hi = fma(de, K.ln2_hi, logc);
+    const double t = fma(r2, p, de * K.ln2_lo);
+    return hi + (r + t);
+}
+
+// Entry j of the LDS copy of the log table.
+__device__ __forceinline__ double2 walk_log_table(uint32_t j)
+{
+    const double invc = dev::procell_log_table[j][0];
+    return make_double2(j < 64 ? 2.0 * invc : invc, dev::procell_log_table[j][1]);
 }
 
 // The stream's Box-Muller pair (dev::normal_pair) with the walk's constants:
@@ -225,7 +259,7 @@ __device__ __forceinline__ void walk_pair(const dev::Words &w, double &z0, doubl
     const double cm = a2 * fma(a2, fma(a2, K.c3, K.c2), K.c1);
     const double sn = sa + fma(sa, cm, ca * st), cs = ca + fma(ca, cm, -(sa * st));
     // (u = 1: log 0, for which the least normal number keeps rho finite and 0 in effect)
-    const double x = fmax(-2.0 * dev::log_with_entry(u, jl, invc, logc, K), 0x1p-1022);
+    const double x = fmax(-2.0 * walk_log(u, jl, invc, logc, K), 0x1p-1022);
     const double y = __builtin_amdgcn_rsq(x);
     const double h = 0.5 * y;
     double g = x * y;
@@ -372,16 +406,16 @@ __device__ __forceinline__ P *again(P *p)
 // lanes.
 //
 // What bounds it is the vector unit's issue rate (4 cycles per SIMD for nearly
-// every FP64 and integer instruction): the forward pass takes 285 of them per
-// step, root steps and hand-outs included, with 64 of 64 lanes in work, and a
-// CU 320 cycles per step; the Jacobian pass, 5 LDS and up to 6 memory accesses
-// more, is at 0.75 of that rate.  One static range of walks per wavefront,
+// every FP64 and integer instruction): the forward pass takes some 275 of them
+// per step, root steps and hand-outs included, with 64 of 64 lanes in work, and
+// a CU 320 cycles per step; the Jacobian pass, 5 LDS and up to 6 memory
+// accesses more, issues 0.81 per cycle.  One static range of walks per wavefront,
 // roots drawn in the walks' own steps and no sharing at the end kept 40 to 45
-// lanes busy at 0.71-0.73.  1e6 cells: 330 -> 223 us, adjoint 424 -> 249;
-// Jacobian of 64 sets x 2e5 cells 3.63 -> 2.15 ms, calibration step of 256
-// sets 14.0 -> 9.0 ms, with a quarter of the cells 7.4 -> 4.3 ms.
-//  * constants, arguments: see WalkConst and args_again; 285 against 330
-//    instructions per step with the compiler's own choice.
+// lanes busy at 0.71-0.73.  1e6 cells: 330 -> 219 us, adjoint 424 -> 245;
+// Jacobian of 64 sets x 2e5 cells 3.63 -> 2.13 ms, calibration step of 256
+// sets 14.0 -> 9.0 ms, with a quarter of the cells 7.4 -> 4.2 ms.
+//  * constants, arguments: see WalkConst and args_again; the compiler's own choice
+//    took 45 instructions per step more.
 //  * the most recently pushed daughter stays in registers (the frame F): it is
 //    the next one popped.  A push writes an F that is not in memory yet to its
 //    level's frame in device memory; a pop lets the next step
@@ -389,7 +423,8 @@ __device__ __forceinline__ P *again(P *p)
 //    memory traffic and took as long (the LDS then has more to do).
 //  * a node's frame holds what its own expansion needs, W d and its daughters'
 //    tangents, rather than W, d and its own tangents: the sigmoid is not kept.
-//  * p_j multiplies the sums, not the records (h is linear in p_j).
+//  * p_j and, for the tangents, 1 / beta multiply the sums, not the records:
+//    gm and gs are beta dlogW/dmean and beta dlogW/dsd.
 //  * a timer <= 0 waits for the next steps, which draw from its redraw stream
 //    on that lane beside the other lanes' expansions.
 //  * the window is kept in up to 8 copies where it is small: the adds of 64
@@ -457,8 +492,9 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
     const bool all_in = w_lo == r_lo && n_win == r_hi - r_lo + 1;
     const uint64_t h0 = S.h_base + (uint64_t)(w_lo - S.row_base) * KT;  // tally index of the window
     for (uint32_t i = tid; i < 128; i += kWalkThreads) {
-        m_log[i][0] = dev::procell_log_table[i][0];
-        m_log[i][1] = dev::procell_log_table[i][1];
+        const double2 e = walk_log_table(i);
+        m_log[i][0] = e.x;
+        m_log[i][1] = e.y;
     }
     for (uint32_t i = tid; i < 256; i += kWalkThreads) {
         m_sc[i][0] = dev::procell_sincos_table[i][0];
@@ -674,7 +710,7 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
                     const bool in_win = wrow < n_win;
                     const uint64_t e = set_again().h_base + (uint64_t)(row - set_again().row_base) * KT + j;
                     if (valid && ge_phi) {
-                        const double q = d0 * e0 * ib;
+                        const double q = d0 * e0;
                         const double vm = q * U1, vs = q * b0;
                         if (Grad) {
                             const double gv = in_win ? *(LdsDouble *)(uintptr_t)at : args_again().g[e];
@@ -691,6 +727,7 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
                             const double p = theta[2 * T + j];
                             unsafeAtomicAdd(args_again().h + e, p * e0);
                             if (Jac) {
+                                const double p = theta[2 * T + j] * ib;
                                 unsafeAtomicAdd(args_again().jac + e, p * vm);
                                 unsafeAtomicAdd(args_again().jac + args_again().h_total + e, p * vs);
                             }
@@ -788,11 +825,11 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
                 s = q.s;
                 W = q.d;
                 if constexpr (Tan) {
-                    const double f = (1.0 - q.d) * ib;
+                    const double e = 1.0 - q.d;
                     u1 = q.u1;
                     b = q.b;
-                    gm = -(f * u1);
-                    gs = -(f * b);
+                    gm = -(e * u1);
+                    gs = -(e * b);
                 }
                 cell = q.cell;
                 tbl = q.tb;
@@ -915,17 +952,15 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
                 gv = *(LdsDouble *)(uintptr_t)at;
             const double dA = sigmoid_scaled(t_max - sA, ib, C), dB = sigmoid_scaled(t_max - sB, ib, C);
             const double eA = 1.0 - dA, eB = 1.0 - dB, e2 = eA + eB;
-            double a1 = 0.0, bA = 0.0, bB = 0.0, fA = 0.0, fB = 0.0, vm = 0.0, vs = 0.0;
+            double a1 = 0.0, bA = 0.0, bB = 0.0, vm = 0.0, vs = 0.0;
             const double vh = W * e2;
             if constexpr (Tan) {
-                // the recorded W (1 - d) in mean_j, sd_j:
-                // W ((1 - d) dlogW/dtheta + d (1 - d) / beta ds/dtheta)
+                // beta times the derivative of the recorded W (1 - d) in mean_j,
+                // sd_j: W ((1 - d) beta dlogW/dtheta + d (1 - d) ds/dtheta)
                 a1 = u1 + (double)k1;
                 bA = b + z0;
                 bB = b + z1;
-                fA = eA * ib;
-                fB = eB * ib;
-                const double qA = dA * fA, qB = dB * fB;
+                const double qA = dA * eA, qB = dB * eB;
                 vm = W * fma(e2, gm, (qA + qB) * a1);
                 vs = W * fma(e2, gs, fma(qA, bA, qB * bB));
             }
@@ -947,6 +982,7 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
                         const double p = theta[2 * T + (rowt >> 24)];
                         unsafeAtomicAdd(args_again().h + e, p * vh);
                         if constexpr (Jac) {
+                            const double p = theta[2 * T + (rowt >> 24)] * ib;
                             unsafeAtomicAdd(args_again().jac + e, p * vm);
                             unsafeAtomicAdd(args_again().jac + args_again().h_total + e, p * vs);
                         }
@@ -978,15 +1014,15 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
                         F_w = WB;
                         if constexpr (Tan) {
                             F_b = bB;
-                            F_gm = fma(-fB, a1, gm);
-                            F_gs = fma(-fB, bB, gs);
+                            F_gm = fma(-eB, a1, gm);
+                            F_gs = fma(-eB, bB, gs);
                         }
                     }
                     s = sA;
                     W = WA;
                     if constexpr (Tan) {
-                        gm = fma(-fA, a1, gm);
-                        gs = fma(-fA, bA, gs);
+                        gm = fma(-eA, a1, gm);
+                        gs = fma(-eA, bA, gs);
                         b = bA;
                     }
                 } else if (expB) {
@@ -994,8 +1030,8 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
                     s = sB;
                     W = WB;
                     if constexpr (Tan) {
-                        gm = fma(-fB, a1, gm);
-                        gs = fma(-fB, bB, gs);
+                        gm = fma(-eB, a1, gm);
+                        gs = fma(-eB, bB, gs);
                         b = bB;
                     }
                 } else {
@@ -1017,8 +1053,8 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
                 k = k1 - sh;
             }
         }
-        const uint64_t done = __ballot(expanded);
-        redoing = busy & ~over & ~done;
+        redoing = __ballot(redo != 0);
+        const uint64_t done = busy & ~over & ~redoing;
         popped = __ballot(pop);
         dirty = (dirty & ~popped) | __ballot(push);
         w_exp += (uint64_t)__popcll(done);
@@ -1036,11 +1072,11 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
     }
     if constexpr (Grad) {
         for (uint32_t i = tid; i < 3 * T; i += kWalkThreads) {
-            // dL/dmean and dL/dsd carry p_j
+            // dL/dmean and dL/dsd carry p_j / beta
             double v = gsum[i];
             for (uint32_t k = 1; k < sums; ++k)
                 v += gsum[k * 3 * T + i];
-            v *= (i < 2 * T ? theta[2 * T + i % T] : 1.0);
+            v *= (i < 2 * T ? theta[2 * T + i % T] * ib : 1.0);
             if (v != 0.0)
                 unsafeAtomicAdd(args_again().grad + set_again().theta_base + i, v);
         }
@@ -1052,7 +1088,7 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
             if (v != 0.0) {
                 const uint32_t e = i / kParts, part = i - e * kParts;
                 double *dst = part == 0 ? args_again().h : args_again().jac + (uint64_t)(part - 1) * args_again().h_total;
-                unsafeAtomicAdd(dst + h0 + e, v * theta[2 * T + e % T]);
+                unsafeAtomicAdd(dst + h0 + e, v * theta[2 * T + e % T] * (part ? ib : 1.0));
             }
         }
     }
