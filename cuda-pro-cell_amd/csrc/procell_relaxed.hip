@@ -768,14 +768,9 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
                         origin[lane] = lane;
                         __builtin_amdgcn_wave_barrier();
                     }
-                    // every F into memory, then the thieves read theirs
-                    if (real != 0 && __builtin_amdgcn_inverse_ballot_w64(dirty))
-                        store_frame(k - low_bit(pend), F_s, F_w, F_b, F_gm, F_gs);
-                    dirty = 0;
-                    frames_read();  // (and written: vmcnt counts both)
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                    // the daughter taken is F where it is the only one and in
+                    // the registers; any other lies in memory
+                    const uint64_t in_reg = __ballot((real & (real - 1)) == 0) & ~popped;
                     const uint32_t my_up = real ? top_bit(real) : 0u;
                     const uint32_t r = lane_rank(idle);
                     const bool thief = pend == 0 && r < nd;
@@ -788,18 +783,35 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
                     const double d_mean = __shfl(mean, (int)src), d_sd = __shfl(sd, (int)src);
                     const double d_u1 = Tan ? __shfl(u1, (int)src) : 0.0;
                     const uint32_t d_origin = origin[src];
-                    if (real != 0 && lane_rank(donors) < nd)
+                    const bool given = real != 0 && lane_rank(donors) < nd;
+                    if (given)
                         pend &= ~((N)1 << my_up);
+                    dirty &= ~(__ballot(given) & in_reg);
+                    const double d_s = __shfl(F_s, (int)src), d_w = __shfl(F_w, (int)src);
+                    const double d_b = Tan ? __shfl(F_b, (int)src) : 0.0, d_gm = Tan ? __shfl(F_gm, (int)src) : 0.0;
+                    const double d_gs = Tan ? __shfl(F_gs, (int)src) : 0.0;
+                    const bool from_memory = thief && ((in_reg >> src) & 1ull) == 0;
+                    if (__ballot(from_memory))
+                        frames_read();  // (and written: vmcnt counts both)
                     if (thief) {
                         k = d_k - up;
-                        const Frame *f = (const Frame *)(stk0 + (size_t)k * kLevelBytes + src * sizeof(Frame));
-                        s = f->s;
-                        W = f->w;
+                        s = d_s;
+                        W = d_w;
                         if constexpr (Tan) {
-                            b = f->b;
-                            gm = f->gm;
-                            gs = f->gs;
+                            b = d_b;
+                            gm = d_gm;
+                            gs = d_gs;
                             u1 = d_u1;
+                        }
+                        if (from_memory) {
+                            const Frame *f = (const Frame *)(stk0 + (size_t)k * kLevelBytes + src * sizeof(Frame));
+                            s = f->s;
+                            W = f->w;
+                            if constexpr (Tan) {
+                                b = f->b;
+                                gm = f->gm;
+                                gs = f->gs;
+                            }
                         }
                         node = (d_node >> up) | (N)1;
                         pend = (N)1 << k;
