@@ -106,6 +106,12 @@ constexpr uint32_t kMinWalks = 256;
 // cells 18.5 (8), 20.6 (16).
 constexpr uint32_t kMultiSetFactor = 8;
 
+// Copies of a call's counters, one 128-byte line each; workgroup b adds to copy
+// b mod 64.  One copy for all wavefronts: at 1e6 shallow walks their adds to
+// one address came within 10 us and held up every CU's memory accesses for 30
+// us (forward pass of the 1e6-cell calibration instance 107 -> 74 us).
+constexpr uint32_t kCountCopies = 64, kCountWords = 16;
+
 // One parameter set of a relaxed plan (a single-set plan has one).  Rows,
 // initial cells, tally entries and type blocks of the sets are concatenated.
 struct RelaxSet {
@@ -147,7 +153,8 @@ struct RelaxArgs {
     double *h;                 // per set [rows][kdim][n_types] relaxed tally (forward)
     const double *g;           // cotangent, layout of h (backward)
     double *grad;              // per set [3][n_types] gradient (backward)
-    unsigned long long *expansions;  // [2] expansions of the call (roots drawn + nodes expanded), walks cut
+    unsigned long long *expansions;  // [kCountCopies][kCountWords] expansions of the call (roots drawn + nodes
+                                     // expanded), walks cut; the sum over the copies counts
     unsigned long long *set_cuts;    // [n_sets] walks cut per set (NULL: not kept)
     // Cell stride: a pass walks only the initial cells c (set-local id) with
     // (c + phase) & stride_mask == 0; phase = (*step + phase) & stride_mask
@@ -369,7 +376,7 @@ __device__ __forceinline__ uint32_t nth_set_bit(uint64_t m, uint32_t r)
 
 // LDS of a workgroup before its window: log and sin/cos tables | theta [3][T]
 // | (adjoint) gradient sums, up to 16 copies of [3][T] | proliferating types
-// u32 [T] | cursor of the root steps u32 [4] | entries, per wavefront [64]
+// u32 [T] | cursor of the root steps, walks cut, expansions u32 [4] | entries, per wavefront [64]
 // (once the roots are done: the walks' expansions by origin lane, u32 [64],
 // and each lane's origin, u32 [64]) | redraws' timers, per lane.  16 bytes
 // more for the gap behind the window's last copy.
@@ -516,8 +523,8 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
         prolif[i] = a.prolif[S.prolif_base + i];
     for (uint32_t i = tid; i < (Grad ? win_n : copies * win_stride); i += kWalkThreads)
         win[i] = Grad ? a.g[h0 + i] : 0.0;
-    if (tid == 0)
-        *cursor = 0u;
+    if (tid < 4)
+        cursor[tid] = 0u;
     __syncthreads();
 
     // Quiescent types: each initial cell of a row with value >= phi records p_j
@@ -1072,15 +1079,22 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
         w_exp += (uint64_t)__popcll(done);
     }
 
-    __syncthreads();
-    if (lane == 0)
-        atomicAdd(args_again().expansions, (unsigned long long)w_exp);
     for (int o = 32; o > 0; o >>= 1)
         n_cut += __shfl_xor(n_cut, o);
-    if (lane == 0 && n_cut) {
-        atomicAdd(args_again().expansions + 1, (unsigned long long)n_cut);
-        if (args_again().set_cuts)
-            atomicAdd(args_again().set_cuts + set_id, (unsigned long long)n_cut);
+    if (lane == 0) {
+        atomicAdd((unsigned long long *)(cursor + 2), (unsigned long long)w_exp);
+        if (n_cut)
+            atomicAdd(cursor + 1, n_cut);
+    }
+    __syncthreads();
+    if (tid == 0) {
+        unsigned long long *count = args_again().expansions + (seg % kCountCopies) * kCountWords;
+        atomicAdd(count, *(unsigned long long *)(cursor + 2));
+        if (cursor[1]) {
+            atomicAdd(count + 1, (unsigned long long)cursor[1]);
+            if (args_again().set_cuts)
+                atomicAdd(args_again().set_cuts + set_id, (unsigned long long)cursor[1]);
+        }
     }
     if constexpr (Grad) {
         for (uint32_t i = tid; i < 3 * T; i += kWalkThreads) {
@@ -1446,7 +1460,7 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
     const size_t o_sr = take(seg_row.size() * 4 + 4), o_rs = take(row_start.size() * 4);
     const size_t o_ri = take(row_info.size() * 4 + 4);
     const size_t o_pr = take(prolif.size() * 4 + 4), o_qu = take(quiet.size() * 4 + 4);
-    const size_t o_ex = take(16 + (size_t)n * 8);  // expansions, walks cut, walks cut per set
+    const size_t o_ex = take((kCountCopies * kCountWords + (size_t)n) * 8);  // counters, walks cut per set
     if (hipMalloc(&c.d_block, off) != hipSuccess)
         return PROCELL_E_OUT_OF_MEMORY;
     char *base = (char *)c.d_block;
@@ -1477,7 +1491,7 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
     a.prolif = (const uint32_t *)(base + o_pr);
     a.quiet = (const uint32_t *)(base + o_qu);
     a.expansions = (unsigned long long *)(base + o_ex);
-    a.set_cuts = a.expansions + 2;
+    a.set_cuts = a.expansions + kCountCopies * kCountWords;
     a.h_total = c.h_total;
     if (c.n_segments) {
         const size_t stack_bytes = (size_t)c.n_segments * kWalkThreads * (kdim_max + 1) * kFrameBytes;
@@ -1754,6 +1768,19 @@ void destroy_calib(procell_calib *c)
     delete c;
 }
 
+// Expansions and walks cut of a pass, from its device counters.
+hipError_t read_counts(const unsigned long long *counts, uint64_t &expansions, uint64_t &cut)
+{
+    unsigned long long c[kCountCopies * kCountWords];
+    const hipError_t e = hipMemcpy(c, counts, sizeof c, hipMemcpyDeviceToHost);
+    expansions = cut = 0;
+    for (uint32_t i = 0; i < kCountCopies && e == hipSuccess; ++i) {
+        expansions += c[i * kCountWords];
+        cut += c[i * kCountWords + 1];
+    }
+    return e;
+}
+
 int relaxed_call(procell_relaxed *r, int mode, const double *theta, double *h, const double *g, double *gr,
                  double *jac, void *stream)
 {
@@ -1765,11 +1792,11 @@ int relaxed_call(procell_relaxed *r, int mode, const double *theta, double *h, c
     a.g = g;
     a.grad = gr;
     a.jac = jac;
-    const uint64_t n_h = r->core.h_total;
+    const uint64_t n_h = r->core.h_total, n_counts = kCountCopies * kCountWords + a.n_sets;
     if (mode == kAdjoint)
-        RELAX_TRY(clear_ranges(a.expansions, 2ull + a.n_sets, gr, 3ull * r->core.types_total, nullptr, 0, st));
+        RELAX_TRY(clear_ranges(a.expansions, n_counts, gr, 3ull * r->core.types_total, nullptr, 0, st));
     else
-        RELAX_TRY(clear_ranges(a.expansions, 2ull + a.n_sets, h, n_h, jac, mode == kJacobian ? 2 * n_h : 0, st));
+        RELAX_TRY(clear_ranges(a.expansions, n_counts, h, n_h, jac, mode == kJacobian ? 2 * n_h : 0, st));
     RELAX_TRY(core_launch(r->core, a, mode, st));
     return PROCELL_OK;
 }
@@ -1902,12 +1929,9 @@ int procell_relaxed_expansions(procell_relaxed *r, uint64_t *n)
         return PROCELL_E_INVALID;
     RELAX_TRY(hipSetDevice(r->core.device));
     RELAX_TRY(hipDeviceSynchronize());
-    unsigned long long v = 0;
-    unsigned long long v2[2] = {0, 0};
-    RELAX_TRY(hipMemcpy(v2, r->core.args.expansions, sizeof v2, hipMemcpyDeviceToHost));
-    v = v2[0];
-    *n = v;
-    return v2[1] ? PROCELL_E_DEPTH : PROCELL_OK;
+    uint64_t cut = 0;
+    RELAX_TRY(read_counts(r->core.args.expansions, *n, cut));
+    return cut ? PROCELL_E_DEPTH : PROCELL_OK;
 }
 
 int procell_relaxed_set_cuts(procell_relaxed *r, uint64_t *cuts, void *stream)
@@ -2054,7 +2078,7 @@ int procell_calib_create(const procell_params *sets, uint32_t n_sets, double bet
     c->jac_route = cell_stride == 1;
     const size_t jac_words = c->jac_route ? 2ull * core.h_total : 0;
     const size_t s_h = stake(0);
-    const size_t clear_bytes = (core.h_total + jac_words) * 8 + P * 8 + 16;
+    const size_t clear_bytes = (core.h_total + jac_words + P + kCountCopies * kCountWords) * 8;
     so = (clear_bytes + 255) / 256 * 256;
     const size_t s_x = stake(P * 8), s_m1 = stake(P * 8), s_m2 = stake(P * 8), s_th = stake(P * 8);
     const size_t s_g = stake(c->jac_route ? 8 : core.h_total * 8 + 8), s_hb = stake(n_bins_total * 8 + 8);
@@ -2197,11 +2221,11 @@ int procell_calib_loss(procell_calib *c, double *loss, uint32_t capacity, uint64
         RELAX_TRY(hipMemcpy(&s, c->cargs.step, 8, hipMemcpyDeviceToHost));
         *steps = s;
     }
-    unsigned long long ex[2] = {0, 0};
-    RELAX_TRY(hipMemcpy(ex, c->fwd.expansions, sizeof ex, hipMemcpyDeviceToHost));
+    uint64_t ex = 0, cut = 0;
+    RELAX_TRY(read_counts(c->fwd.expansions, ex, cut));
     if (expansions)
-        *expansions = ex[0];
-    return ex[1] ? PROCELL_E_DEPTH : PROCELL_OK;
+        *expansions = ex;
+    return cut ? PROCELL_E_DEPTH : PROCELL_OK;
 }
 
 void *procell_calib_stream(procell_calib *c) { return c ? (void *)c->stream : nullptr; }
