@@ -66,7 +66,7 @@ typedef struct {
 /* Launch knobs.  0 means "choose automatically".  Results never depend on
  * them; only speed does. */
 typedef struct {
-    uint32_t block_size;    /* threads per workgroup: 64..256, multiple of 64 */
+    uint32_t block_size;    /* threads per workgroup: 64..256, multiple of 64 (automatic: up to 512) */
     uint32_t blocks_per_cu; /* resident workgroups per CU */
     uint32_t segments;      /* segments of initial cells per resident workgroup (1..64); the
                                workgroups of later segments start as earlier ones finish */
@@ -98,7 +98,7 @@ typedef struct {
     uint64_t rejected;    /* normal draws rejected because the timer was <= 0 */
     uint64_t cells;       /* initial cells */
     uint64_t pool;        /* initial cells that divided at least once */
-    double ms_tree;       /* device time of the last run's kernels: clearing, roots, trees (PROCELL_FLAG_TIMING) */
+    double ms_tree;       /* device time of the last run's kernels: clearing, simulation (PROCELL_FLAG_TIMING) */
     double ms_run;        /* device time of the whole run incl. clearing (PROCELL_FLAG_TIMING; = ms_tree) */
     uint32_t workgroups;  /* launch shape chosen for the run */
     uint32_t block_size;
@@ -167,17 +167,17 @@ int procell_plan_destroy(procell_plan *plan);
 void *procell_plan_stream(procell_plan *plan);                       /* hipStream_t */
 /* With PROCELL_FLAG_TIMING: device time (ms) of the kernels of each of the
  * last min(runs, 256, max_runs) runs since the previous call (the clearing
- * kernel, the root kernel and the tree kernel, back to back), oldest first,
- * from HIP events recorded on the plan's stream around the three kernels.
+ * kernel and the simulation kernel, back to back), oldest first, from HIP
+ * events recorded on the plan's stream around the two.
  * Waits for the stream; resets the run count. */
 int procell_plan_kernel_times(procell_plan *plan, double *ms, uint32_t max_runs, uint32_t *n_runs);
 
 /* ---- batched plain method: many parameter sets per launch --------------
  * No reference counterpart (the reference simulates one parameter set per
  * process).  The sets' initial cells, rows, types and tallies are
- * concatenated and run by one launch of each kernel; every tree workgroup
+ * concatenated and run by one launch of each kernel; every workgroup
  * works on one set.  Set i's result equals procell_simulate of sets[i] with
- * seed seeds[i], bit for bit.  Runs replay one hipGraph of the three
+ * seed seeds[i], bit for bit.  Runs replay one hipGraph of the two
  * kernels, captured on the first run.  All sets must name the same device;
  * the launch knobs, flags and stream of sets[0] apply to the batch.  On a
  * batch plan, procell_plan_run gives every set the same seed and
