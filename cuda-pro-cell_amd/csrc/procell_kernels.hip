@@ -904,7 +904,9 @@ __global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a
     const uint32_t cell0 = (uint32_t)(seg_begin - S.cell_base);
     for (uint32_t i = tid; i < T; i += bdim) {
         const double cum = a.type_cum[S.type_base + i], m = a.type_mean[S.type_base + i], sd = a.type_sd[S.type_base + i];
-        types[i] = FilterType{(float)m, (float)sd, type_err(m, sd, t_max), a.type_file[S.type_base + i]};
+        // the sign of a quiescent type's mean from the 64-bit value: one above
+        // -2^-150 rounds to -0 in single precision
+        types[i] = FilterType{m < 0.0 ? -1.0f : (float)m, (float)sd, type_err(m, sd, t_max), a.type_file[S.type_base + i]};
         // w 2^-32 < cum for a whole number w: w < ceil(cum 2^32); a limit of
         // 2^32 or more is stored as 2^32 - 1, and a drawn 2^32 - 1 looked at
         // again (the sums are > 0: the largest proportion comes first and the
