@@ -1107,14 +1107,27 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
                 unsafeAtomicAdd(args_again().grad + set_again().theta_base + i, v);
         }
     } else {
+        // p_j and 1 / beta multiply the sums.  Where p_j is not finite, an entry
+        // whose records are all exactly 0 (the sigmoid 1) is not 0 either: the
+        // product reaches every entry that the row's walks of type j may record
+        // in.
+        const uint32_t n_prolif_w = set_again().n_prolif;
+        auto may_record = [&](uint32_t e) {
+            const uint32_t gen = e % KT / T, info = args_again().row_info[w_lo + e / KT];
+            bool walks = false;
+            for (uint32_t q = 0; q < n_prolif_w; ++q)
+                walks = walks || prolif[q] == e % T;
+            return walks && gen <= (info & 255u) && (gen > 0 || ((info >> 8) & 1u) != 0);
+        };
         for (uint32_t i = tid; i < kParts * win_n; i += kWalkThreads) {
             double v = win[i];
             for (uint32_t k = 1; k < copies; ++k)
                 v += win[k * win_stride + i];
-            if (v != 0.0) {
-                const uint32_t e = i / kParts, part = i - e * kParts;
+            const uint32_t e = i / kParts, part = i - e * kParts;
+            const double p = theta[2 * T + e % T];
+            if (v != 0.0 || (!(fabs(p) <= 0x1.fffffffffffffp1023) && may_record(e))) {
                 double *dst = part == 0 ? args_again().h : args_again().jac + (uint64_t)(part - 1) * args_again().h_total;
-                unsafeAtomicAdd(dst + h0 + e, v * theta[2 * T + e % T] * (part ? ib : 1.0));
+                unsafeAtomicAdd(dst + h0 + e, v * p * (part ? ib : 1.0));
             }
         }
     }
