@@ -647,6 +647,12 @@ int run_plan(procell_plan *pl, const uint64_t *seeds, uint64_t seed, bool use_gr
 {
     HIP_TRY(hipSetDevice(pl->device));
     const uint32_t n_sets = pl->args.n_sets;
+    {
+        // from here on the device's tallies may be this run's, also if a later
+        // step fails: sets staged from an earlier run are not served any more
+        std::lock_guard<std::mutex> lk(pl->result_mu);
+        ++pl->run_id;
+    }
     // timing events bracket the whole run: an event recorded between two
     // kernels of the run would add a gap of several microseconds there
     const size_t slot = (size_t)(pl->runs % kTimedRuns);
@@ -685,7 +691,6 @@ int run_plan(procell_plan *pl, const uint64_t *seeds, uint64_t seed, bool use_gr
         pl->timed = true;
     }
     ++pl->runs;
-    ++pl->run_id;
     pl->ran = true;
     return PROCELL_OK;
 }
