@@ -55,6 +55,7 @@
 
 #include "procell_internal.hpp"
 #include "procell_stream.hpp"
+#include "procell_walk.hpp"
 
 namespace procell {
 namespace {
@@ -1241,49 +1242,6 @@ void core_free(RelaxCore &c)
     c.d_stack = nullptr;
 }
 
-// One workgroup's initial cells.
-struct Segment {
-    uint32_t set;
-    uint32_t c0, c1;  // first and end initial cell (set-local)
-    uint32_t r0, r1;  // first and last row (global)
-};
-
-// Splits the initial cells of one set into `n_seg` segments of equal cost
-// (fewer where a cell costs more than that).
-void split_set(const Setup &s, const std::vector<double> &cell_cost, uint64_t n_seg, uint32_t set, uint32_t row_base,
-               std::vector<Segment> &out)
-{
-    const uint32_t n_rows = (uint32_t)s.v.size();
-    double total = 0.0;
-    for (uint32_t i = 0; i < n_rows; ++i)
-        total += cell_cost[i] * (double)(s.start[i + 1] - s.start[i]);
-    auto row_of = [&](uint64_t cell) {
-        return row_base + (uint32_t)(std::upper_bound(s.start.begin(), s.start.end() - 1, cell) - s.start.begin() - 1);
-    };
-    uint32_t row = 0;
-    double acc = 0.0;  // cost of the rows before `row`
-    uint64_t c0 = 0;
-    for (uint64_t v = 1; v <= n_seg; ++v) {
-        uint64_t c1 = s.n_cells;
-        if (v < n_seg) {
-            const double want = total * ((double)v / (double)n_seg);
-            for (; row < n_rows; ++row) {
-                const double rc = cell_cost[row] * (double)(s.start[row + 1] - s.start[row]);
-                if (acc + rc > want)
-                    break;
-                acc += rc;
-            }
-            if (row < n_rows) {
-                c1 = s.start[row] + (uint64_t)std::max(0.0, ceil((want - acc) / cell_cost[row]));
-                c1 = std::max(c0, std::min<uint64_t>(c1, s.start[row + 1]));
-            }
-        }
-        if (c1 > c0)
-            out.push_back(Segment{set, (uint32_t)c0, (uint32_t)c1, row_of(c0), row_of(c1 - 1)});
-        c0 = c1;
-    }
-}
-
 // Validates the sets, cuts their initial cells into the workgroups' segments
 // and uploads the tables.
 int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, bool want_bins)
@@ -1416,7 +1374,7 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
         const double share = all_cost > 0.0 ? set_cost[i] / all_cost * (double)budget : 1.0;
         const uint64_t most = (units[i] + kMinWalks - 1) / kMinWalks;
         split_set(s, cell_cost[i], std::max<uint64_t>(1, std::min((uint64_t)floor(share + 0.5), most)), i,
-                  c.sets[i].row_base, segs);
+                  c.sets[i].row_base, kMaxSegmentUnits / ((c.sets[i].n_prolif + 63) / 64), segs);
     }
     if (segs.size() > 0x7FFFFFFFull)
         return PROCELL_E_TOO_MANY_CELLS;
