@@ -71,10 +71,6 @@ constexpr uint32_t kWalkBudget = 1u << 22;
 // (for untruncated normal timers it would diverge beyond sd / mean = 0.85,
 // where mean^2 / (2 sd^2) = ln 2), so the bound keeps the walks cheap.
 constexpr double kLogMaxSdRatio = -0.22314355131420976;
-// A workgroup: one wavefront per SIMD, a quarter of a CU's LDS.  128 registers
-// and four wavefronts per SIMD; five (the forward pass: six) gained nothing,
-// the walks in flight then being more and the end of a launch longer.
-constexpr uint32_t kWalkThreads = 256;
 constexpr uint32_t kWalkWaves = kWalkThreads / 64;
 constexpr size_t kWalkLds = 40960;
 // Idle lanes a wavefront tolerates before it draws roots (some 220
@@ -84,14 +80,6 @@ constexpr size_t kWalkLds = 40960;
 constexpr uint32_t kWalkIdle = 12;
 constexpr uint32_t kNoWindow = 0xFFFFFFFFu;
 constexpr uint32_t kMaxCopies = 8;   // of a workgroup's window
-constexpr uint32_t kGradSums = 384;  // gradient sums of a workgroup, all copies
-
-// What a pass of the walk computes.
-enum WalkMode : int {
-    kForward = 0,   // h
-    kAdjoint = 1,   // gradient of <g, h>
-    kJacobian = 2,  // h and its derivatives in each type's mean and sd
-};
 
 // Expected expansions of a walk from which the last root steps of a segment
 // are claimed in parts: a root step of short walks costs more than the
@@ -338,6 +326,9 @@ struct alignas(16) WalkEntry<true> {
     uint32_t cell, tb, rowt, kcap;
 };
 
+static_assert(sizeof(WalkEntry<false>) == walk_entry_bytes(false) && sizeof(WalkEntry<true>) == walk_entry_bytes(true),
+              "LDS layout");
+
 // Stacked right daughter: completion time and W d; tangent passes also ds/dsd
 // and its daughters' dlogW/dmean, dlogW/dsd (padded to 16-byte words).
 template <bool Tan>
@@ -373,19 +364,6 @@ __device__ __forceinline__ uint32_t nth_set_bit(uint64_t m, uint32_t r)
     for (; r; --r)
         m &= m - 1;
     return (uint32_t)__builtin_ctzll(m);
-}
-
-// LDS of a workgroup before its window: log and sin/cos tables | theta [3][T]
-// | (adjoint) gradient sums, up to 16 copies of [3][T] | proliferating types
-// u32 [T] | cursor of the root steps, walks cut, expansions u32 [4] | entries, per wavefront [64]
-// (once the roots are done: the walks' expansions by origin lane, u32 [64],
-// and each lane's origin, u32 [64]) | redraws' timers, per lane.  16 bytes
-// more for the gap behind the window's last copy.
-__host__ __device__ constexpr size_t walk_lds_fixed(uint32_t n_types, int mode)
-{
-    const size_t theta = 3 * (size_t)n_types, sums = mode == kAdjoint ? (theta > kGradSums ? theta : kGradSums) : 0;
-    return 384 * 16 + (theta + sums) * 8 + ((size_t)n_types * 4 + 15) / 16 * 16 + 16 +
-           kWalkThreads * (16 + (mode == kForward ? sizeof(WalkEntry<false>) : sizeof(WalkEntry<true>))) + 16;
 }
 
 __device__ __forceinline__ uint64_t again_value(uint64_t x)
@@ -444,7 +422,7 @@ __device__ __forceinline__ P *again(P *p)
 //    SIMD's wavefronts, so that the youngest ends alone, at a third of the
 //    rate; a wavefront of a segment with more left to claim takes a higher
 //    priority (242 -> 232 us).
-// LDS: see walk_lds_fixed; the window follows.
+// LDS: see walk_lds.
 // ======================================================================
 template <int Mode, typename N>
 __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
@@ -476,16 +454,17 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
     const uint32_t first = uni(c_begin + ((0u - (c_begin + phase)) & a.stride_mask));
     const uint32_t n_sel = uni(first >= c_begin && c_end > first ? ((c_end - 1u - first) >> sshift) + 1u : 0u);
 
+    const WalkLds at_lds = walk_lds(T, Mode);
     double(*m_log)[2] = (double(*)[2])lds_raw;
     double(*m_sc)[2] = (double(*)[2])(lds_raw + 128 * 16);
-    double *theta = (double *)(lds_raw + 384 * 16);
-    double *gsum = theta + 3 * T;
-    uint32_t *prolif = (uint32_t *)(gsum + (Grad ? max(kGradSums, 3 * T) : 0u));
-    uint32_t *cursor = (uint32_t *)((unsigned char *)prolif + ((size_t)T * 4 + 15) / 16 * 16);
-    Entry *ent = (Entry *)(cursor + 4) + wave * 64;
-    double *held = (double *)((Entry *)(cursor + 4) + kWalkThreads) + tid * 2;  // a waiting lane's timers
+    double *theta = (double *)(lds_raw + at_lds.theta);
+    double *gsum = (double *)(lds_raw + at_lds.sums);
+    uint32_t *prolif = (uint32_t *)(lds_raw + at_lds.prolif);
+    uint32_t *cursor = (uint32_t *)(lds_raw + at_lds.cursor);
+    Entry *ent = (Entry *)(lds_raw + at_lds.entries) + wave * 64;
+    double *held = (double *)(lds_raw + at_lds.held) + tid * 2;  // a waiting lane's timers
     uint32_t *origin_exp = (uint32_t *)ent, *origin = origin_exp + 64;  // (steals)
-    double *win = (double *)((Entry *)(cursor + 4) + kWalkThreads) + kWalkThreads * 2;
+    double *win = (double *)(lds_raw + at_lds.window);
     const uint32_t win_base = (uint32_t)(uintptr_t)(LdsDouble *)win;
     const uint32_t n_win = min(r_hi - w_lo + 1, a.win_doubles[Mode] / (KT * kParts));  // rows with a window
     const uint32_t win_n = n_win * KT;
@@ -1320,7 +1299,7 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
     uint32_t win_cap[3];
     int occ = 0;
     for (int m = 0; m < 3; ++m) {
-        const size_t fixed = walk_lds_fixed(t_max_types, m);
+        const size_t fixed = (size_t)walk_lds(t_max_types, m).fixed;
         win_cap[m] = fixed < kWalkLds ? (uint32_t)((kWalkLds - fixed) / 8) : 0u;
         int o = 0;
         RELAX_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, walk_kernel_of(m, kdim_max), (int)kWalkThreads,
@@ -1415,7 +1394,7 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
     }
     for (int m = 0; m < 3; ++m) {
         c.args.win_doubles[m] = (uint32_t)std::min<uint64_t>(win_cap[m], (entries * (m == kJacobian ? 3 : 1) + 1) * (m == kAdjoint ? 1 : 8));
-        c.lds_bytes[m] = walk_lds_fixed(t_max_types, m) + (size_t)c.args.win_doubles[m] * 8;
+        c.lds_bytes[m] = (size_t)walk_lds(t_max_types, m).fixed + (size_t)c.args.win_doubles[m] * 8;
     }
 
     // ---- upload ----

@@ -11,7 +11,58 @@
 
 #include "procell_setup.hpp"
 
+#ifdef __HIP__
+#define PROCELL_WALK_HD __host__ __device__
+#else
+#define PROCELL_WALK_HD
+#endif
+
 namespace procell {
+
+// What a pass of the walk computes.
+enum WalkMode : int {
+    kForward = 0,   // h
+    kAdjoint = 1,   // gradient of <g, h>
+    kJacobian = 2,  // h and its derivatives in each type's mean and sd
+};
+
+// A workgroup: one wavefront per SIMD, a quarter of a CU's LDS.  128 registers
+// and four wavefronts per SIMD; five (the forward pass: six) gained nothing,
+// the walks in flight then being more and the end of a launch longer.
+constexpr uint32_t kWalkThreads = 256;
+constexpr uint32_t kWalkTables = 384;  // entries of the log and sin/cos tables
+constexpr uint32_t kGradSums = 384;    // gradient sums of a workgroup, all copies
+
+// Bytes of a buffered root walk: without and with tangents.
+PROCELL_WALK_HD constexpr uint32_t walk_entry_bytes(bool tan) { return tan ? 48u : 32u; }
+
+// LDS of a workgroup, in bytes from its start: log and sin/cos tables | theta
+// [3][T] | (adjoint) gradient sums, up to 16 copies of [3][T] | proliferating
+// types u32 [T] | cursor of the root steps, walks cut, expansions u32 [4] |
+// entries, per wavefront [64] (once the roots are done: the walks' expansions
+// by origin lane, u32 [64], and each lane's origin, u32 [64]) | redraws'
+// timers, per lane | window.  Entries and timers are read and written in
+// 16-byte words, so every part starts at a multiple of 16 (3 T doubles are
+// not one where T is odd); 16 bytes more at the end (`fixed`) for the gap
+// behind the window's last copy.
+struct WalkLds {
+    uint32_t theta, sums, prolif, cursor, entries, held, window, fixed;
+};
+
+PROCELL_WALK_HD constexpr WalkLds walk_lds(uint32_t n_types, int mode)
+{
+    const uint32_t n = 3 * n_types, sums = mode == kAdjoint ? (n > kGradSums ? n : kGradSums) : 0u;
+    WalkLds l{};
+    l.theta = kWalkTables * 16;
+    l.sums = l.theta + n * 8;
+    l.prolif = (l.sums + sums * 8 + 15) / 16 * 16;
+    l.cursor = l.prolif + (n_types * 4 + 15) / 16 * 16;
+    l.entries = l.cursor + 16;
+    l.held = l.entries + kWalkThreads * walk_entry_bytes(mode != kForward);
+    l.window = l.held + kWalkThreads * 16;
+    l.fixed = l.window + 16;
+    return l;
+}
 
 // One workgroup's initial cells.
 struct Segment {

@@ -46,12 +46,30 @@ static void check_segments()
             }
 }
 
+// Every part of a workgroup's LDS starts at a multiple of 16 bytes and holds
+// what it is for, for any number of types; entries and timers, read and
+// written in 16-byte words, stay on them for every lane.
+static void check_lds()
+{
+    for (int mode : {kForward, kAdjoint, kJacobian})
+        for (uint32_t t = 1; t <= 256; ++t) {
+            const WalkLds l = walk_lds(t, mode);
+            const uint32_t sums = mode == kAdjoint ? std::max(kGradSums, 3 * t) : 0;
+            for (uint32_t at : {l.theta, l.prolif, l.cursor, l.entries, l.held, l.window, walk_entry_bytes(mode != kForward)})
+                CHECK(at % 16 == 0);
+            CHECK(l.theta >= kWalkTables * 16 && l.sums >= l.theta + 3 * t * 8 && l.sums % 8 == 0);
+            CHECK(l.prolif >= l.sums + sums * 8 && l.cursor >= l.prolif + 4 * t && l.entries >= l.cursor + 16);
+            CHECK(l.held >= l.entries + kWalkThreads * walk_entry_bytes(mode != kForward));
+            CHECK(l.window >= l.held + kWalkThreads * 16 && l.fixed >= l.window + 8 && l.fixed <= 40960);
+        }
+}
+
 int main(int argc, char **argv)
 {
     const struct {
         const char *name;
         void (*f)();
-    } checks[] = {{"segments", check_segments}};
+    } checks[] = {{"segments", check_segments}, {"lds", check_lds}};
     for (const auto &c : checks)
         if (argc == 2 && !strcmp(argv[1], c.name)) {
             c.f();

@@ -31,3 +31,7 @@ def walk_checks(tmp_path_factory):
 
 def test_segments_of_any_size(walk_checks):
     walk_checks("segments")
+
+
+def test_lds_parts_are_aligned(walk_checks):
+    walk_checks("lds")
