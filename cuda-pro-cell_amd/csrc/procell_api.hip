@@ -180,9 +180,9 @@ uint32_t segments_per_workgroup(double lane_steps, bool filter)
 // With `arena` (device memory of `arena_bytes`, already on ps[0].device) the
 // plan's device block is carved from it instead of allocated, no stream or
 // event is created (the plan runs on ps[0].stream, NULL: the default stream)
-// and timing is off.
+// and timing is off.  Without `may_filter` the plan keeps the 64-bit kernel.
 int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, void *arena = nullptr,
-                size_t arena_bytes = 0)
+                size_t arena_bytes = 0, bool may_filter = true)
 {
     if (!ps || !out || n_sets == 0)
         return PROCELL_E_INVALID;
@@ -278,7 +278,7 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     // 2.65 ms per run at 2 workgroups per CU, 5.9 ms at 3 or 4 without a window).
     const bool gstack = n_sets > 1 && a.stack_levels > kLdsStackLevels;
     const uint32_t lds_levels = gstack ? 0u : a.stack_levels;
-    const bool filter = filter_covers(pl->setups);
+    const bool filter = may_filter && filter_covers(pl->setups);
     // row tables (8 bytes per row) go to LDS when they are small and do not
     // cost a resident workgroup (the root steps read them when a wavefront's
     // rows advance, so from device memory they cost little).  The filtered
@@ -493,8 +493,12 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     const size_t o_seed = off; off = align_up(off + (size_t)n_sets * 8, 256);
     const size_t o_gs = off; off = align_up(off + (gstack ? (size_t)g * sim_stack_bytes(a.stack_levels, (uint32_t)bs, filter) : 0), 256);
     if (arena) {
-        if (off > arena_bytes)
-            return fail(PROCELL_E_SCRATCH);
+        if (off > arena_bytes) {
+            // the filtered kernel's tables take 4 bytes per row more: what only
+            // fits without them runs on the 64-bit kernel
+            destroy_plan(pl);
+            return filter ? create_plan(ps, n_sets, out, arena, arena_bytes, false) : PROCELL_E_SCRATCH;
+        }
         pl->stream = (hipStream_t)ps[0].stream;
         pl->d_block = arena;
         pl->own_block = false;

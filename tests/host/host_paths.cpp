@@ -71,12 +71,29 @@ static void check_stage()
     CHECK(procell_plan_destroy(b) == PROCELL_OK);
 }
 
+// procell_simulate_noalloc: 16 MiB of static memory for the counters, 8 bytes
+// per tally entry and 8 of tables per row, so some 1.04e6 rows of one
+// generation and one type, and not many more.
+static void check_noalloc()
+{
+    for (uint64_t n : {1000ull, 835000ull, 900000ull, 1040000ull, 1060000ull}) {
+        std::vector<procell_row> rows(n);
+        for (uint64_t i = 0; i < n; ++i)
+            rows[i] = {1.0 + (double)i / (double)(2 * n), 1};
+        Case c(rows, {{1.0, 20.0, 5.0}}, 90.0, 1.0);
+        const uint64_t before = fake::sim_runs;
+        const int rc = procell_simulate_noalloc(&c.p, &c.r);
+        CHECK(rc == (n > 1050000 ? PROCELL_E_SCRATCH : PROCELL_OK));
+        CHECK(fake::sim_runs == before + (rc == PROCELL_OK) && fake::memory_alive == 0);
+    }
+}
+
 int main(int argc, char **argv)
 {
     const struct {
         const char *name;
         void (*f)();
-    } checks[] = {{"stage", check_stage}};
+    } checks[] = {{"stage", check_stage}, {"noalloc", check_noalloc}};
     for (const auto &c : checks)
         if (argc == 2 && !strcmp(argv[1], c.name)) {
             c.f();

@@ -40,3 +40,7 @@ def host_paths(procell_lib, tmp_path_factory):
 
 def test_results_after_a_run_that_failed_late(host_paths):
     host_paths("stage")
+
+
+def test_rows_that_fit_the_static_scratch(host_paths):
+    host_paths("noalloc")
