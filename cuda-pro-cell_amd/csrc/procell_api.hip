@@ -812,23 +812,55 @@ int plan_result(procell_plan *pl, uint32_t set, procell_result *r)
     return merge_tally(s, *bin_of, tally.data(), r);
 }
 
-// Streams of procell_simulate calls: making and destroying one took 58 us of
-// a small call's 190.  Up to kKeptStreams idle ones per device wait for the
-// next call; a call takes one for itself and gives it back once its work has
-// ended, so concurrent calls never share one.
+// Streams of procell_simulate calls: making and destroying one took 58 us of a
+// small call's 146.  Up to kKeptStreams idle ones per device wait for the next
+// call; a call takes one for itself and gives it back once its work has ended,
+// so concurrent calls never share one.  The host program's hipDeviceReset
+// deletes them with everything else on the device, and their handles may then
+// belong to streams of its own.  So a small device allocation is kept beside
+// them: while the runtime knows it by the same allocation id (unique in the
+// process; 0.06 us to ask for), there was no reset, else the handles are
+// forgotten and never used.
 constexpr int kKeptDevices = 64, kKeptStreams = 4;
-std::mutex g_stream_mu;
-hipStream_t g_streams[kKeptDevices][kKeptStreams];
-int g_n_streams[kKeptDevices];
+struct KeptStreams {
+    std::mutex mu;
+    hipStream_t stream[kKeptStreams];
+    int n = 0;
+    void *mark = nullptr;
+    uint64_t mark_id = 0;
+};
+KeptStreams g_kept[kKeptDevices];
+
+// The id of a device allocation, 0 if there is none at p.
+uint64_t allocation_id(void *p)
+{
+    uint64_t id = 0;
+    if (!p || hipPointerGetAttribute(&id, HIP_POINTER_ATTRIBUTE_BUFFER_ID, (hipDeviceptr_t)p) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return id;
+}
+
+// Whether k's streams still exist (under k.mu).
+bool kept_valid(KeptStreams &k)
+{
+    if (k.mark && allocation_id(k.mark) == k.mark_id)
+        return true;
+    k.n = 0;
+    k.mark = nullptr;
+    return false;
+}
 
 hipStream_t borrow_stream(int device)
 {
     if (device < 0 || device >= kKeptDevices)
         return nullptr;
     {
-        std::lock_guard<std::mutex> lk(g_stream_mu);
-        if (g_n_streams[device] > 0)
-            return g_streams[device][--g_n_streams[device]];
+        KeptStreams &k = g_kept[device];
+        std::lock_guard<std::mutex> lk(k.mu);
+        if (kept_valid(k) && k.n > 0)
+            return k.stream[--k.n];
     }
     int n_cu = 0;
     hipStream_t st = nullptr;
@@ -842,9 +874,20 @@ void return_stream(int device, hipStream_t st)
     if (!st)
         return;
     if (hipSetDevice(device) == hipSuccess && hipStreamSynchronize(st) == hipSuccess) {
-        std::lock_guard<std::mutex> lk(g_stream_mu);
-        if (g_n_streams[device] < kKeptStreams) {
-            g_streams[device][g_n_streams[device]++] = st;
+        KeptStreams &k = g_kept[device];
+        std::lock_guard<std::mutex> lk(k.mu);
+        if (!kept_valid(k)) {
+            void *mark = nullptr;
+            if (hipMalloc(&mark, 8) == hipSuccess) {
+                k.mark_id = allocation_id(mark);
+                if (k.mark_id)
+                    k.mark = mark;
+                else  // a runtime without ids: nothing is kept
+                    (void)hipFree(mark);
+            }
+        }
+        if (k.mark && k.n < kKeptStreams) {
+            k.stream[k.n++] = st;
             return;
         }
     }

@@ -19,19 +19,24 @@ namespace fake {
 std::vector<Launch> launches;
 uint64_t sim_runs = 0;
 int fail_event_record = 0;
-uint64_t dead_stream_uses = 0, streams_alive = 0, memory_alive = 0;
+uint64_t dead_stream_uses = 0, foreign_stream_uses = 0, streams_alive = 0, memory_alive = 0;
 static float one_ms() { return 1.0f; }
 float (*elapsed_ms)() = one_ms;
 std::vector<uint32_t> segment_cells;
 
 static std::map<const void *, std::string> names;
 static std::map<const void *, void *> symbols;  // static device variables
-static std::set<void *> memory, streams;
+static std::map<void *, uint64_t> memory;       // and the id of each allocation
+static std::set<void *> streams, foreign, freed;  // freed: small allocations, whose addresses come again
+static uint64_t next_id = 0;
+constexpr uintptr_t kFirstStream = 0x10;
+static uintptr_t next_stream = kFirstStream;
 static std::map<void *, std::vector<std::function<void()>>> capturing, graphs;
 static uintptr_t next_handle = 0x1000;
 
 static hipError_t check(hipStream_t st)
 {
+    foreign_stream_uses += foreign.count((void *)st);
     if (!st || streams.count((void *)st))
         return hipSuccess;
     ++dead_stream_uses;
@@ -40,11 +45,26 @@ static hipError_t check(hipStream_t st)
 
 void device_reset()
 {
-    for (void *p : memory)
-        free(p);
+    for (const auto &m : memory)
+        freed.insert(m.first);
     memory.clear();
     streams.clear();
+    foreign.clear();
+    next_stream = kFirstStream;
     memory_alive = streams_alive = 0;
+}
+
+void take_stream()
+{
+    hipStream_t st;
+    (void)hipStreamCreateWithFlags(&st, 0);
+    foreign.insert((void *)st);
+}
+
+void take_memory()
+{
+    void *p;
+    (void)hipMalloc(&p, 8);
 }
 
 static void run(const Launch &l, const procell::RunArgs *a)
@@ -132,8 +152,13 @@ hipError_t hipGetSymbolAddress(void **p, const void *host)
 }
 hipError_t hipMalloc(void **p, size_t n)
 {
-    *p = calloc(1, n ? n : 1);
-    memory.insert(*p);
+    if (n <= 64 && !freed.empty()) {
+        *p = *freed.begin();
+        freed.erase(freed.begin());
+    } else {
+        *p = calloc(1, n < 64 ? 64 : n);
+    }
+    memory[*p] = ++next_id;
     ++memory_alive;
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }
@@ -143,6 +168,13 @@ hipError_t hipFree(void *p)
         return hipErrorInvalidValue;
     memory_alive -= p != nullptr;
     free(p);
+    return hipSuccess;
+}
+hipError_t hipPointerGetAttribute(void *out, hipPointer_attribute what, hipDeviceptr_t p)
+{
+    if (what != HIP_POINTER_ATTRIBUTE_BUFFER_ID || !memory.count(p))
+        return hipErrorInvalidValue;
+    memcpy(out, &memory[p], 8);
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return *p = calloc(1, n), hipSuccess; }
@@ -158,7 +190,7 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipSt
 hipError_t hipMemset(void *p, int v, size_t n) { return memset(p, v, n), hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *st, unsigned)
 {
-    *st = (hipStream_t)(next_handle += 16);
+    *st = (hipStream_t)(next_stream += 16);
     streams.insert((void *)*st);
     ++streams_alive;
     return hipSuccess;

@@ -88,12 +88,35 @@ static void check_noalloc()
     }
 }
 
+// What procell_simulate keeps between calls (a few streams, one small
+// allocation) does not outlive a reset of the device: the next call uses
+// neither the handles from before, nor streams that the host program has got
+// under the same handles since, nor memory under the old address.
+static void check_reset()
+{
+    Case c({{100.0, 500}, {30.0, 300}}, {{1.0, 20.0, 5.0}}, 90.0, 1.0);
+    uint64_t runs = 0;
+    for (int i = 0; i < 4; ++i) {
+        for (int k = 0; k < 2; ++k) {
+            CHECK(procell_simulate(&c.p, &c.r) == PROCELL_OK);
+            CHECK(c.r.stats.divisions == ++runs);
+            CHECK(fake::streams_alive <= 4 + (i > 0) && fake::memory_alive <= 1 + (i > 0));
+        }
+        CHECK(fake::foreign_stream_uses == 0);
+        fake::device_reset();  // from here on the first handles and addresses come again
+        fake::take_stream();
+        if (i > 0)
+            fake::take_memory();
+    }
+    CHECK(fake::dead_stream_uses == 0);
+}
+
 int main(int argc, char **argv)
 {
     const struct {
         const char *name;
         void (*f)();
-    } checks[] = {{"stage", check_stage}, {"noalloc", check_noalloc}};
+    } checks[] = {{"stage", check_stage}, {"noalloc", check_noalloc}, {"reset", check_reset}};
     for (const auto &c : checks)
         if (argc == 2 && !strcmp(argv[1], c.name)) {
             c.f();

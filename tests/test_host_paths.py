@@ -44,3 +44,7 @@ def test_results_after_a_run_that_failed_late(host_paths):
 
 def test_rows_that_fit_the_static_scratch(host_paths):
     host_paths("noalloc")
+
+
+def test_calls_around_a_device_reset(host_paths):
+    host_paths("reset")
