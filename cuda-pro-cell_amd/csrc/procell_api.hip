@@ -278,7 +278,7 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     // 2.65 ms per run at 2 workgroups per CU, 5.9 ms at 3 or 4 without a window).
     const bool gstack = n_sets > 1 && a.stack_levels > kLdsStackLevels;
     const uint32_t lds_levels = gstack ? 0u : a.stack_levels;
-    const bool filter = may_filter && filter_covers(pl->setups);
+    const bool filter = may_filter && filter_covers(pl->setups) && filter_pays(pl->setups);
     // row tables (8 bytes per row) go to LDS when they are small and do not
     // cost a resident workgroup (the root steps read them when a wavefront's
     // rows advance, so from device memory they cost little).  The filtered

@@ -22,6 +22,7 @@
 // window over the first rows of the workgroup's segment and are added to the
 // int64 device tally at the end; rows outside the window use 64-bit device
 // atomics (aggregated per (row, type) for generation 0).
+#include "procell_filter.hpp"
 #include "procell_internal.hpp"
 #include "procell_stream.hpp"
 
@@ -674,10 +675,9 @@ __global__ void __launch_bounds__(256, 4) sim_kernel(RunArgs a)
 // t_max, so a value near the threshold is small, and no partial sum of a path
 // exceeds t_max) and 3.5 of those for t_max and the root's phase.  After k
 // levels below the root that is (k + 2) e + (k + 3.5) 2^-24 t_max with e =
-// 6.7e-6 |sd| + 1.2e-7 |mean|; type_err and cell_err round it up, with the
+// 6.7e-6 |sd| + 1.2e-7 |mean|; filter_type_err and filter_cell_err round it up, with the
 // row's cap for k.
 // ----------------------------------------------------------------------
-constexpr float kPairErr = 7.0e-6f;
 constexpr uint32_t kPairLow = 1u << 16;
 
 __device__ __forceinline__ bool pair_sure(uint32_t w0) { return w0 - kPairLow < 0u - 2u * kPairLow; }
@@ -691,15 +691,8 @@ __device__ __forceinline__ void normal_pair_f32(uint32_t w0, uint32_t w2, float 
     z1 = rho * __builtin_amdgcn_sinf(turn);
 }
 
-__device__ __forceinline__ float type_err(double mean, double sd, double t_max)
-{
-    return (float)(fabs(sd) * ((double)kPairErr + 0x1p-20) + 0x1p-22 * fabs(mean) + 0x1p-23 * t_max);
-}
-
 // Smaller of two magnitudes.
 __device__ __forceinline__ float min_abs(float x, float y) { return fminf(fabsf(x), fabsf(y)); }
-
-__device__ __forceinline__ float cell_err(uint32_t kcap, float terr) { return (float)(kcap + 4u) * terr; }
 
 // Completion times in 64 bits, minus t_max and rounded to single precision
 // (which keeps the sign of the 64-bit comparison: the difference of two
@@ -906,7 +899,7 @@ __global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a
         const double cum = a.type_cum[S.type_base + i], m = a.type_mean[S.type_base + i], sd = a.type_sd[S.type_base + i];
         // the sign of a quiescent type's mean from the 64-bit value: one above
         // -2^-150 rounds to -0 in single precision
-        types[i] = FilterType{m < 0.0 ? -1.0f : (float)m, (float)sd, type_err(m, sd, t_max), a.type_file[S.type_base + i]};
+        types[i] = FilterType{m < 0.0 ? -1.0f : (float)m, (float)sd, (float)filter_type_err(m, sd, t_max), a.type_file[S.type_base + i]};
         // w 2^-32 < cum for a whole number w: w < ceil(cum 2^32); a limit of
         // 2^32 or more is stored as 2^32 - 1, and a drawn 2^32 - 1 looked at
         // again (the sums are > 0: the largest proportion comes first and the
@@ -1014,7 +1007,7 @@ __global__ void __launch_bounds__(kFilterThreads, 6) sim_filter_kernel(RunArgs a
                             }
                     }
                     const FilterType ty = types[jt];
-                    const float err = cell_err(kc, ty.err);
+                    const float err = filter_cell_err(kc, ty.err);
                     const bool quiescent = ty.mean < 0.0f;
                     const bool live = valid && !quiescent;
                     // first timer (cell.cu:106-122): two candidates from the root

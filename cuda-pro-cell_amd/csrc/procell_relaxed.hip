@@ -1151,7 +1151,7 @@ thread_local hipError_t g_relaxed_hip = hipSuccess;
 // Expected expansions of one walk of a type in a row with this generation
 // cap: its root and, per generation, the nodes whose completion time s lies at
 // most 34.5 beta past t_max (beyond it d < 1e-15).  s_k is taken as normal (as
-// in the plain method's row_cost).  Only used to balance the segments.
+// in the plain method's cost_caps).  Only used to balance the segments.
 double walk_cost(uint32_t kcap, double t_max, double beta, double mean, double sd)
 {
     double e = 1.0;

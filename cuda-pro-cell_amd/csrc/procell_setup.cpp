@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "procell_filter.hpp"
 #include "procell_setup.hpp"
 
 namespace procell {
@@ -110,18 +111,7 @@ static void build_bins(Setup &s)
             }
 }
 
-// row_cost of every row depends on the row through its generation cap alone, so
-// it is evaluated once per cap (1024 rows, 5 types, 11 caps: 0.3 ms
-// of erfc evaluations -> 30 us, needed four times per plan).
-static void cost_caps(Setup &s)
-{
-    s.cap_cost.assign((size_t)s.kmax + 1, -1.0);
-    for (uint32_t r = 0; r < (uint32_t)s.v.size(); ++r) {
-        double &c = s.cap_cost[s.row_info[r] & 0xFFu];
-        if (c < 0.0)
-            c = row_cost(s, r);
-    }
-}
+static void cost_caps(Setup &s);
 
 int build_setup(const procell_params *p, Setup &s, bool want_bins, bool want_costs)
 {
@@ -209,38 +199,155 @@ int build_setup(const procell_params *p, Setup &s, bool want_bins, bool want_cos
     return PROCELL_OK;
 }
 
+static double normal_cdf(double z) { return 0.5 * erfc(-z / sqrt(2.0)); }
+
+// Mean and variance of the completion time D = tau0 (1 + U) + tau_1 + ... +
+// tau_k of a type's division k+1, approximated as normal (truncation ignored).
+static void completion(double m, double sd, int k, double &mu, double &var)
+{
+    mu = 1.5 * m + k * m;
+    var = (7.0 / 3.0) * sd * sd + m * m / 12.0 + k * sd * sd;
+    if (!(var > 0.0))
+        var = 1e-300;
+}
+
 // Lane-steps of one initial cell of a row: its root step (one lane of a
 // full-width step, about what a division costs) plus the expected number of
-// divisions, with division k+1 completing at D = tau0 (1 + U) + tau_1 + ... +
-// tau_k approximated as normal (truncation ignored).  Only used to balance
-// the workgroups' segments; claims and stealing even out its errors.
+// divisions.  Only used to balance the workgroups' segments (claims and
+// stealing even out its errors) and to choose the kernel.  It depends on the
+// row through its generation cap alone, and on the type through prefix sums
+// over the levels, so every completion probability is evaluated once (1024
+// rows, 5 types, 11 caps: 0.3 ms of erfc evaluations by row, 30 us by cap).
 constexpr double kRootCost = 1.0;
-double row_cost(const Setup &s, uint32_t row)
+static void cost_caps(Setup &s)
 {
-    const int kcap = (int)(s.row_info[row] & 0xFFu);
-    double w = kRootCost;
+    s.cap_cost.assign((size_t)s.kmax + 1, kRootCost);
+    s.in_time.assign((size_t)s.n_types * (size_t)s.kmax, 0.0);
     double p_prev = 0.0;
     for (uint32_t j = 0; j < s.n_types; ++j) {
-        const double m = s.type_mean[j];
-        const double sd = fabs(s.type_sd[j]);
-        const double p = s.type_cum[j] - p_prev;
+        const double m = s.type_mean[j], sd = fabs(s.type_sd[j]), p = s.type_cum[j] - p_prev;
         p_prev = s.type_cum[j];
         if (m < 0.0)
             continue;
-        double e = 0.0;
-        for (int k = 0; k < kcap; ++k) {
-            const double mu = 1.5 * m + k * m;
-            const double var = (7.0 / 3.0) * sd * sd + m * m / 12.0 + k * sd * sd;
-            const double z = (s.t_max - mu) / sqrt(var > 0.0 ? var : 1e-300);
-            const double prob = 0.5 * erfc(-z / sqrt(2.0));
-            const double add = ldexp(prob, k);
-            e += add;
-            if (prob < 1e-12)
-                break;
+        double e = 0.0, prob = 1.0;
+        for (int cap = 1; cap <= s.kmax; ++cap) {
+            if (!(prob < 1e-12)) {
+                double mu, var;
+                completion(m, sd, cap - 1, mu, var);
+                prob = normal_cdf((s.t_max - mu) / sqrt(var));
+                s.in_time[(size_t)j * s.kmax + cap - 1] = prob;
+                e += ldexp(prob, cap - 1);
+            }
+            s.cap_cost[cap] += p * e;
         }
-        w += p * e;
     }
-    return w;
+}
+
+// Expected work of a set on the filtered kernel, in lane-steps (normal
+// approximation as in cost_caps).
+struct FilterWork {
+    double divisions = 0.0;
+    double redraws = 0.0;  // steps that draw a refused timer again
+    double unsure = 0.0;   // divisions with a test within the error bound, evaluated again in 64 bits
+    double levels = 0.0;   // divisions, each times its level
+    double chain = 0.0;    // expected longest chain of such evaluations on one lane, in levels
+};
+
+static FilterWork filter_work(const Setup &s)
+{
+    FilterWork f;
+    std::vector<double> cells((size_t)s.kmax + 1, 0.0);  // by generation cap
+    for (size_t r = 0; r < s.v.size(); ++r)
+        cells[s.row_info[r] & 0xFFu] += (double)(s.start[r + 1] - s.start[r]);
+    double p_prev = 0.0;
+    for (uint32_t j = 0; j < s.n_types && !s.v.empty(); ++j) {
+        const double m = s.type_mean[j], sd = fabs(s.type_sd[j]), p = s.type_cum[j] - p_prev;
+        p_prev = s.type_cum[j];
+        if (m < 0.0 || !(p > 0.0))
+            continue;
+        const double refused = sd > 0.0 ? normal_cdf(-m / sd) : 0.0;
+        const double redraws = 2.0 * refused / (1.0 - refused * refused);  // per division; two candidates a block
+        const double terr = filter_type_err(m, sd, s.t_max);
+        const double at0 = sd > 0.0 ? 0.3989422804014327 * exp(-0.5 * (m / sd) * (m / sd)) / sd : 0.0;  // timers' density there
+        // over the levels above a cap: divisions, levels; over its daughters'
+        // levels: density of completion times at t_max, of all and of one per level
+        double e = 0.0, lv = 0.0, dens = 0.0, dens1 = 0.0;
+        for (int cap = 1; cap <= s.kmax; ++cap) {
+            const double prob = s.in_time[(size_t)j * s.kmax + cap - 1];
+            if (prob > 0.0) {
+                e += ldexp(prob, cap - 1);
+                lv += ldexp(prob, cap - 1) * cap;
+                double mu, var;
+                completion(m, sd, cap, mu, var);
+                const double z = (s.t_max - mu) / sqrt(var), d = 0.3989422804014327 * exp(-0.5 * z * z) / sqrt(var);
+                dens += ldexp(d, cap);
+                dens1 += d;
+            }
+            const double n = cells[cap] * p, err = (cap + 4.0) * terr;
+            if (!(n > 0.0) || !(e > 0.0))
+                continue;
+            const double near0 = err < 0.1 * sd ? 2.0 * err * at0
+                                 : sd > 0.0     ? normal_cdf((err - m) / sd) - normal_cdf((-err - m) / sd)
+                                                : (m < err ? 1.0 : 0.0);
+            f.divisions += n * e;
+            f.redraws += n * e * redraws;
+            f.unsure += n * (std::min(1.0, 2.0 * near0) * e + std::min(e, 2.0 * err * dens));
+            f.levels += n * lv;
+            // a cell within the bound of t_max, and the share of its last
+            // daughters that then are
+            const double chain = std::min(1.0, 2.5 * err / (sd * sqrt(lv / e) + 1e-300)) * 0.5 * lv;
+            if (chain > f.chain)
+                f.chain = std::max(f.chain, chain * (1.0 - exp(-2.0 * err * n * dens1)));
+        }
+    }
+    return f;
+}
+
+// A step of a wavefront, in steps of the filtered kernel without any of the
+// following:
+//  * with a lane whose refused timer is drawn again, both kernels take their
+//    longer branch, the filtered one a longer one (the more such lanes);
+//  * an unsure division walks its path from the root again in 64 bits, about
+//    1.8 steps per level, while the wavefront's other lanes wait;
+//  * where a type's timers hardly differ, a cell within the bound of t_max has
+//    many daughters that are, evaluated one after the other on its lane.
+// With fewer than 3 wavefronts of initial cells per SIMD a run is as long as
+// its wavefronts' own instruction streams take, with more the vector units'
+// issue limits it; there the filtered kernel gains more and loses less.
+// Measured, 64-bit against filtered kernel, microseconds per run (two rows of
+// 11 generations; t_max / mean, sd / mean): 3e4 cells at 8.3, 0.3: 172 / 135;
+// 0.4: 202 / 194; 0.45: 217 / 228; 0.6: 221 / 264; 1: 156 / 230; 8.0, 0:
+// 99 / 395; 8.0, 1e-3: 97 / 74; 4e4, 0.25: 802 / 680; 1.6e5, 0.25: 801 / 2091;
+// 1e4, 0.4: 887 / 2403.  3e5 cells at 3.3, 0.4: 46 / 32; 1: 60 / 60; 1.5:
+// 57 / 61.  1024 rows and 1e7 cells of four types, 0.25: 542 / 305; 0.6: 619 /
+// 494; 1: 722 / 683.
+bool filter_pays(const std::vector<Setup> &sets)
+{
+    constexpr double kSimds = 1024.0, kResident = 6.0 * kSimds;  // filtered kernel: wavefronts
+    double cells = 0.0;
+    for (const Setup &s : sets)
+        cells += (double)s.n_cells;
+    const double waves = std::max(1.0, cells / 64.0);
+    const bool few = waves < 3.0 * kSimds;
+    double all = 0.0, filter = 0.0, wide = 0.0, chain = 0.0;
+    for (const Setup &s : sets) {
+        const FilterWork f = filter_work(s);
+        const double steps = f.divisions + f.redraws;
+        if (!(steps > 0.0))
+            continue;
+        const double r = f.redraws / steps, redo = 1.0 - pow(1.0 - r, 64.0);
+        const double unsure = 1.8 * f.levels / f.divisions * (1.0 - pow(1.0 - std::min(1.0, f.unsure / steps), 64.0));
+        filter += steps * (few ? 1.0 + 0.75 * redo + 3.2 * r + unsure : 1.0 + 0.1 * redo + 2.2 * r + unsure);
+        wide += steps * (few ? 1.42 + 0.23 * redo : 1.78);
+        all += steps;
+        chain = std::max(chain, f.chain);
+    }
+    if (!(all > 0.0))
+        return true;
+    // the run in a wavefront's steps: six wavefronts of a SIMD take 2.5 times
+    // as long for one as one alone
+    const double run = all / 64.0 / std::min(waves, kResident) * (few ? 1.0 : 2.5);
+    return !(filter + all * 1.8 * chain / run > wide);
 }
 
 static std::vector<double> row_costs(const Setup &s)

@@ -46,18 +46,21 @@ struct Setup {
     double t_max = 0.0;
     int kmax = 0;
     std::vector<double> bins;       // output bin set, ascending, distinct
-    std::vector<double> cap_cost;   // row_cost by generation cap (-1: no such row)
+    std::vector<double> cap_cost;   // expected lane-steps of a cell, by its row's generation cap
+    std::vector<double> in_time;    // [n_types][kmax] probability that division k+1 of a path completes by t_max
 };
 
 int generation_cap(double v, double phi);
 double resolve_phi(const procell_params *p);
-// want_bins: bins; want_costs: cap_cost (what set_cost, order_rows and
-// split_segments work from).
+// want_bins: bins; want_costs: cap_cost and in_time (what set_cost, order_rows,
+// split_segments and filter_pays work from).
 int build_setup(const procell_params *p, Setup &s, bool want_bins, bool want_costs = true);
 
-// Expected lane-steps of one initial cell of row `row` and of a whole set.
-double row_cost(const Setup &s, uint32_t row);
+// Expected lane-steps of a whole set.
 double set_cost(const Setup &s);
+// Whether a run of these sets takes less time on the filtered kernel than on
+// the 64-bit one, from the shares of its divisions that cost the filter more.
+bool filter_pays(const std::vector<Setup> &sets);
 // The same problem with its rows in order of decreasing cost per cell (file
 // order among equals): values, starts and row_info permuted, file_row[i] the
 // place of the i-th row in s.  Cell starts count the cells in the new order.

@@ -2,6 +2,7 @@
 // (fake_hip.cpp): which device memory, streams and launches the entry points
 // use, and which run their results come from.  usage: host_paths <check>; exit
 // status 0 when it held.
+#include <math.h>
 #include <stdio.h>
 #include <string.h>
 
@@ -111,12 +112,60 @@ static void check_reset()
     CHECK(fake::dead_stream_uses == 0);
 }
 
+// The kernel of a run: the filtered one, unless the sets' times leave what its
+// error bound covers or make it the slower one (each case measured on both).
+static void check_kernel()
+{
+    // two rows of 11 generations, t_max 240; cells, t_max / mean, sd / mean
+    struct {
+        uint64_t cells;
+        double ratio, sd;
+        bool filter;
+    } const cases[] = {
+        {30000, 3.3, 0.2, true},     {30000, 8.3, 0.3, true},    {30000, 50.0, 0.3, true},   {30000, 8.3, 0.45, false},
+        {30000, 50.0, 0.5, false},   {30000, 8.3, 1.0, false},   {30000, 50.0, 3.0, false},  {30000, 5.3, 2.0, false},
+        {300000, 3.3, 0.3, true},    {300000, 3.3, 0.6, true},   {300000, 3.3, 1.5, false},  {300000, 3.3, 2.0, false},
+        {30000, 5e3, 0.25, true},    {30000, 1.6e5, 0.25, false}, {30000, 5e5, 0.25, false}, {30000, 5e6, 0.25, false},
+        {30000, 1e4, 0.4, false},    {30000, 4e4, 0.1, true},    {30000, 1e6, 0.05, false},  {30000, 5e6, 0.0, false},
+        {30000, 8.0, 0.0, false},    {30000, 8.0, 1e-5, false},  {30000, 8.0, 1e-3, true},   {30000, 8.0, 0.03, true},
+        {30000, 50.0, 0.0, true},    {300000, 8.0, 0.0, false},
+    };
+    auto filtered = [] { return fake::launches.back().kernel.find("sim_filter") != std::string::npos; };
+    auto types = [](double ratio, double sd) {
+        const double m = 240.0 / ratio;
+        return std::vector<procell_type>{{0.6, m, sd * m}, {0.4, 1.3 * m, sd * 1.3 * m}};
+    };
+    for (const auto &k : cases) {
+        Case c({{1500.0, k.cells * 2 / 3}, {1050.0, k.cells / 3}}, types(k.ratio, k.sd), 240.0, 1.0);
+        CHECK(procell_simulate(&c.p, &c.r) == PROCELL_OK);
+        CHECK(filtered() == k.filter);
+        if (filtered() != k.filter)
+            fprintf(stderr, "  %llu cells, t_max / mean %g, sd / mean %g\n", (unsigned long long)k.cells, k.ratio, k.sd);
+    }
+    // times outside the bound's range
+    for (double t_max : {0.0, 1e-10, 2e12, (double)INFINITY}) {
+        Case c({{1500.0, 1000}}, {{1.0, 20.0, 4.0}}, t_max, 1.0);
+        CHECK(procell_simulate(&c.p, &c.r) == PROCELL_OK && !filtered());
+    }
+    // a batch: by what its sets cost together
+    for (bool small : {true, false}) {
+        Case a({{1500.0, 200000}}, types(4.0, 0.25), 240.0, 1.0), b({{1500.0, small ? 5u : 20000u}}, types(5e5, 0.25), 240.0, 1.0);
+        std::vector<procell_params> sets(16, a.p);
+        sets[3] = b.p;
+        std::vector<uint64_t> seeds(16, 1);
+        procell_plan *pl = nullptr;
+        CHECK(procell_batch_create(sets.data(), 16, &pl) == PROCELL_OK);
+        CHECK(procell_batch_run(pl, seeds.data()) == PROCELL_OK && filtered() == small);
+        CHECK(procell_plan_destroy(pl) == PROCELL_OK);
+    }
+}
+
 int main(int argc, char **argv)
 {
     const struct {
         const char *name;
         void (*f)();
-    } checks[] = {{"stage", check_stage}, {"noalloc", check_noalloc}, {"reset", check_reset}};
+    } checks[] = {{"stage", check_stage}, {"noalloc", check_noalloc}, {"reset", check_reset}, {"kernel", check_kernel}};
     for (const auto &c : checks)
         if (argc == 2 && !strcmp(argv[1], c.name)) {
             c.f();

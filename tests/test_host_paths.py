@@ -48,3 +48,7 @@ def test_rows_that_fit_the_static_scratch(host_paths):
 
 def test_calls_around_a_device_reset(host_paths):
     host_paths("reset")
+
+
+def test_kernel_of_a_run(host_paths):
+    host_paths("kernel")
