@@ -323,10 +323,6 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     a.rows_in_lds = lds_rows ? 1u : 0u;
     occ = std::min<int>(occ, want);
     ls.block_size = bs;
-    const size_t base = sim_lds_bytes(0, kdim, T, lds_levels, (uint32_t)bs, lds_rows, filter);
-    const size_t budget = std::min(lds_per_cu / (size_t)occ, lds_per_block);
-    const size_t row_bytes = (size_t)kdim * T * 4;
-    uint32_t win_rows = budget > base + 16 ? (uint32_t)((budget - base - 16) / row_bytes) : 0;
 
     // the sets in the order their cells are simulated: the filtered kernel's
     // rows by decreasing cost, so that the runs end with short trees
@@ -335,31 +331,26 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     for (uint32_t i = 0; i < n_sets && filter; ++i)
         ordered[i] = order_rows(pl->setups[i], file_row[i]);
     const std::vector<Setup> &lay = filter ? ordered : pl->setups;
+    std::vector<double> cost(n_sets);  // expected work of each set
+    double all_cost = 0.0;
+    for (uint32_t i = 0; i < n_sets; ++i) {
+        cost[i] = set_cost(lay[i]);
+        all_cost += cost[i];
+    }
 
-    // ---- segments: one per workgroup, each within one set ----
-    // `per_wg` segments per resident workgroup in total, of about equal
-    // expected work: workgroups beyond the resident ones start as others
-    // finish, so the dispatcher balances the segments over the CUs.  In a
-    // batch each set gets segments in proportion to its expected work (at
-    // least one).
-    const uint32_t resident = (uint32_t)((int64_t)n_cu * occ);
-    const uint32_t per_wg = tu.segments   ? std::min<uint32_t>(tu.segments, 64)
-                            : n_sets == 1 ? segments_per_workgroup(set_cost(lay[0]) / resident, filter)
-                                          : kBatchSegmentsPerWorkgroup;
-    std::vector<uint32_t> g_set(n_sets, 1);
-    if (n_sets == 1) {
-        g_set[0] = (uint32_t)std::min<uint64_t>((uint64_t)resident * per_wg,
-                                                std::max<uint64_t>(1, (lay[0].n_cells + 63) / 64));
-    } else {
-        std::vector<double> w(n_sets);
-        double wt = 0.0;
-        for (uint32_t i = 0; i < n_sets; ++i) {
-            w[i] = set_cost(lay[i]);
-            wt += w[i];
+    // u32 window counters must not overflow: bound the leaves any window can
+    // see.  leaves[]: those of the rows before each row, one sum per set (a row
+    // counts for 1e10 at most, which is over the limit by itself and keeps the
+    // differences of the sums exact enough)
+    std::vector<double> leaves;
+    for (uint32_t i = 0; i < n_sets; ++i) {
+        const Setup &s = lay[i];
+        double sum = 0.0;
+        for (size_t r = 0; r < s.v.size(); ++r) {
+            leaves.push_back(sum);
+            sum += std::min(1e10, (double)(s.start[r + 1] - s.start[r]) * ldexp(1.0, (int)(s.row_info[r] & 0xFFu)));
         }
-        const double target = (double)per_wg * (double)resident;
-        for (uint32_t i = 0; i < n_sets; ++i)
-            g_set[i] = wt > 0.0 ? (uint32_t)std::max(1.0, std::floor(w[i] / wt * target + 0.5)) : 1u;
+        leaves.push_back(sum);
     }
     // Segment sizes: a single set's decrease geometrically in launch order
     // (rounds of `resident` segments, each round's segments a factor q
@@ -382,92 +373,156 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
         uint64_t b0, b1;  // cells, relative to the set
         uint32_t row;
     };
-    std::vector<Seg> segs;
-    for (uint32_t i = 0; i < n_sets; ++i) {
-        const Setup &s = lay[i];
-        const uint32_t gi = g_set[i];
-        std::vector<double> wseg(gi, 1.0);
-        if (n_sets == 1 && per_wg > 1 && gi == resident * per_wg) {
-            const double q = pow(filter ? 0.05 : 0.125, 1.0 / (double)(per_wg - 1));
+    // The segments and the window for `occ` resident workgroups per CU.
+    struct Layout {
+        int occ = 0;
+        std::vector<uint64_t> begin, end;  // cells, over all sets
+        std::vector<uint32_t> row, set;
+        uint32_t win_rows = 0;
+        size_t lds_bytes = 0;
+        double load = 0.0;                 // expected lane-steps per resident workgroup
+        double outside = 0.0;              // share of the expected work in rows beyond its segment's window
+    };
+    auto lay_out = [&](int occ, Layout &L) -> int {
+        L = Layout{};
+        L.occ = occ;
+        // ---- segments: one per workgroup, each within one set ----
+        // `per_wg` segments per resident workgroup in total, of about equal
+        // expected work: workgroups beyond the resident ones start as others
+        // finish, so the dispatcher balances the segments over the CUs.  In a
+        // batch each set gets segments in proportion to its expected work (at
+        // least one).
+        const uint32_t resident = (uint32_t)((int64_t)n_cu * occ);
+        const uint32_t per_wg = tu.segments   ? std::min<uint32_t>(tu.segments, 64)
+                                : n_sets == 1 ? segments_per_workgroup(cost[0] / resident, filter)
+                                              : kBatchSegmentsPerWorkgroup;
+        std::vector<uint32_t> g_set(n_sets, 1);
+        if (n_sets == 1) {
+            g_set[0] = (uint32_t)std::min<uint64_t>((uint64_t)resident * per_wg,
+                                                    std::max<uint64_t>(1, (lay[0].n_cells + 63) / 64));
+        } else {
+            const double target = (double)per_wg * (double)resident;
+            for (uint32_t i = 0; i < n_sets; ++i)
+                g_set[i] = all_cost > 0.0 ? (uint32_t)std::max(1.0, std::floor(cost[i] / all_cost * target + 0.5)) : 1u;
+        }
+        std::vector<Seg> segs;
+        for (uint32_t i = 0; i < n_sets; ++i) {
+            const Setup &s = lay[i];
+            const uint32_t gi = g_set[i];
+            std::vector<double> wseg(gi, 1.0);
+            if (n_sets == 1 && per_wg > 1 && gi == resident * per_wg) {
+                const double q = pow(filter ? 0.05 : 0.125, 1.0 / (double)(per_wg - 1));
+                for (uint32_t k = 0; k < gi; ++k) {
+                    const uint32_t slot = (k % resident) / (uint32_t)n_cu;  // 0: oldest on its CU
+                    wseg[k] = pow(q, (double)(k / resident)) * pow(filter ? 1.1 : 1.32, (double)(occ - 1 - (int)slot));
+                }
+            }
+            std::vector<double> cum(gi);
+            double acc = 0.0, tot = 0.0;
+            for (double x : wseg)
+                tot += x;
             for (uint32_t k = 0; k < gi; ++k) {
-                const uint32_t slot = (k % resident) / (uint32_t)n_cu;  // 0: oldest on its CU
-                wseg[k] = pow(q, (double)(k / resident)) * pow(filter ? 1.1 : 1.32, (double)(occ - 1 - (int)slot));
+                acc += wseg[k];
+                cum[k] = k + 1 == gi ? 1.0 : acc / tot;
+            }
+            std::vector<uint64_t> b;
+            std::vector<uint32_t> r;
+            split_segments(s, cum, b, r);
+            for (uint32_t k = 0; k < gi; ++k)
+                segs.push_back(Seg{cost[i] * wseg[k] / tot, i, b[k], b[k + 1], r[k]});
+        }
+        std::stable_sort(segs.begin(), segs.end(), [](const Seg &x, const Seg &y) { return x.cost > y.cost; });
+        for (const Seg &sg : segs) {
+            const SetInfo &si = info[sg.set];
+            L.begin.push_back(si.cell_base + sg.b0);
+            L.end.push_back(si.cell_base + sg.b1);
+            L.row.push_back(si.row_base + sg.row);
+            L.set.push_back(sg.set);
+        }
+        const uint32_t g = (uint32_t)L.row.size();
+        L.load = all_cost / resident;
+        // no more window rows than a segment spans
+        const size_t base = sim_lds_bytes(0, kdim, T, lds_levels, (uint32_t)bs, lds_rows, filter);
+        const size_t budget = std::min(lds_per_cu / (size_t)occ, lds_per_block);
+        const size_t row_bytes = (size_t)kdim * T * 4;
+        L.win_rows = budget > base + 16 ? (uint32_t)((budget - base - 16) / row_bytes) : 0;
+        uint32_t span = 1;
+        std::vector<uint32_t> last(g, 0);  // rows, relative to the set
+        for (uint32_t k = 0; k < g; ++k) {
+            const Setup &s = lay[L.set[k]];
+            const SetInfo &si = info[L.set[k]];
+            if (!s.n_cells)
+                continue;
+            const uint64_t first = L.begin[k] - si.cell_base;
+            const uint64_t end = L.end[k] - si.cell_base;
+            const uint64_t lc = end > first ? end - 1 : first;
+            const uint64_t lcc = lc < s.n_cells ? lc : s.n_cells - 1;
+            last[k] = (uint32_t)(std::upper_bound(s.start.begin(), s.start.end() - 1, lcc) - s.start.begin()) - 1;
+            span = std::max(span, last[k] - (L.row[k] - si.row_base) + 1);
+        }
+        L.win_rows = std::min(L.win_rows, span);
+        for (uint32_t k = 0; k < g && L.win_rows; ++k) {
+            const uint32_t nr = (uint32_t)lay[L.set[k]].v.size();
+            const uint32_t r0 = L.row[k] - info[L.set[k]].row_base;
+            const double *before = &leaves[info[L.set[k]].row_base + L.set[k]];
+            if (before[std::min<uint32_t>(nr, r0 + L.win_rows)] - before[std::min(nr, r0)] >= 4.0e9)
+                L.win_rows = 0;
+        }
+        // the window must not cost a resident workgroup (LDS allocation granularity)
+        for (;;) {
+            L.lds_bytes = sim_lds_bytes(L.win_rows, kdim, T, lds_levels, (uint32_t)bs, lds_rows, filter);
+            int occ_w = 0;
+            if (sim_occupancy(bs, L.lds_bytes, lds_rows != 0, kdim, gstack, filter, &occ_w) != hipSuccess)
+                return PROCELL_E_HIP;
+            // keep a margin for the per-workgroup LDS allocation granularity
+            const bool fits = (size_t)occ * align_up(L.lds_bytes, 2048) <= lds_per_cu;
+            if ((occ_w >= occ && fits) || L.win_rows == 0)
+                break;
+            L.win_rows -= std::max(1u, L.win_rows / 8);
+        }
+        for (uint32_t k = 0; k < g && L.win_rows < span && all_cost > 0.0; ++k) {
+            const Setup &s = lay[L.set[k]];
+            const SetInfo &si = info[L.set[k]];
+            for (uint32_t r = L.row[k] - si.row_base + L.win_rows; r <= last[k] && r < (uint32_t)s.v.size(); ++r) {
+                const uint64_t b = std::max(s.start[r], L.begin[k] - si.cell_base), e = std::min(s.start[r + 1], L.end[k] - si.cell_base);
+                L.outside += e > b ? s.cap_cost[s.row_info[r] & 0xFFu] * (double)(e - b) / all_cost : 0.0;
             }
         }
-        std::vector<double> cum(gi);
-        double acc = 0.0, tot = 0.0;
-        for (double x : wseg)
-            tot += x;
-        for (uint32_t k = 0; k < gi; ++k) {
-            acc += wseg[k];
-            cum[k] = k + 1 == gi ? 1.0 : acc / tot;
+        return PROCELL_OK;
+    };
+    // Tallies of rows beyond the window are device atomics, which cost up to
+    // several times the run's other work, the more of it there is.  A workgroup
+    // less per CU leaves the others more LDS; it costs some 12 % of a run, two
+    // some 30 %, and a wider window takes longer to clear and flush.  5 types,
+    // 14 generations, microseconds per run with 3 / 2 / 1 workgroups per CU
+    // (64-bit kernel): 6000 rows and 1e7 cells 1188 / 187 / 197 (306), 1e5 rows
+    // 816 / 401 / 303 (756), with 1e6 cells 120 / 71 / 89 (120); 2 types: 25,000
+    // rows and 1e7 cells 734 / 290 / 299 (500), with 1e5 29 / 32 / 39 (39); 2
+    // types, 11 generations, 1e5 rows and 1e7 cells (3 % outside) 264 / 277 /
+    // 279 (689).  Runs below 2000 lane-steps per workgroup are mostly their
+    // start and end.
+    Layout L;
+    if (const int rc = lay_out(occ, L); rc != PROCELL_OK)
+        return fail(rc);
+    if (filter && !tu.blocks_per_cu && L.outside > 0.02 && L.load >= 2000.0) {
+        auto price = [&](const Layout &l) {
+            const double d = occ - l.occ;
+            return (1.0 + 1.2 * log10(l.load / 600.0) * l.outside) * (1.0 + 0.12 * d + 0.03 * d * (d - 1.0)) +
+                   (l.occ > 1 ? 0.3 : 0.7) * (double)l.win_rows * kdim * T / l.load;
+        };
+        for (int o = occ - 1; o >= 1; --o) {
+            Layout less;
+            if (const int rc = lay_out(o, less); rc != PROCELL_OK)
+                return fail(rc);
+            if (price(less) < price(L))
+                L = std::move(less);
         }
-        std::vector<uint64_t> b;
-        std::vector<uint32_t> r;
-        split_segments(s, cum, b, r);
-        const double sc = set_cost(s);
-        for (uint32_t k = 0; k < gi; ++k)
-            segs.push_back(Seg{sc * wseg[k] / tot, i, b[k], b[k + 1], r[k]});
     }
-    std::stable_sort(segs.begin(), segs.end(), [](const Seg &x, const Seg &y) { return x.cost > y.cost; });
-    std::vector<uint64_t> seg_begin, seg_end;
-    std::vector<uint32_t> seg_row, seg_set;
-    for (const Seg &sg : segs) {
-        const SetInfo &si = info[sg.set];
-        seg_begin.push_back(si.cell_base + sg.b0);
-        seg_end.push_back(si.cell_base + sg.b1);
-        seg_row.push_back(si.row_base + sg.row);
-        seg_set.push_back(sg.set);
-    }
-    const uint32_t g = (uint32_t)seg_row.size();
-    // no more window rows than a segment spans
-    uint32_t span = 1;
-    for (uint32_t k = 0; k < g; ++k) {
-        const Setup &s = lay[seg_set[k]];
-        const SetInfo &si = info[seg_set[k]];
-        if (!s.n_cells)
-            continue;
-        const uint64_t first = seg_begin[k] - si.cell_base;
-        const uint64_t end = seg_end[k] - si.cell_base;
-        const uint64_t lc = end > first ? end - 1 : first;
-        const uint64_t lcc = lc < s.n_cells ? lc : s.n_cells - 1;
-        const uint32_t lr = (uint32_t)(std::upper_bound(s.start.begin(), s.start.end() - 1, lcc) - s.start.begin()) - 1;
-        span = std::max(span, lr - (seg_row[k] - si.row_base) + 1);
-    }
-    win_rows = std::min(win_rows, span);
-    // u32 window counters must not overflow: bound the leaves any window can
-    // see.  leaves[]: those of the rows before each row, one sum per set (a row
-    // counts for 1e10 at most, which is over the limit by itself and keeps the
-    // differences of the sums exact enough)
-    std::vector<double> leaves;
-    for (uint32_t i = 0; i < n_sets; ++i) {
-        const Setup &s = lay[i];
-        double sum = 0.0;
-        for (size_t r = 0; r < s.v.size(); ++r) {
-            leaves.push_back(sum);
-            sum += std::min(1e10, (double)(s.start[r + 1] - s.start[r]) * ldexp(1.0, (int)(s.row_info[r] & 0xFFu)));
-        }
-        leaves.push_back(sum);
-    }
-    for (uint32_t k = 0; k < g && win_rows; ++k) {
-        const uint32_t nr = (uint32_t)lay[seg_set[k]].v.size();
-        const uint32_t r0 = seg_row[k] - info[seg_set[k]].row_base;
-        const double *before = &leaves[info[seg_set[k]].row_base + seg_set[k]];
-        if (before[std::min<uint32_t>(nr, r0 + win_rows)] - before[std::min(nr, r0)] >= 4.0e9)
-            win_rows = 0;
-    }
-    // the window must not cost a resident workgroup (LDS allocation granularity)
-    for (;;) {
-        ls.lds_bytes = sim_lds_bytes(win_rows, kdim, T, lds_levels, (uint32_t)bs, lds_rows, filter);
-        int occ_w = 0;
-        if (sim_occupancy(bs, ls.lds_bytes, lds_rows != 0, kdim, gstack, filter, &occ_w) != hipSuccess)
-            return fail(PROCELL_E_HIP);
-        // keep a margin for the per-workgroup LDS allocation granularity
-        const bool fits = (size_t)occ * align_up(ls.lds_bytes, 2048) <= lds_per_cu;
-        if ((occ_w >= occ && fits) || win_rows == 0)
-            break;
-        win_rows = win_rows > 8 ? win_rows - win_rows / 8 : 0;
-    }
+    const uint32_t g = (uint32_t)L.row.size();
+    const uint32_t win_rows = L.win_rows;
+    ls.lds_bytes = L.lds_bytes;
+    const std::vector<uint64_t> &seg_begin = L.begin, &seg_end = L.end;
+    const std::vector<uint32_t> &seg_row = L.row, &seg_set = L.set;
     ls.blocks = (int)g;
     a.win_rows = win_rows;
     a.idle_limit = tu.idle_lanes ? std::min<uint32_t>(tu.idle_lanes, 63) : 12;

@@ -160,12 +160,43 @@ static void check_kernel()
     }
 }
 
+// The tally window: rows of many generations and types, of which three
+// workgroups of 512 per CU leave no room for as many as a segment spans, get
+// fewer workgroups per CU; the others keep three.
+static void check_window()
+{
+    const std::vector<procell_type> five{{0.2, 35, 9}, {0.2, 55, 14}, {0.2, 75, 19}, {0.2, 95, 24}, {0.2, -1, -1}};
+    const std::vector<procell_type> two{{0.5, 35, 9}, {0.5, 95, 24}};
+    struct {
+        const std::vector<procell_type> &types;
+        double top, phi;  // values from 1 to top
+        uint32_t rows;
+        double cells;
+        uint32_t per_cu, window;  // workgroups; least rows
+    } const cases[] = {
+        {five, 1e5, 50.0, 1024, 1e7, 3, 4},  {five, 1e4, 1.0, 1500, 1e6, 3, 3},  {five, 1e4, 1.0, 6000, 1e7, 2, 10},
+        {five, 1e4, 1.0, 100000, 1e7, 1, 100}, {two, 1e4, 1.0, 100, 1e6, 3, 2},  {two, 1e4, 1.0, 25000, 1e7, 2, 50},
+        {two, 1e4, 1.0, 25000, 1e5, 3, 10},  {two, 1e3, 1.0, 25000, 1e7, 3, 20},
+    };
+    for (const auto &k : cases) {
+        std::vector<procell_row> rows(k.rows);
+        for (uint32_t i = 0; i < k.rows; ++i)
+            rows[i] = {pow(k.top, (double)i / (k.rows - 1)), (uint64_t)(k.cells / k.rows)};
+        Case c(rows, k.types, 168.0, k.phi);
+        CHECK(procell_simulate(&c.p, &c.r) == PROCELL_OK);
+        const uint32_t per_cu = (uint32_t)(163840 / c.r.stats.lds_bytes);
+        CHECK((per_cu > 3 ? 3 : per_cu) == k.per_cu && c.r.stats.window_rows >= k.window);
+        printf("%u types to %g, %u rows, %g cells: %u per CU, %u window rows\n", c.p.n_types, k.top, k.rows, k.cells,
+               per_cu, c.r.stats.window_rows);
+    }
+}
+
 int main(int argc, char **argv)
 {
     const struct {
         const char *name;
         void (*f)();
-    } checks[] = {{"stage", check_stage}, {"noalloc", check_noalloc}, {"reset", check_reset}, {"kernel", check_kernel}};
+    } checks[] = {{"stage", check_stage}, {"noalloc", check_noalloc}, {"reset", check_reset}, {"kernel", check_kernel}, {"window", check_window}};
     for (const auto &c : checks)
         if (argc == 2 && !strcmp(argv[1], c.name)) {
             c.f();

@@ -52,3 +52,7 @@ def test_calls_around_a_device_reset(host_paths):
 
 def test_kernel_of_a_run(host_paths):
     host_paths("kernel")
+
+
+def test_tally_window_of_deep_rows(host_paths):
+    host_paths("window")
