@@ -45,6 +45,7 @@ struct procell_plan {
     std::vector<Setup> setups;         // per set
     std::vector<size_t> tally_base, tally_len;  // per set, in tally entries
     LaunchShape shape{};
+    int per_cu = 0;  // resident workgroups per CU that the layout is for
     RunArgs args{};
     void *d_block = nullptr;  // one allocation holding every table
     bool own_block = true;    // false: d_block is the static scratch array
@@ -524,6 +525,7 @@ int create_plan(const procell_params *ps, uint32_t n_sets, procell_plan **out, v
     const std::vector<uint64_t> &seg_begin = L.begin, &seg_end = L.end;
     const std::vector<uint32_t> &seg_row = L.row, &seg_set = L.set;
     ls.blocks = (int)g;
+    pl->per_cu = L.occ;
     a.win_rows = win_rows;
     a.idle_limit = tu.idle_lanes ? std::min<uint32_t>(tu.idle_lanes, 63) : 12;
 
@@ -1066,7 +1068,8 @@ int procell_plan_autotune(procell_plan *plan, const uint64_t *seeds, uint32_t re
     HIP_TRY(hipSetDevice(plan->device));
     // layouts: resident workgroups per CU (sets the LDS tally window's
     // width) x segments per resident workgroup; for each, the idle-lane
-    // threshold, which needs no new layout
+    // threshold, which needs no new layout.  More workgroups than a CU holds
+    // are the layout of as many as it holds: timed once, and reported as that.
     static const uint32_t kBlocks[] = {2, 3, 4};
     static const uint32_t kSegments[] = {1, 2, 3, 4, 8};
     static const uint32_t kIdle[] = {6, 8, 12, 16};
@@ -1081,8 +1084,9 @@ int procell_plan_autotune(procell_plan *plan, const uint64_t *seeds, uint32_t re
     float best = -1.f;
     procell_plan *best_plan = nullptr;
     procell_tuning best_tu{};
-    int rc = PROCELL_OK;
+    int rc = PROCELL_OK, per_cu = 0;
     for (uint32_t bpc : kBlocks) {
+        const int timed = per_cu;  // workgroups per CU of the layouts before
         for (uint32_t seg : kSegments) {
             for (procell_params &p : ps) {
                 p.tuning.blocks_per_cu = bpc;
@@ -1096,6 +1100,11 @@ int procell_plan_autotune(procell_plan *plan, const uint64_t *seeds, uint32_t re
             if (rc != PROCELL_OK)
                 break;
             cand->own_stream = false;
+            per_cu = cand->per_cu;
+            if (per_cu == timed) {
+                destroy_plan(cand);
+                break;
+            }
             bool kept = false;
             for (uint32_t idle : kIdle) {
                 cand->args.idle_limit = idle;
@@ -1106,6 +1115,7 @@ int procell_plan_autotune(procell_plan *plan, const uint64_t *seeds, uint32_t re
                 if (best < 0.f || ms < best) {
                     best = ms;
                     best_tu = ps[0].tuning;
+                    best_tu.blocks_per_cu = (uint32_t)per_cu;
                     best_tu.idle_lanes = idle;
                     if (best_plan && best_plan != cand)
                         destroy_plan(best_plan);
@@ -1134,6 +1144,7 @@ int procell_plan_autotune(procell_plan *plan, const uint64_t *seeds, uint32_t re
     // and timing ring stay
     drop_graph(plan);
     std::swap(plan->shape, best_plan->shape);
+    std::swap(plan->per_cu, best_plan->per_cu);
     std::swap(plan->args, best_plan->args);
     std::swap(plan->d_block, best_plan->d_block);
     std::swap(plan->tally_total, best_plan->tally_total);

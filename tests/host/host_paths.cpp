@@ -6,6 +6,9 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
+#include <map>
+
 #include "fake_hip.hpp"
 #include "procell.h"
 
@@ -191,12 +194,43 @@ static void check_window()
     }
 }
 
+// The autotuner times no layout twice and reports the workgroups per CU that
+// the plan runs with, also where later candidates are the faster ones.
+static float g_ms = 100.0f;
+static void check_autotune()
+{
+    fake::elapsed_ms = [] { return g_ms -= 0.5f; };
+    for (double top : {1e5, 1e15}) {  // the second: trees so deep that a CU holds one or two workgroups
+        std::vector<procell_row> rows(1024);
+        for (int i = 0; i < 1024; ++i)
+            rows[i] = {pow(top, i / 1023.0), 9765};
+        Case c(rows, {{0.4, 35, 9}, {0.3, 55, 14}, {0.3, -1, -1}}, 240.0, 50.0);
+        procell_plan *pl = nullptr;
+        CHECK(procell_plan_create(&c.p, &pl) == PROCELL_OK);
+        fake::launches.clear();
+        const uint64_t seed = 1;
+        procell_tuning t{};
+        CHECK(procell_plan_autotune(pl, &seed, 1, &t) == PROCELL_OK);
+        std::map<std::pair<unsigned, size_t>, int> runs;  // of each layout: four idle-lane thresholds, a warm-up and a run each
+        for (const fake::Launch &l : fake::launches)
+            if (l.kernel.find("sim_") != std::string::npos)
+                ++runs[{l.grid, l.lds}];
+        for (const auto &r : runs)
+            CHECK(r.second == 8);
+        CHECK(procell_plan_run(pl, 1) == PROCELL_OK && procell_plan_result(pl, &c.r) == PROCELL_OK);
+        const uint32_t fit = std::min<uint32_t>(24 * 64 / c.r.stats.block_size, (uint32_t)(163840 / c.r.stats.lds_bytes));
+        CHECK(t.blocks_per_cu >= 1 && t.blocks_per_cu <= fit);
+        CHECK(procell_plan_destroy(pl) == PROCELL_OK);
+    }
+}
+
 int main(int argc, char **argv)
 {
     const struct {
         const char *name;
         void (*f)();
-    } checks[] = {{"stage", check_stage}, {"noalloc", check_noalloc}, {"reset", check_reset}, {"kernel", check_kernel}, {"window", check_window}};
+    } checks[] = {{"stage", check_stage}, {"noalloc", check_noalloc}, {"reset", check_reset}, {"kernel", check_kernel}, {"window", check_window},
+                  {"autotune", check_autotune}};
     for (const auto &c : checks)
         if (argc == 2 && !strcmp(argv[1], c.name)) {
             c.f();

@@ -56,3 +56,7 @@ def test_kernel_of_a_run(host_paths):
 
 def test_tally_window_of_deep_rows(host_paths):
     host_paths("window")
+
+
+def test_autotuner_times_each_layout_once(host_paths):
+    host_paths("autotune")
