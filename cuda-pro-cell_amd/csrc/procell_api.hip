@@ -1274,4 +1274,28 @@ int procell_debug_draws(int32_t device, uint64_t seed, const uint64_t *cell, con
     return PROCELL_OK;
 }
 
+// For tests, not part of the C ABI: bounds[4] as launch_pair_bounds.
+int procell_debug_pair_bounds(int32_t device, double *bounds)
+{
+    if (!bounds)
+        return PROCELL_E_INVALID;
+    int n_cu = 0;
+    const int rc = check_device(device, &n_cu);
+    if (rc != PROCELL_OK)
+        return rc;
+    void *d = nullptr;
+    if (hipMalloc(&d, 4 * sizeof(double)) != hipSuccess)
+        return PROCELL_E_OUT_OF_MEMORY;
+    hipError_t e = launch_zero((unsigned long long *)d, 4, nullptr);
+    if (e == hipSuccess) e = launch_pair_bounds((unsigned long long *)d, nullptr);
+    if (e == hipSuccess) e = hipDeviceSynchronize();
+    if (e == hipSuccess) e = hipMemcpy(bounds, d, 4 * sizeof(double), hipMemcpyDeviceToHost);
+    (void)hipFree(d);
+    if (e != hipSuccess) {
+        g_last_hip = e;
+        return PROCELL_E_HIP;
+    }
+    return PROCELL_OK;
+}
+
 }  // extern "C"

@@ -114,6 +114,8 @@ hipError_t launch_sim(const RunArgs &a, const LaunchShape &ls, hipStream_t st);
 hipError_t launch_debug_draws(uint64_t seed, const uint64_t *cell, const uint64_t *node,
                               const uint32_t *attempt, uint64_t n, uint32_t *words, double *z,
                               hipStream_t st);
+// Worst errors of the single-precision pair (bits of doubles >= 0; out[4] cleared before).
+hipError_t launch_pair_bounds(unsigned long long *out, hipStream_t st);
 hipError_t sim_occupancy(int block_size, size_t lds_bytes, bool rows_in_lds, uint32_t kdim, bool gstack, bool filter,
                          int *blocks_per_cu);
 

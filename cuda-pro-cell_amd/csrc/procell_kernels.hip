@@ -669,7 +669,7 @@ __global__ void __launch_bounds__(256, 4) sim_kernel(RunArgs a)
 // normal_pair_f32 is within 5.6e-6 of the 64-bit pair.  Measured on gfx950
 // over all 2^32 values of each word: the radius is off by at most 5.42e-6 (next to u1 = 1, where it
 // is below 0.01) and 3.64e-6 for u1 <= 1/2, sine and cosine by 2.7e-7 (times
-// a radius of at most 4.71).  kPairErr allows 7e-6.  A timer fma(z, sd, mean)
+// a radius of at most 4.71); pair_bounds_kernel repeats it.  kPairErr allows 7e-6.  A timer fma(z, sd, mean)
 // adds the rounding of sd, mean and itself: at most 2^-23 (|mean| + 8.6 |sd|);
 // a completion time adds 2^-24 t_max per addition (times are kept relative to
 // t_max, so a value near the threshold is small, and no partial sum of a path
@@ -682,13 +682,26 @@ constexpr uint32_t kPairLow = 1u << 16;
 
 __device__ __forceinline__ bool pair_sure(uint32_t w0) { return w0 - kPairLow < 0u - 2u * kPairLow; }
 
-__device__ __forceinline__ void normal_pair_f32(uint32_t w0, uint32_t w2, float &z0, float &z1)
+__device__ __forceinline__ float radius_f32(uint32_t w0)
 {
     const float u1 = (float)w0 * 0x1p-32f;
-    const float rho = __builtin_amdgcn_sqrtf(__builtin_amdgcn_logf(u1) * -1.3862943611198906f);  // -2 ln 2
+    return __builtin_amdgcn_sqrtf(__builtin_amdgcn_logf(u1) * -1.3862943611198906f);  // -2 ln 2
+}
+
+__device__ __forceinline__ void turn_f32(uint32_t w2, float &cs, float &sn)
+{
     const float turn = (float)w2 * 0x1p-32f;
-    z0 = rho * __builtin_amdgcn_cosf(turn);
-    z1 = rho * __builtin_amdgcn_sinf(turn);
+    cs = __builtin_amdgcn_cosf(turn);
+    sn = __builtin_amdgcn_sinf(turn);
+}
+
+__device__ __forceinline__ void normal_pair_f32(uint32_t w0, uint32_t w2, float &z0, float &z1)
+{
+    const float rho = radius_f32(w0);
+    float cs, sn;
+    turn_f32(w2, cs, sn);
+    z0 = rho * cs;
+    z1 = rho * sn;
 }
 
 // Smaller of two magnitudes.
@@ -1314,7 +1327,49 @@ __global__ void debug_draws_kernel(uint64_t seed, const uint64_t *cell, const ui
     z[2 * i + 1] = z1;
 }
 
+// The errors behind kPairErr, over all values of a block's words: word 0 with
+// the least and the largest word 1 and word 2 with the least and the largest
+// word 3 (the 64-bit radius and angle are monotone in them).  First pass
+// (pairs 0): sine and cosine; second: the radius, and with the first pass's
+// result a candidate: the radius' error, its sine's, and the rounding of their
+// product.  out: the radius, the radius where the uniform is at most 1/2, sine
+// and cosine, a candidate; as bits of doubles >= 0, which order like integers.
+__global__ void pair_bounds_kernel(uint32_t pairs, unsigned long long *out)
+{
+    const dev::Tables tb = dev::global_tables();
+    constexpr dev::Coeffs K = dev::coeffs();
+    const double sc_err = __builtin_bit_cast(double, (uint64_t)out[2]);
+    double worst[4] = {0.0, 0.0, 0.0, 0.0};
+    const uint32_t stride = gridDim.x * blockDim.x, tid = blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint64_t w = tid; w < 1ull << 32; w += stride)
+        for (uint32_t lo : {0u, 0xFFFFFFFFu}) {
+            if (!pairs) {
+                float cs, sn;
+                turn_f32((uint32_t)w, cs, sn);
+                double c64, s64;
+                dev::sincos_turns((uint32_t)w, lo, s64, c64, K, tb);
+                worst[2] = fmax(worst[2], fmax(fabs(cs - c64), fabs(sn - s64)));
+            } else if (pair_sure((uint32_t)w)) {
+                const double rho = dev::sqrt_nonneg(-2.0 * dev::log_pos(dev::uniform_oc((uint32_t)w, lo), K, tb));
+                const double e = fabs(radius_f32((uint32_t)w) - rho);
+                worst[0] = fmax(worst[0], e);
+                worst[1] = fmax(worst[1], w < 0x80000000u ? e : 0.0);
+                worst[3] = fmax(worst[3], e * (1.0 + sc_err) + rho * sc_err + 0x1p-24 * (rho + e));
+            }
+        }
+    for (int i = 0; i < 4; ++i)
+        if (worst[i] > 0.0)
+            atomicMax(&out[i], (unsigned long long)__builtin_bit_cast(uint64_t, worst[i]));
+}
+
 }  // namespace
+
+hipError_t launch_pair_bounds(unsigned long long *out, hipStream_t st)
+{
+    hipLaunchKernelGGL(pair_bounds_kernel, dim3(4096), dim3(256), 0, st, 0u, out);
+    hipLaunchKernelGGL(pair_bounds_kernel, dim3(4096), dim3(256), 0, st, 1u, out);
+    return hipGetLastError();
+}
 
 size_t sim_lds_bytes(uint32_t win_rows, uint32_t kdim, uint32_t n_types, uint32_t stack_levels, uint32_t block_size,
                      uint32_t lds_rows, bool filter)
