@@ -54,7 +54,7 @@ struct procell_plan {
     uint64_t *d_seeds = nullptr;       // [n_sets] seeds of the current batch run (in d_block)
     uint64_t *h_seeds = nullptr;       // pinned [kSeedSlots][n_sets]
     hipEvent_t seed_ev[kSeedSlots] = {};
-    hipGraph_t graph = nullptr;        // batch runs: clearing, root and tree kernels
+    hipGraph_t graph = nullptr;        // batch runs: clearing and simulation kernels
     hipGraphExec_t graph_exec = nullptr;
     std::vector<hipEvent_t> kev;   // PROCELL_FLAG_TIMING: start/stop of each run's kernels (ring)
     uint64_t runs = 0;             // runs since the last kernel-time read
@@ -149,7 +149,8 @@ void destroy_plan(procell_plan *pl)
 // Whether the filtered kernel's error bounds cover these sets: times, means
 // and standard deviations of magnitudes that single precision holds with
 // their products and the differences of their 64-bit values (t_max 0 or
-// infinite, or beyond these ranges, goes to the 64-bit kernel).
+// infinite, or beyond these ranges, goes to the 64-bit kernel).  Whether it
+// is the faster kernel is filter_pays' matter.
 bool filter_covers(const std::vector<Setup> &sets)
 {
     for (const Setup &s : sets) {
@@ -671,7 +672,7 @@ hipError_t launch_run(procell_plan *pl)
     return e;
 }
 
-// Batch runs replay one graph of the three kernels; it is captured on the
+// Batch runs replay one graph of the two kernels; it is captured on the
 // first run (the kernels read the seeds from device memory, so the graph
 // does not change between runs) and again after the launch knobs change.
 int capture_graph(procell_plan *pl)

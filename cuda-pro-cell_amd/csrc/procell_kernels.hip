@@ -659,18 +659,19 @@ __global__ void __launch_bounds__(256, 4) sim_kernel(RunArgs a)
 //
 // Why: the 64-bit Box-Muller pair is 87 of a division step's 180 vector
 // instructions at 4 cycles each; the hardware's log2, sqrt, sin and cos take
-// 8 cycles each and single-precision multiplies and adds 2.  Five-type
+// 8 cycles each and single-precision multiplies and adds 2 to 3.  Five-type
 // histogram, 1024 bins: 0.219 -> 0.143 ms per run at 1e7 cells, 2.05 -> 1.10
 // ms at 1e8 (2.58e8 divisions: 1.26e11 -> 2.35e11 per second; vector
 // instructions per division 4.56 -> 2.70).
 //
 // The bound.  For a block whose first word w0 lies in [2^16, 2^32 - 2^16)
 // (pair_sure; the others, 1 in 2^15, are evaluated in 64 bits)
-// normal_pair_f32 is within 5.6e-6 of the 64-bit pair.  Measured on gfx950
-// over all 2^32 values of each word: the radius is off by at most 5.42e-6 (next to u1 = 1, where it
-// is below 0.01) and 3.64e-6 for u1 <= 1/2, sine and cosine by 2.7e-7 (times
-// a radius of at most 4.71); pair_bounds_kernel repeats it.  kPairErr allows 7e-6.  A timer fma(z, sd, mean)
-// adds the rounding of sd, mean and itself: at most 2^-23 (|mean| + 8.6 |sd|);
+// normal_pair_f32 is within 5.42e-6 of the 64-bit pair.  Measured on gfx950
+// over all 2^32 values of each word (pair_bounds_kernel repeats it): the
+// radius is off by at most 5.42e-6 (next to u1 = 1, where it is below 0.01)
+// and 3.64e-6 for u1 <= 1/2, sine and cosine by 2.7e-7 (times a radius of at
+// most 4.71).  kPairErr allows 7e-6.  A timer fma(z, sd, mean) adds the
+// rounding of sd, mean and itself: at most 2^-23 (|mean| + 8.6 |sd|);
 // a completion time adds 2^-24 t_max per addition (times are kept relative to
 // t_max, so a value near the threshold is small, and no partial sum of a path
 // exceeds t_max) and 3.5 of those for t_max and the root's phase.  After k
@@ -786,13 +787,15 @@ __device__ __forceinline__ ExactTimes exact_times(uint64_t seed, uint32_t cell, 
 // sim_filter_kernel: the same run as sim_kernel (segments, claims, root
 // steps, hand-outs and division steps as there), with the two tests on times
 // filtered as described above; it runs every plan whose times the bound
-// covers (the host's filter_covers).  What bounds it is the vector unit's
-// issue rate (4 cycles per SIMD for nearly every instruction; 0.95 per CU and
-// clock at 1e8 cells) and, with fewer instructions per step than sim_kernel,
-// the latency of a wavefront's own instruction stream: 6 wavefronts per SIMD
-// instead of 4 gave 1.24 -> 1.09 ms, which holds it to 80 registers (the
-// 64-bit evaluation spills a few, in its own branch only).  The tree logic is
-// arranged for few instructions and few values carried round the loop:
+// covers (the host's filter_covers) and which it does not slow down
+// (filter_pays).  What bounds it is the vector unit's issue rate (1.04
+// instructions per CU and clock at 1e8 cells; most take 4 cycles of a SIMD,
+// additions, logic, moves and single-precision arithmetic on vector registers
+// 2 to 3) and, with fewer instructions per step than sim_kernel, the latency
+// of a wavefront's own instruction stream: 6 wavefronts per SIMD instead of 4
+// gave 1.24 -> 1.09 ms, which holds it to 80 registers (the 64-bit evaluation
+// spills a few, in its own branch only).  The tree logic is arranged for few
+// instructions and few values carried round the loop:
 //  * a set's rows come in order of decreasing cost (the host's order_rows), so
 //    the last trees of a segment, and of the run, are its shallowest: 0.143 ->
 //    0.136 ms at 1e7 cells.

@@ -416,8 +416,8 @@ __device__ __forceinline__ P *again(P *p)
 //  * the window is kept in up to 8 copies where it is small: the adds of 64
 //    lanes meet in some 30 entries (Jacobian pass of 64 sets 2.58 -> 2.31 ms).
 //  * the quiescent types' records are written here too and everything is
-//    cleared in one launch: four launches per pass became two (5000 cells: 20
-//    -> 14 us).
+//    cleared in one launch: four launches per pass became two (forward
+//    pass of one cell 23 -> 16 us).
 //  * where all segments run at once, the hardware prefers the older of a
 //    SIMD's wavefronts, so that the youngest ends alone, at a third of the
 //    rate; a wavefront of a segment with more left to claim takes a higher
