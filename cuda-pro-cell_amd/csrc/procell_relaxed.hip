@@ -95,6 +95,11 @@ constexpr uint32_t kMinWalks = 256;
 // cells 18.5 (8), 20.6 (16).
 constexpr uint32_t kMultiSetFactor = 8;
 
+// Device memory of a plan's lane stacks at most: a plan of more segments
+// (every set has one; at 14 generations 50,000 fit) runs a pass as several
+// launches, one after the other, over the same stacks.
+constexpr size_t kStackBytes = 8ull << 30;
+
 // Copies of a call's counters, one 128-byte line each; workgroup b adds to copy
 // b mod 64.  One copy for all wavefronts: at 1e6 shallow walks their adds to
 // one address came within 10 us and held up every CU's memory accesses for 30
@@ -128,6 +133,8 @@ struct RelaxArgs {
     uint32_t kdim_max;         // most generations + 1 of any set
     uint32_t even_ends;        // nonzero: every segment is resident at once
     uint32_t win_doubles[3];   // LDS window of a workgroup, per WalkMode
+    uint32_t n_segments;
+    uint32_t seg_first;        // first segment of a launch
     const RelaxSet *sets;
     const uint32_t *seg_set;   // [segments] set of each segment
     const uint32_t *seg_cell;  // [segments][2] first and end initial cell (set-local)
@@ -138,7 +145,7 @@ struct RelaxArgs {
     const uint32_t *prolif;    // file index of each proliferating type, per set
     const uint32_t *quiet;     // file index of each quiescent type, per set
     const double *theta;       // per set [3][n_types]: mean, sd, proportion, file order
-    double *stack;             // per segment and wavefront [kdim_max + 1 levels][64 lanes] frames
+    double *stack;             // per workgroup of a launch and wavefront [kdim_max + 1 levels][64 lanes] frames
     double *h;                 // per set [rows][kdim][n_types] relaxed tally (forward)
     const double *g;           // cotangent, layout of h (backward)
     double *grad;              // per set [3][n_types] gradient (backward)
@@ -433,7 +440,7 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
     using Frame = WalkFrame<Tan>;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = uni(tid >> 6);
-    const uint32_t seg = blockIdx.x;
+    const uint32_t seg = args.seg_first + blockIdx.x;
     const uint32_t set_id = args.seg_set[seg];
     // The arguments and the set's values are read again (scalar loads) where
     // they are rarely used: held through the loop they would take the scalar
@@ -446,7 +453,7 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
     const ConstSet &S = *sp;
     const uint32_t T = S.n_types, T8 = T * 8, TW = T8 * kParts, KT = S.kdim * T;
     const uint32_t r_lo = a.seg_row[2 * seg], r_hi = a.seg_row[2 * seg + 1];
-    const uint32_t w_lo = a.seg_win[Mode * gridDim.x + seg];  // first row of the window
+    const uint32_t w_lo = a.seg_win[Mode * a.n_segments + seg];  // first row of the window
     // selected cells of the segment: first, first + stride, ... (set-local)
     const uint32_t sshift = (uint32_t)__popc(a.stride_mask);
     const uint32_t phase = ((a.step ? (uint32_t)a.step[0] : 0u) + a.phase) & a.stride_mask;
@@ -562,7 +569,7 @@ __global__ __launch_bounds__(kWalkThreads, 4) void walk_kernel(RelaxArgs args)
     // frame's fields apart (16 bytes per lane): 2.44 ms.
     constexpr uint32_t kLevelBytes = 64 * sizeof(Frame);
     const size_t levels = (size_t)args_again().kdim_max + 1;
-    unsigned char *const stk0 = (unsigned char *)args_again().stack + ((size_t)seg * kWalkThreads + wave * 64) * levels * kFrameBytes;
+    unsigned char *const stk0 = (unsigned char *)args_again().stack + ((size_t)blockIdx.x * kWalkThreads + wave * 64) * levels * kFrameBytes;
     unsigned char *const stk = stk0 + (size_t)lane * sizeof(Frame);
 
     // lane state: the node to expand
@@ -1202,6 +1209,7 @@ struct RelaxCore {
     std::vector<RelaxSet> sets;
     std::vector<uint32_t> quiet_flag;  // per type of every set: 1 = quiescent
     uint32_t n_segments = 0;
+    uint32_t per_launch = 0;   // segments that the stacks are for
     size_t lds_bytes[3] = {0, 0, 0};  // of the walk kernel, per WalkMode
     uint64_t h_total = 0;      // tally entries of all sets
     uint32_t types_total = 0;  // types of all sets
@@ -1430,6 +1438,7 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
     a.beta = beta;
     a.n_sets = n;
     a.n_rows = rows;
+    a.n_segments = c.n_segments;
     a.kdim_max = kdim_max;
     a.sets = (const RelaxSet *)(base + o_sets);
     a.seg_set = (const uint32_t *)(base + o_ss);
@@ -1444,8 +1453,9 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
     a.set_cuts = a.expansions + kCountCopies * kCountWords;
     a.h_total = c.h_total;
     if (c.n_segments) {
-        const size_t stack_bytes = (size_t)c.n_segments * kWalkThreads * (kdim_max + 1) * kFrameBytes;
-        if (hipMalloc((void **)&c.d_stack, stack_bytes) != hipSuccess)
+        const size_t seg_bytes = (size_t)kWalkThreads * (kdim_max + 1) * kFrameBytes;
+        c.per_launch = (uint32_t)std::min<uint64_t>(c.n_segments, kStackBytes / seg_bytes);
+        if (hipMalloc((void **)&c.d_stack, c.per_launch * seg_bytes) != hipSuccess)
             return PROCELL_E_OUT_OF_MEMORY;
         a.stack = c.d_stack;
     }
@@ -1456,10 +1466,15 @@ int core_build(RelaxCore &c, const procell_params *ps, uint32_t n, double beta, 
 // the gradient, and the expansion counter).
 hipError_t core_launch(const RelaxCore &c, const RelaxArgs &a, int mode, hipStream_t st)
 {
-    if (c.n_segments == 0)
-        return hipSuccess;
-    hipLaunchKernelGGL(walk_kernel_of(mode, a.kdim_max), dim3(c.n_segments), dim3(kWalkThreads), c.lds_bytes[mode], st, a);
-    return hipGetLastError();
+    RelaxArgs part = a;
+    for (part.seg_first = 0; part.seg_first < c.n_segments; part.seg_first += c.per_launch) {
+        const uint32_t n = std::min(c.per_launch, c.n_segments - part.seg_first);
+        hipLaunchKernelGGL(walk_kernel_of(mode, a.kdim_max), dim3(n), dim3(kWalkThreads), c.lds_bytes[mode], st, part);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess)
+            return e;
+    }
+    return hipSuccess;
 }
 
 // ---------------------------------------------------------------------------

@@ -19,7 +19,7 @@ namespace fake {
 std::vector<Launch> launches;
 uint64_t sim_runs = 0;
 int fail_event_record = 0;
-uint64_t dead_stream_uses = 0, foreign_stream_uses = 0, streams_alive = 0, memory_alive = 0;
+uint64_t dead_stream_uses = 0, foreign_stream_uses = 0, streams_alive = 0, memory_alive = 0, memory_bytes = 0;
 static float one_ms() { return 1.0f; }
 float (*elapsed_ms)() = one_ms;
 std::vector<uint32_t> segment_cells;
@@ -159,6 +159,7 @@ hipError_t hipMalloc(void **p, size_t n)
         *p = calloc(1, n < 64 ? 64 : n);
     }
     memory[*p] = ++next_id;
+    memory_bytes = n > memory_bytes ? n : memory_bytes;
     ++memory_alive;
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }

@@ -21,7 +21,7 @@ extern uint64_t sim_runs;                  // simulation kernels so far; each le
 extern int fail_event_record;              // > 0: that many calls of hipEventRecord from now on, the last one fails
 extern uint64_t dead_stream_uses;          // calls that named a stream that does not exist
 extern uint64_t foreign_stream_uses;       // calls that named a stream of take_stream()
-extern uint64_t streams_alive, memory_alive;
+extern uint64_t streams_alive, memory_alive, memory_bytes;  // memory_bytes: the largest allocation so far
 extern float (*elapsed_ms)();              // what hipEventElapsedTime reports
 extern std::vector<uint32_t> segment_cells;  // the cells [first, end) of the walk kernel's segments, last launch
 

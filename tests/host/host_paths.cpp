@@ -224,13 +224,39 @@ static void check_autotune()
     }
 }
 
+// A relaxed plan over very many sets: bounded lane stacks, every segment
+// walked by one of a pass's launches.
+static void check_stacks()
+{
+    for (uint32_t n : {1000u, 120000u}) {
+        Case c({{8000.0, 1}}, {{1.0, 20.0, 5.0}}, 90.0, 1.0);
+        std::vector<procell_params> sets(n, c.p);
+        procell_relaxed *r = nullptr;
+        fake::memory_bytes = 0;
+        CHECK(procell_relaxed_create_batch(sets.data(), n, 0.5, &r) == PROCELL_OK);
+        CHECK(fake::memory_bytes <= 8ull << 30);
+        double x = 0.0;
+        fake::launches.clear();
+        CHECK(procell_relaxed_jacobian(r, &x, &x, &x, nullptr) == PROCELL_OK);
+        uint64_t segments = 0, walks = 0;
+        for (const fake::Launch &l : fake::launches)
+            if (l.kernel.find("walk_kernel") != std::string::npos) {
+                segments += l.grid;
+                ++walks;
+            }
+        CHECK(segments == n && walks == (n > 1000 ? 3 : 1));
+        CHECK(procell_relaxed_destroy(r) == PROCELL_OK);
+    }
+}
+
 int main(int argc, char **argv)
 {
     const struct {
         const char *name;
         void (*f)();
     } checks[] = {{"stage", check_stage}, {"noalloc", check_noalloc}, {"reset", check_reset}, {"kernel", check_kernel}, {"window", check_window},
-                  {"autotune", check_autotune}};
+                  {"autotune", check_autotune},
+                  {"stacks", check_stacks}};
     for (const auto &c : checks)
         if (argc == 2 && !strcmp(argv[1], c.name)) {
             c.f();

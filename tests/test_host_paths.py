@@ -60,3 +60,7 @@ def test_tally_window_of_deep_rows(host_paths):
 
 def test_autotuner_times_each_layout_once(host_paths):
     host_paths("autotune")
+
+
+def test_relaxed_plans_of_many_sets_bound_their_stacks(host_paths):
+    host_paths("stacks")
